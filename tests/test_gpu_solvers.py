@@ -1,0 +1,98 @@
+"""The device solvers (Jacobi-PCG and BiCGStab) on systems whose nodes have
+one, two or three free equations, from one element to several workgroups of
+row groups: the residual of the returned solution on the assembled matrix,
+formed by scipy on the host, meets the requested tolerance.
+
+The solvers stop on their recursive residual; its gap to the true one is a
+few rounding errors of K x per iteration, eps * its * |K| |x| / |b| < 1e-11
+relative here, so the true residual is checked to rtol + 1e-10.
+"""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from warp3d_amd import _abi
+from warp3d_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+MESHES = {"one": lambda: M.box_hex8(1),
+          "hex8": lambda: M.box_hex8(5, 4, 3, jitter=0.1, seed=3),
+          "hex8_wide": lambda: M.box_hex8(16, 15, 11, jitter=0.1, seed=4),
+          "hex20": lambda: M.box_hex20(3, 2, 4, jitter=0.05, seed=5),
+          "tet10": lambda: M.box_tet10(3, 3, 2, seed=6)}
+
+
+def _model(name, mat, partial):
+    from warp3d_amd.model import BlockModel
+    m = MESHES[name]()
+    cst = np.zeros(3 * m.nonode, np.int32)
+    base = np.abs(m.coords[:, 2]) < 1e-9
+    for k in range(3):
+        cst[k::3][base] = 1
+    if partial:      # nodes with one or two free equations
+        rng = np.random.default_rng(1)
+        cst[rng.random(cst.size) < 0.3] = 1
+    kw = {}
+    if mat.model == _abi.W3D_MM10:
+        kw["angles"] = M.random_orientations(m.noelem, seed=2)
+    dev = BlockModel(m.model(mat, auto_size=32, **kw))
+    x = m.coords
+    du = np.zeros_like(x)
+    du[:, 2] = 5e-4 * x[:, 2]
+    return dev, cst, du.ravel()
+
+
+@pytest.mark.parametrize("partial", [False, True])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_pcg_residual(name, partial):
+    mat = _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0)
+    dev, cst, du = _model(name, mat, partial)
+    neq, _ = dev.pattern(cst)
+    dev.recover(1, 0, np.zeros_like(du), du)
+    dev.tangent(1, 0)
+    kd, kc = dev.assemble_vss()
+    _, _, ptr, idx = dev.get_pattern()
+    rp = np.concatenate([[0], np.cumsum(ptr)])
+    up = sp.csr_matrix((kc, idx - 1, rp), (neq, neq))
+    K = up + up.T + sp.diags(kd)
+    rng = np.random.default_rng(7)
+    b = rng.uniform(-1, 1, neq)
+    for rtol, x0 in ((1e-8, None), (1e-10, rng.uniform(-1, 1, neq))):
+        x, its, rel = dev.solve_pcg(b, x0=x0, rtol=rtol, maxit=5000)
+        assert rel <= rtol
+        r = np.linalg.norm(b - K @ x) / np.linalg.norm(b)
+        assert r <= rtol + 1e-10, (name, partial, r)
+    # the solution as the guess: no iteration; a zero right-hand side: zero
+    _, its, _ = dev.solve_pcg(b, x0=x, rtol=1e-6)
+    assert its == 0
+    z, its, rel = dev.solve_pcg(np.zeros(neq), x0=x)
+    assert its == 0 and rel == 0.0 and not z.any()
+    if neq > 100:     # the iteration limit is reported
+        from warp3d_amd.model import W3DError
+        with pytest.raises(W3DError, match="no convergence in 3 iterations"):
+            dev.solve_pcg(b, rtol=1e-14, maxit=3)
+
+
+@pytest.mark.parametrize("partial", [False, True])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_bicgstab_residual(name, partial):
+    mat = _abi.mm10_material(tau_y=50.0, tau_v=100.0, theta_0=250.0)
+    dev, cst, du = _model(name, mat, partial)
+    dev.set_asymmetric(True)
+    neq, _ = dev.pattern(cst)
+    u = np.zeros_like(du)
+    dev.recover(1, 0, u, du)
+    dev.recover(1, 1, u, du)
+    dev.tangent(1, 1)
+    rp, col, val = dev.assemble_csr()
+    A = sp.csr_matrix((val, col, rp), (neq, neq))
+    b = np.random.default_rng(8).uniform(-1, 1, neq)
+    x, its, rel = dev.solve_bicgstab(b, rtol=1e-8, maxit=5000)
+    assert rel <= 1e-8 and its > 0
+    r = np.linalg.norm(b - A @ x) / np.linalg.norm(b)
+    # BiCGStab's recursive residual drifts by eps times the largest of its
+    # intermediate residuals (up to 1e4 |b| on these systems)
+    assert r <= 1e-8 + 1e-9, (name, partial, r)
+    z, its, rel = dev.solve_bicgstab(np.zeros(neq))
+    assert its == 0 and rel == 0.0 and not z.any()

@@ -198,7 +198,18 @@ struct w3d_ctx {
   int32_t* d_csr_col = nullptr;
   uint32_t* d_csr_vidx = nullptr;
   double* d_csr_val = nullptr;
+  int32_t* d_csr_grp = nullptr;  // row groups (RowGroups)
+  int csr_ngrp = 0;
+  w3d::RowGroups groups() const {
+    return {d_csr_rp, d_csr_col, d_csr_grp, csr_ngrp};
+  }
   double* d_pcg = nullptr;   // solver work vectors and scalars
+  // solve_poll's pinned state images (2 words each) and events, and the
+  // pinned scalars of a finished solve; made with the context, so that a
+  // solve allocates nothing
+  int32_t* h_poll[2] = {};
+  double* h_poll_sc = nullptr;
+  hipEvent_t poll_ev[2] = {};
   // BiCGStab of the asymmetric CSR: b, x and the work vectors, allocated
   // with the gather map, once per pattern
   double* d_bicg = nullptr;

@@ -211,6 +211,16 @@ int launch_assemble(const double* ek64, const float* ek32, int fp32,
                     const uint16_t* hdr, const uint32_t* src,
                     const int64_t* wbase, int64_t nseg, int64_t neq,
                     double* diag, double* coef, hipStream_t s);
+// Full CSR rows in groups of consecutive rows that share their columns:
+// the free equations of one structure node (at most 3 rows; group g is
+// rows grp[g] .. grp[g + 1] - 1, their lengths equal).
+struct RowGroups {
+  const int64_t* rp;
+  const int32_t* col;
+  const int32_t* grp;
+  int32_t ngrp;
+};
+
 // Asymmetric assembly (w3d_asym.hip): full FP64 Ke of every element of
 // the work list into ekf (block b's elements from ekf_off[b], T*T words
 // each), and its gather into the values of the full CSR rows.
@@ -222,15 +232,14 @@ int launch_tangent_full(const DevModel& M, const WorkItem* d_work,
                         hipStream_t s);
 constexpr int kAsmMaxRow = 768;  // longest CSR row the gather takes
 // Jacobi-BiCGStab on full CSR rows from x = 0; work holds
-// bicgstab_words(n) = 9 n + kBicgScalars + solver_npart(n) doubles.
-// W3D_ERR_NUMERIC after maxit iterations or on a breakdown (a zero rho or
-// (rh, v)), x then the last iterate.  Clears its work array with kernels
-// (no memsets).
-constexpr int kBicgScalars = 16;
-int bicgstab_words(int n);
-int bicgstab(int n, const int64_t* rp, const int32_t* col, const double* val,
-             const double* b, double* x, double* work, double rtol, int maxit,
-             int* iters, double* relres, hipStream_t st);
+// bicgstab_words(n, ngrp) doubles.  W3D_ERR_NUMERIC after maxit iterations
+// or on a breakdown (a zero rho or (rh, v)), x then the last iterate.
+// h, ev: the pinned state images and events of solve_poll.
+int bicgstab_words(int n, int ngrp);
+int bicgstab(int n, const RowGroups& A, const double* val, const double* b,
+             double* x, double* work, double rtol, int maxit, int* iters,
+             double* relres, int32_t* const h[2], const hipEvent_t ev[2],
+             hipStream_t st);
 constexpr int kAsmNone = 0xFFFF;  // constrained column in the gather map
 int launch_assemble_full(const double* ekf, const int64_t* ebase,
                          const int64_t* atoff, const uint16_t* at,
@@ -260,29 +269,101 @@ __host__ __device__ constexpr int tan_batch(int ngp, int tbytes) {
              : (64 / ngp < 1 ? 1 : (64 / ngp > 16 ? 16 : 64 / ngp));
 }
 
-// Jacobi-PCG building blocks (w3d_solver.hip)
+// Solver building blocks (w3d_solver.hip)
 int solver_csr_values(const double* diag, const double* coef, int neq,
                       const uint32_t* vidx, int64_t nnz, double* vals,
                       hipStream_t s);
-int solver_spmv(int n, const int64_t* rp, const int32_t* col,
-                const double* val, const double* x, double* y, hipStream_t s);
-int solver_npart(int n);
+int solver_spmv(const RowGroups& A, const double* val, const double* x,
+                double* y, hipStream_t s);
+
+// One system of a Jacobi-PCG: the full CSR rows of its assembled matrix,
+// its diagonal, right-hand side and vectors, the workgroups of its matrix
+// and vector launches (from its size alone) and their partial sums.
+// single: x holds the initial guess and r A x on entry, the convergence
+// test runs before the first iteration too and a residual that is no
+// number ends the solve; a system of a batch starts from x = 0.
+constexpr int kPcgMaxMul = 2048, kPcgMaxVec = 1024;
+constexpr int32_t kPcgZeroRhs = 4;  // a single solve's state on |b| = 0
+struct PcgSys {
+  const int64_t* rp;
+  const int32_t* col;
+  const int32_t* grp;
+  const double* val;
+  const double* diag;
+  const double* b;
+  double* x;
+  double* r;
+  double* p;
+  double* q;
+  double2* zp;            // (z, p) of every equation
+  double* part;           // pcg_part_words of partial sums
+  double rtol;            // |r| <= rtol |b| ends the solve
+  int32_t maxit;          // or this many iterations
+  int32_t n, ngrp;
+  int32_t mul0, nmul;     // workgroups of the matrix launch
+  int32_t vec0, nvec;     // and of the vector launch
+  int32_t single;
+  __host__ __device__ int off_pq() const { return 0; }
+  __host__ __device__ int off_bb() const { return nmul; }
+  __host__ __device__ int off_rr() const { return nmul + nvec; }
+  __host__ __device__ int off_rz(int k) const { return nmul + (2 + k) * nvec; }
+};
+int pcg_mul_wgs(int ngrp);
+int pcg_vec_wgs(int n);
+inline int pcg_part_words(int nmul, int nvec) { return nmul + 4 * nvec; }
+// A single solve's work array: 5 n doubles of vectors ((z, p) pairs, r, p,
+// q), then 2 scalars (|b|, r.r), the state (done: 0 running, 1 converged,
+// 2 iteration limit, kPcgZeroRhs; iterations; two gates) and the partial
+// sums.
+constexpr int kPcgTail = 8 + kPcgMaxMul + 4 * kPcgMaxVec;
+int launch_pcg_init(const PcgSys& one, hipStream_t s, int32_t* state,
+                    double* sc);
+int launch_pcg_iter(const PcgSys& one, int it, int32_t* state, double* sc,
+                    hipStream_t s);
 // w3d_solve_pcg_static's work memory: a file-scope device array of
-// 4 kStaticMaxEq + 8 + 1024 doubles, its address on `device` (the caller
+// 5 kStaticMaxEq + kPcgTail doubles, its address on `device` (the caller
 // has made that device current)
 constexpr int kStaticMaxEq = 1 << 19;
 constexpr int kMaxDevices = 64;
 int solver_static_scratch(int device, double** out);
-int solver_dot(int n, const double* a, const double* b, double* part,
-               double* out, hipStream_t s);
-int solver_jacobi(int n, const double* diag, const double* r, double* z,
-                  hipStream_t s);
-int solver_update_p(int n, const double* z, const double* sc, double* p,
-                    hipStream_t s);
-int solver_update_xr(int n, const double* p, const double* q,
-                     const double* sc, double* x, double* r, hipStream_t s);
-int solver_residual(int n, const double* b, double* r, hipStream_t s);
-int solver_shift(double* sc, hipStream_t s);
+
+// Solver iterations enqueued per look at the states: about 100 us of work
+// on a few thousand equations, so the enqueueing host stays ahead.
+constexpr int kPollChunk = 8;
+
+// Iterations enqueued ahead of the host: chunks of `chunk` iterations with
+// a copy of the systems' states behind each; the host looks at a chunk's
+// states while the next one runs, so the device never waits for it (an
+// iteration of a finished system returns at once).  enqueue(it) launches
+// iteration it (0 .. maxit; maxit only tests).  h[0], h[1]: pinned images
+// of 2 nsys words; *out points to the one with the final states.
+template <typename Enq>
+int solve_poll(const Enq& enqueue, int nsys, int maxit, int chunk,
+               const int32_t* d_state, int32_t* const h[2],
+               const hipEvent_t ev[2], hipStream_t s, const int32_t** out) {
+  int rc;
+  for (int it = 0, k = 0;; ++k) {
+    const int end = maxit - it > chunk ? it + chunk : maxit;
+    for (; it < end; ++it)
+      if ((rc = enqueue(it))) return rc;
+    const bool last = it >= maxit;
+    if (last && (rc = enqueue(it))) return rc;
+    *out = h[k & 1];
+    if (hipMemcpyAsync(h[k & 1], d_state, 2 * nsys * sizeof(int32_t),
+                       hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipEventRecord(ev[k & 1], s) != hipSuccess)
+      return W3D_ERR_DEVICE;
+    bool done = last;
+    if (!last && k > 0) {
+      const int j = (k - 1) & 1;
+      if (hipEventSynchronize(ev[j]) != hipSuccess) return W3D_ERR_DEVICE;
+      done = true;
+      for (int i = 0; i < nsys; ++i) done = done && h[j][2 * i] != 0;
+    }
+    if (done)
+      return hipStreamSynchronize(s) == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+  }
+}
 
 // ---------------------------------------------------------------------
 // Batches of independent problems (w3d_serve.cpp): one launch covers the
@@ -305,35 +386,20 @@ int launch_mm10_batch(const Mm10Slot* d_slots, int nslot, int nwork_total,
 // Rows of one tile of a batched vector kernel (one workgroup each).
 constexpr int kTileRows = 128;
 
-// One system of a batched Jacobi-PCG: the full CSR of its assembled
-// matrix, its diagonal, right-hand side and vectors, and its tiles.
-// Per system the batch keeps 7 partial-sum rows of ntile words (b.b, then
-// p.q, r.r and r.z by iteration parity), the state (done: 0 running,
-// 1 converged, 2 iteration limit; iterations) and the scalars (|b|, r.r).
-struct PcgSys {
-  const int64_t* rp;
-  const int32_t* col;
-  const double* val;
-  const double* diag;
-  const double* b;
-  double* x;
-  double* r;
-  double* p;
-  double* q;
-  double rtol;            // |r| <= rtol |b| ends the solve
-  int32_t maxit;          // or this many iterations
-  int32_t n;
-  int32_t tile0;
-  int32_t ntile;
+// A batch of Jacobi-PCG systems: owner tables give each workgroup of the
+// two launches its system.
+struct PcgBatch {
+  const PcgSys* sys;
+  const int32_t* mul_owner;
+  const int32_t* vec_owner;
+  int nsys, nmul, nvec;
 };
-// x = 0, r = b, p = D^-1 b and the partial sums; then |b| per system
-int launch_pcg_batch_init(const PcgSys* d_sys, int nsys, int ntile_total,
-                          double* part, int32_t* state, double* sc,
+// x = 0, r = b, z = D^-1 b and the partial sums; then |b| per system
+int launch_pcg_batch_init(const PcgBatch& b, int32_t* state, double* sc,
                           hipStream_t s);
-// iteration it (0-based) of every running system: q = A p; x, r; p
-int launch_pcg_batch_iter(const PcgSys* d_sys, int nsys, int ntile_total,
-                          int it, double* part, int32_t* state, double* sc,
-                          hipStream_t s);
+// iteration it (0-based) of every running system (last: the test alone)
+int launch_pcg_batch_iter(const PcgBatch& b, int it, int last, int32_t* state,
+                          double* sc, hipStream_t s);
 
 // One problem's Newton bookkeeping for the batched residual and update:
 // rhs = -ifv on the equations, |rhs|^2, the reaction |ifv|^2 on the

@@ -96,8 +96,8 @@ struct w3d_problem {
   int64_t nd = 0;
   double *d_u = nullptr, *d_du = nullptr, *d_ifv = nullptr;
   double* d_k = nullptr;  // assembled diagonal, then coefficients
-  double *d_rhs = nullptr, *d_x = nullptr, *d_r = nullptr, *d_p = nullptr,
-         *d_q = nullptr;
+  // the solver's vectors: rhs, x, then (z, p) pairs, r, p, q in d_work
+  double *d_rhs = nullptr, *d_x = nullptr, *d_work = nullptr;
   double* d_cimp = nullptr;  // a full step's imposed increments (cdof order)
   int32_t *d_eqdof = nullptr, *d_cdof = nullptr, *d_ldof = nullptr;
   int64_t bytes = 0;
@@ -124,7 +124,6 @@ struct w3d_batch {
   hipStream_t stream = nullptr;
   int n_cu = 0;
   int mm10_grid = 0;
-  int pcg_chunk = 8;
   // device tables and their pinned host images, grown on demand
   Mm10Slot *d_slots = nullptr, *h_slots = nullptr;
   PcgSys *d_pcg = nullptr, *h_pcg = nullptr;
@@ -132,7 +131,12 @@ struct w3d_batch {
   int cap_sys = 0;
   double* d_part = nullptr;
   int64_t cap_part = 0;
-  int32_t *d_state = nullptr, *h_state = nullptr;
+  // the solver's states, two pinned images of them and their events
+  // (solve_poll), and the systems owning the workgroups of its launches
+  int32_t *d_state = nullptr, *h_state[2] = {};
+  hipEvent_t poll_ev[2] = {};
+  int32_t *d_owner = nullptr, *h_owner = nullptr;
+  int64_t cap_owner = 0;
   double *d_sc = nullptr, *d_out = nullptr, *h_out = nullptr;
   int* d_counter = nullptr;
   // device time per phase of the advances (w3d_batch_phase_times):
@@ -155,7 +159,7 @@ namespace {
 
 void free_problem(w3d_problem* p) {
   dfree(p->d_u); dfree(p->d_du); dfree(p->d_ifv); dfree(p->d_k);
-  dfree(p->d_rhs); dfree(p->d_x); dfree(p->d_r); dfree(p->d_p); dfree(p->d_q);
+  dfree(p->d_rhs); dfree(p->d_x); dfree(p->d_work);
   dfree(p->d_cimp);
   dfree(p->d_eqdof); dfree(p->d_cdof); dfree(p->d_ldof);
 }
@@ -190,12 +194,12 @@ void free_batch_tables(w3d_batch* b) {
   dfree(b->d_slots); hfree(b->h_slots);
   dfree(b->d_pcg); hfree(b->h_pcg);
   dfree(b->d_res); hfree(b->h_res);
-  dfree(b->d_state); hfree(b->h_state);
+  dfree(b->d_state); hfree(b->h_state[0]); hfree(b->h_state[1]);
   dfree(b->d_sc); dfree(b->d_out); hfree(b->h_out);
   b->cap_sys = 0;
 }
 
-int reserve(w3d_batch* b, int nsys, int64_t part_words) {
+int reserve(w3d_batch* b, int nsys, int64_t part_words, int64_t owners) {
   int rc;
   if (nsys > b->cap_sys) {
     free_batch_tables(b);
@@ -203,8 +207,9 @@ int reserve(w3d_batch* b, int nsys, int64_t part_words) {
     if ((rc = dalloc(&b->d_slots, cap)) || (rc = halloc(&b->h_slots, cap)) ||
         (rc = dalloc(&b->d_pcg, cap)) || (rc = halloc(&b->h_pcg, cap)) ||
         (rc = dalloc(&b->d_res, cap)) || (rc = halloc(&b->h_res, cap)) ||
-        (rc = dalloc(&b->d_state, 2 * (size_t)cap)) ||
-        (rc = halloc(&b->h_state, 2 * (size_t)cap)) ||
+        (rc = dalloc(&b->d_state, 4 * (size_t)cap)) ||
+        (rc = halloc(&b->h_state[0], 2 * (size_t)cap)) ||
+        (rc = halloc(&b->h_state[1], 2 * (size_t)cap)) ||
         (rc = dalloc(&b->d_sc, 2 * (size_t)cap)) ||
         (rc = dalloc(&b->d_out, 8 * (size_t)cap)) ||
         (rc = halloc(&b->h_out, 8 * (size_t)cap)))
@@ -214,8 +219,18 @@ int reserve(w3d_batch* b, int nsys, int64_t part_words) {
   if (part_words > b->cap_part) {
     dfree(b->d_part);
     const int64_t cap = std::max(part_words, 2 * b->cap_part);
+    b->cap_part = 0;
     if ((rc = dalloc(&b->d_part, cap))) return rc;
     b->cap_part = cap;
+  }
+  if (owners > b->cap_owner) {
+    dfree(b->d_owner);
+    hfree(b->h_owner);
+    b->cap_owner = 0;
+    const int64_t cap = std::max<int64_t>(owners, 1024);
+    if ((rc = dalloc(&b->d_owner, cap)) || (rc = halloc(&b->h_owner, cap)))
+      return rc;
+    b->cap_owner = cap;
   }
   return W3D_OK;
 }
@@ -285,8 +300,8 @@ int w3d_problem_create(w3d_ctx* c, const int32_t* cstmap, const double* du0,
       (rc = dalloc(&p->d_ifv, p->nd)) ||
       (rc = dalloc(&p->d_k, neq + (size_t)nco)) ||
       (rc = dalloc(&p->d_rhs, neq)) || (rc = dalloc(&p->d_x, neq)) ||
-      (rc = dalloc(&p->d_r, neq)) || (rc = dalloc(&p->d_p, neq)) ||
-      (rc = dalloc(&p->d_q, neq)) || (rc = upload(&p->d_cimp, cimp)) ||
+      (rc = dalloc(&p->d_work, 5 * (int64_t)neq)) ||
+      (rc = upload(&p->d_cimp, cimp)) ||
       (rc = upload(&p->d_eqdof, eqdof)) ||
       (rc = upload(&p->d_cdof, cdof)) || (rc = upload(&p->d_ldof, ldof))) {
     free_problem(p);
@@ -379,9 +394,12 @@ int w3d_batch_create(int32_t device, w3d_batch** out) {
     for (int k = 0; k < 2; ++k)
       if (hipEventCreate(&b->ev[ph][k]) != hipSuccess) b->ev[ph][k] = nullptr;
   int rc = dalloc(&b->d_counter, 1);
+  for (int k = 0; k < 2 && !rc; ++k)
+    if (hipEventCreateWithFlags(&b->poll_ev[k], hipEventDisableTiming) !=
+        hipSuccess)
+      rc = fail(W3D_ERR_DEVICE, "w3d_batch_create: events");
   if (rc) {
-    (void)hipStreamDestroy(b->stream);
-    delete b;
+    w3d_batch_destroy(b);
     return rc;
   }
   *out = b;
@@ -395,6 +413,10 @@ int w3d_batch_destroy(w3d_batch* b) {
   free_batch_tables(b);
   dfree(b->d_part);
   dfree(b->d_counter);
+  dfree(b->d_owner);
+  hfree(b->h_owner);
+  for (int k = 0; k < 2; ++k)
+    if (b->poll_ev[k]) (void)hipEventDestroy(b->poll_ev[k]);
   for (int ph = 0; ph < w3d_batch::kPhases; ++ph)
     for (int k = 0; k < 2; ++k)
       if (b->ev[ph][k]) (void)hipEventDestroy(b->ev[ph][k]);
@@ -463,7 +485,7 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
     res_tile0[k] = ntile_res;
     ntile_res += tiles(std::max({run[k]->neq, run[k]->ncdof, run[k]->nldof}));
   }
-  if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res))) return rc;
+  if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res, 0))) return rc;
   for (int ph = 0; ph < w3d_batch::kPhases; ++ph) b->ev_used[ph] = false;
   // 2. recovery: per-problem passes around one mm10 launch
   b->mark(0, 0);
@@ -600,7 +622,8 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
   // 4. tangents, assemblies and the batched solve
   const int ns = (int)solve.size();
   if (ns > 0) {
-    int ntile = 0, maxit = 0;
+    int nmul = 0, nvec = 0, maxit = 0;
+    int64_t npart = 0;
     b->mark(3, 0);
     for (int i = 0; i < ns; ++i) {
       w3d_problem* p = run[solve[i]];
@@ -616,54 +639,67 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
       PcgSys& S = b->h_pcg[i];
       S.rp = c->d_csr_rp;
       S.col = c->d_csr_col;
+      S.grp = c->d_csr_grp;
       S.val = c->d_csr_val;
       S.diag = p->d_k;
       S.b = p->d_rhs;
       S.x = p->d_x;
-      S.r = p->d_r;
-      S.p = p->d_p;
-      S.q = p->d_q;
+      S.zp = reinterpret_cast<double2*>(p->d_work);
+      S.r = p->d_work + 2 * (int64_t)p->neq;
+      S.p = S.r + p->neq;
+      S.q = S.p + p->neq;
       S.rtol = p->o.pcg_rtol;
       S.maxit = p->o.pcg_maxit;
       S.n = p->neq;
-      S.tile0 = ntile;
-      S.ntile = tiles(p->neq);
-      ntile += S.ntile;
+      S.ngrp = c->csr_ngrp;
+      S.mul0 = nmul;
+      S.nmul = pcg_mul_wgs(S.ngrp);
+      S.vec0 = nvec;
+      S.nvec = pcg_vec_wgs(S.n);
+      S.single = 0;
+      nmul += S.nmul;
+      nvec += S.nvec;
+      npart += pcg_part_words(S.nmul, S.nvec);
       maxit = std::max(maxit, S.maxit);
     }
     b->mark(3, 1);
     // the solve's partial sums follow the residual's in d_part
-    if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res + 7 * (int64_t)ntile)))
+    if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res + npart, nmul + nvec)))
       return rc;
     double* part = b->d_part + 3 * (int64_t)ntile_res;
+    for (int i = 0; i < ns; ++i) {
+      PcgSys& S = b->h_pcg[i];
+      S.part = part;
+      part += pcg_part_words(S.nmul, S.nvec);
+      for (int k = 0; k < S.nmul; ++k) b->h_owner[S.mul0 + k] = i;
+      for (int k = 0; k < S.nvec; ++k) b->h_owner[nmul + S.vec0 + k] = i;
+    }
     HIPCHK(hipMemcpyAsync(b->d_pcg, b->h_pcg, ns * sizeof(PcgSys),
                           hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(b->d_owner, b->h_owner,
+                          (nmul + nvec) * sizeof(int32_t),
+                          hipMemcpyHostToDevice, s));
+    const PcgBatch B{b->d_pcg, b->d_owner, b->d_owner + nmul, ns, nmul, nvec};
     b->mark(4, 0);
-    if ((rc = launch_pcg_batch_init(b->d_pcg, ns, ntile, part, b->d_state,
-                                    b->d_sc, s)))
+    if ((rc = launch_pcg_batch_init(B, b->d_state, b->d_sc, s)))
       return fail(rc, "w3d_batch_advance: solver launch");
-    // every system ends by its own test or its own iteration limit; the
-    // host looks at the states once per chunk of iterations
-    int it = 0;
-    bool all_done = false;
-    while (!all_done && it < maxit) {
-      const int end = std::min(maxit, it + b->pcg_chunk);
-      for (; it < end; ++it)
-        if ((rc = launch_pcg_batch_iter(b->d_pcg, ns, ntile, it, part,
-                                        b->d_state, b->d_sc, s)))
-          return fail(rc, "w3d_batch_advance: solver launch");
-      HIPCHK(hipMemcpyAsync(b->h_state, b->d_state, 2 * ns * sizeof(int32_t),
-                            hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
-      all_done = true;
-      for (int i = 0; i < ns; ++i) all_done = all_done && b->h_state[2 * i];
-    }
+    // every system ends by its own test or its own iteration limit
+    const int32_t* st = nullptr;
+    rc = solve_poll(
+        [&](int it) {
+          return launch_pcg_batch_iter(B, it, it >= maxit, b->d_state,
+                                       b->d_sc, s);
+        },
+        ns, maxit, kPollChunk, b->d_state, b->h_state, b->poll_ev, s, &st);
+    if (rc) return fail(rc, "w3d_batch_advance: solver launch");
     b->mark(4, 1);
-    b->pcg_iterations += it;
+    int it = 0;
     for (int i = 0; i < ns; ++i) {
-      run[solve[i]]->pcg_iters_step += b->h_state[2 * i + 1];
+      it = std::max(it, (int)st[2 * i + 1]);
+      run[solve[i]]->pcg_iters_step += st[2 * i + 1];
       b->h_res[solve[i]].solve = 1;
     }
+    b->pcg_iterations += it;
     // 5. du += x
     HIPCHK(hipMemcpyAsync(b->d_res, b->h_res, nr * sizeof(ResSys),
                           hipMemcpyHostToDevice, s));

@@ -10,6 +10,7 @@
 // then one block over the partials), so a solve is bitwise repeatable.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <mutex>
 
 #include "w3d_internal.h"
@@ -19,11 +20,10 @@ namespace w3d {
 constexpr int kRedBlock = 256;
 
 // Work memory of w3d_solve_pcg_static, which allocates nothing: the vectors
-// r, z, p, q of up to kStaticMaxEq equations, then 8 scalars and the dot
-// products' partial sums (solver_npart <= 1024).  Each device holds its own
-// copy for the life of the process; concurrent calls on one device share
-// it.
-constexpr int64_t kStaticWords = 4LL * kStaticMaxEq + 8 + 1024;
+// of up to kStaticMaxEq equations, then the scalars, state and partial
+// sums.  Each device holds its own copy for the life of the process;
+// concurrent calls on one device share it.
+constexpr int64_t kStaticWords = 5LL * kStaticMaxEq + kPcgTail;
 static __device__ __align__(256) double scratch[kStaticWords];
 
 // The device address of this device's scratch (hipGetSymbolAddress once
@@ -57,103 +57,650 @@ __global__ void k_csr_values(const double* __restrict__ diag,
   }
 }
 
-// y = A x, 16 lanes per row; each lane sums its strided share of the row,
-// then a fixed butterfly over the 16 lanes
-__global__ void __launch_bounds__(256)
-    k_spmv(int n, const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
-           const double* __restrict__ val, const double* __restrict__ x,
-           double* __restrict__ y) {
-  const int lane = threadIdx.x & 15;
-  const int row = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4);
-  double s = 0.0;
-  if (row < n) {
-    for (int64_t k = rp[row] + lane; k < rp[row + 1]; k += 16)
-      s = s + val[k] * x[col[k]];
+// ---------------------------------------------------------------------
+// Products with the full CSR rows, one row group (the free equations of
+// one structure node, which share their columns: up to three consecutive
+// rows of one length) per kGrpLanes lanes.  A lane reads a column index and
+// its vector entry once for the group's rows, so an entry of the matrix
+// costs 9.3 bytes (8 + 4/3) and a third of a gather instead of 12 bytes
+// and one, and the value streams of the rows are each contiguous.  32
+// lanes: the 81 columns of a structured brick's node are three passes, and
+// a 1,000-node system still spreads over 32,000 lanes.  Bound by HBM on
+// large systems (124,740 equations, 9.5 M entries: 25 us, 3.5 TB/s).  Each row sums its
+// lanes' strided shares in a fixed butterfly, so products are bitwise
+// repeatable.
+// ---------------------------------------------------------------------
+constexpr int kGrpLanes = 32;
+constexpr int kMulBlock = 512;
+constexpr int kGrpPerWg = kMulBlock / kGrpLanes;
+
+// s[k] = row (row0 + k) . x over the nr rows of one group, every lane of
+// the group holding the sums; x(c) gives the vector's entry c
+template <typename XF>
+__device__ __forceinline__ void group_product(const int64_t* __restrict__ rp,
+                                              const int32_t* __restrict__ col,
+                                              const double* __restrict__ val,
+                                              int row0, int nr, int lane,
+                                              const XF& x, double (&s)[3]) {
+  const int64_t k0 = rp[row0];
+  const int len = (int)(rp[row0 + 1] - k0);
+  const int32_t* cp = col + k0;
+  const double* v0 = val + k0;
+  const int o1 = nr > 1 ? len : 0, o2 = nr > 2 ? 2 * len : 0;
+  s[0] = s[1] = s[2] = 0.0;
+  constexpr int U = 3;  // entries of a lane in flight together
+  for (int k = lane; k < len; k += U * kGrpLanes) {
+    int c[U];
+    double a0[U], a1[U], a2[U], xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // past the end: the group's last entry, dropped below
+      const int kk = k + u * kGrpLanes < len ? k + u * kGrpLanes : len - 1;
+      c[u] = cp[kk];
+      a0[u] = v0[kk];
+      a1[u] = v0[o1 + kk];
+      a2[u] = v0[o2 + kk];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) xv[u] = x(c[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = k + u * kGrpLanes < len;
+      s[0] = in ? s[0] + a0[u] * xv[u] : s[0];
+      s[1] = in ? s[1] + a1[u] * xv[u] : s[1];
+      s[2] = in ? s[2] + a2[u] * xv[u] : s[2];
+    }
   }
 #pragma unroll
-  for (int off = 8; off >= 1; off >>= 1) s = s + __shfl_xor(s, off, 16);
-  if (row < n && lane == 0) y[row] = s;
+  for (int off = kGrpLanes / 2; off >= 1; off >>= 1)
+#pragma unroll
+    for (int r = 0; r < 3; ++r) s[r] = s[r] + __shfl_xor(s[r], off, kGrpLanes);
 }
 
-// block partial sums of a . b
-__global__ void __launch_bounds__(kRedBlock)
-    k_dot_partial(int n, const double* __restrict__ a,
-                  const double* __restrict__ b, double* __restrict__ part) {
-  __shared__ double s[kRedBlock];
-  double t = 0.0;
-  for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n;
-       i += gridDim.x * kRedBlock)
-    t = t + a[i] * b[i];
-  s[threadIdx.x] = t;
+// sums of N values over the workgroup of NT threads in a fixed order
+// (butterfly in each wave, the waves in order); every thread gets them
+template <int N, int NT>
+__device__ __forceinline__ void block_sums(double (&v)[N],
+                                           double (*s_red)[NT / 64]) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = v[k] + __shfl_xor(v[k], off);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < N; ++k) s_red[k][threadIdx.x >> 6] = v[k];
   __syncthreads();
-  for (int w = kRedBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] = s[threadIdx.x] + s[threadIdx.x + w];
-    __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    v[k] = s_red[k][0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) v[k] = v[k] + s_red[k][w];
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__global__ void __launch_bounds__(kRedBlock)
-    k_sum_partials(int np, const double* __restrict__ part,
-                   double* __restrict__ out) {
-  __shared__ double s[kRedBlock];
-  double t = 0.0;
-  for (int i = threadIdx.x; i < np; i += kRedBlock) t = t + part[i];
-  s[threadIdx.x] = t;
   __syncthreads();
-  for (int w = kRedBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] = s[threadIdx.x] + s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = s[0];
 }
 
-// z = r / diag
-__global__ void k_jacobi(int n, const double* __restrict__ diag,
-                         const double* __restrict__ r, double* __restrict__ z) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) z[i] = r[i] / diag[i];
+// y = A x
+__global__ void __launch_bounds__(kMulBlock)
+    k_grp_spmv(RowGroups A, const double* __restrict__ val,
+               const double* __restrict__ x, double* __restrict__ y) {
+  const int lane = threadIdx.x % kGrpLanes;
+  const int g = blockIdx.x * kGrpPerWg + threadIdx.x / kGrpLanes;
+  if (g >= A.ngrp) return;
+  const int row0 = A.grp[g], nr = A.grp[g + 1] - row0;
+  double s[3];
+  group_product(A.rp, A.col, val, row0, nr, lane,
+                [&](int c) { return x[c]; }, s);
+  if (lane < nr) y[row0 + lane] = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
 }
-
-// p = z + (rz_new / rz_old) p   (beta from the device scalars)
-__global__ void k_update_p(int n, const double* __restrict__ z,
-                           const double* __restrict__ sc,
-                           double* __restrict__ p) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = z[i] + (sc[1] / sc[0]) * p[i];
-}
-
-// x += alpha p, r -= alpha q with alpha = rz / pq
-__global__ void k_update_xr(int n, const double* __restrict__ p,
-                            const double* __restrict__ q,
-                            const double* __restrict__ sc,
-                            double* __restrict__ x, double* __restrict__ r) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    double alpha = sc[1] / sc[2];
-    x[i] = x[i] + alpha * p[i];
-    r[i] = r[i] - alpha * q[i];
-  }
-}
-
-// r = b - r (after r = A x)
-__global__ void k_residual(int n, const double* __restrict__ b,
-                           double* __restrict__ r) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) r[i] = b[i] - r[i];
-}
-
-// sc[0] = sc[1] (keep the previous r.z)
-__global__ void k_shift(double* sc) { sc[0] = sc[1]; }
 
 // ---------------------------------------------------------------------
-// Batched Jacobi-PCG over independent systems.  Tile t of a launch is
-// tile t - tile0 of the system that owns it; each system's reductions run
-// over its own tiles in a fixed order, so a system's iterates do not
-// depend on the other systems of the batch.
+// Jacobi-PCG over one system or a batch of independent ones, two launches
+// an iteration:
+//   k_pcg_mul  the convergence test and beta from the last iteration's
+//              partial sums, p = z + beta p formed at the gathered columns
+//              (one 16-byte (z, p) pair each) and kept for the own rows,
+//              q = A p, partial p.q
+//   k_pcg_vec  alpha, x += alpha p, r -= alpha q, z = r / diag, the (z, p)
+//              pairs, partial r.r and r.z
+// The launches are latency bound for small systems (each is a chain of
+// dependent loads) and the host reads the states behind the device, so an
+// iteration costs no synchronisation.  Measured an iteration, against one
+// launch per vector operation and a host read each: 91 -> 33 us on 124,740
+// equations; against three launches of 128-row tiles: k_pcg_mul 6 us for
+// 18, and 4.5 us for 10 in the vector launches, on three systems of 2,000
+// to 3,600 equations.  Each system's reductions run over
+// its own workgroups in a fixed order, whose number depends on the
+// system's size alone, so a system's iterates do not depend on the batch.
+// Every workgroup of a system reaches the same end-of-solve decision from
+// the same partials and the first one writes it.  A launch never reads a
+// word that it writes: state (done, iterations per system) is the host's,
+// gate[0] of a system closes k_pcg_mul and is written by k_pcg_vec, gate[1]
+// closes k_pcg_vec and is written by k_pcg_mul.
 // ---------------------------------------------------------------------
-constexpr int kPartBB = 0, kPartPQ = 1, kPartRR = 3, kPartRZ = 5;
-constexpr int kSpmvLanes = 16;
+template <bool BATCH>
+__global__ void __launch_bounds__(kRedBlock)
+    k_pcg_init(const PcgSys one, const PcgSys* __restrict__ sys,
+               const int32_t* __restrict__ owner) {
+  __shared__ double s_red[3][kRedBlock / 64];
+  const int si =
+      BATCH ? __builtin_amdgcn_readfirstlane(owner[blockIdx.x]) : 0;
+  const PcgSys& S = BATCH ? sys[si] : one;
+  const int wg = blockIdx.x - S.vec0;
+  double v[3] = {0.0, 0.0, 0.0};  // b.b, r.r, r.z
+  for (int i = wg * kRedBlock + threadIdx.x; i < S.n;
+       i += S.nvec * kRedBlock) {
+    const double bi = S.b[i];
+    double ri = bi;
+    if (S.single)
+      ri = bi - S.r[i];  // r holds A x0
+    else
+      S.x[i] = 0.0;
+    const double zi = ri / S.diag[i];
+    S.r[i] = ri;
+    S.zp[i] = make_double2(zi, 0.0);
+    v[0] = v[0] + bi * bi;
+    v[1] = v[1] + ri * ri;
+    v[2] = v[2] + ri * zi;
+  }
+  block_sums<3, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {
+    S.part[S.off_bb() + wg] = v[0];
+    S.part[S.off_rr() + wg] = v[1];
+    S.part[S.off_rz(1) + wg] = v[2];  // the r.z of iteration -1
+  }
+}
+
+// one workgroup per system: |b|; a zero right-hand side is solved
+template <bool BATCH>
+__global__ void __launch_bounds__(kRedBlock)
+    k_pcg_init2(const PcgSys one, const PcgSys* __restrict__ sys,
+                int32_t* __restrict__ state, int32_t* __restrict__ gate,
+                double* __restrict__ sc) {
+  __shared__ double s_red[1][kRedBlock / 64];
+  const PcgSys& S = BATCH ? sys[blockIdx.x] : one;
+  double v[1] = {0.0};
+  for (int i = threadIdx.x; i < S.nvec; i += kRedBlock)
+    v[0] = v[0] + S.part[S.off_bb() + i];
+  block_sums<1, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {
+    sc[2 * blockIdx.x] = sqrt(v[0]);
+    sc[2 * blockIdx.x + 1] = v[0];
+    const int32_t end = v[0] == 0.0 ? (S.single ? kPcgZeroRhs : 1) : 0;
+    state[2 * blockIdx.x] = end;
+    state[2 * blockIdx.x + 1] = 0;
+    gate[2 * blockIdx.x] = gate[2 * blockIdx.x + 1] = end;
+  }
+}
+
+template <bool BATCH>
+__global__ void __launch_bounds__(kMulBlock)
+    k_pcg_mul(const PcgSys one, const PcgSys* __restrict__ sys,
+              const int32_t* __restrict__ owner, int it,
+              int32_t* __restrict__ state, int32_t* __restrict__ gate,
+              double* __restrict__ sc) {
+  __shared__ double s_red[3][kMulBlock / 64];
+  const int si =
+      BATCH ? __builtin_amdgcn_readfirstlane(owner[blockIdx.x]) : 0;
+  if (gate[2 * si]) return;
+  const PcgSys& S = BATCH ? sys[si] : one;
+  const int wg = blockIdx.x - S.mul0;
+  const int tid = threadIdx.x, lane = tid % kGrpLanes;
+  double v[3] = {0.0, 0.0, 0.0};  // r.r, r.z and the r.z before
+  for (int i = tid; i < S.nvec; i += kMulBlock) {
+    v[0] = v[0] + S.part[S.off_rr() + i];
+    v[1] = v[1] + S.part[S.off_rz((it - 1) & 1) + i];
+    if (it > 0) v[2] = v[2] + S.part[S.off_rz(it & 1) + i];
+  }
+  block_sums<3, kMulBlock>(v, s_red);
+  // the end of the solve: |r| <= rtol |b| or the iteration limit (a batch
+  // tests neither before its first iteration; a single solve also stops
+  // on a residual that is no number)
+  const double nr_ = sqrt(v[0]);
+  const bool conv = nr_ <= S.rtol * sc[2 * si];
+  if ((it > 0 || S.single) &&
+      (conv || it >= S.maxit || (S.single && isnan(nr_)))) {
+    if (wg == 0 && tid == 0) {
+      state[2 * si] = conv ? 1 : 2;
+      state[2 * si + 1] = it;
+      gate[2 * si + 1] = 1;
+      sc[2 * si + 1] = v[0];
+    }
+    return;
+  }
+  const double beta = it > 0 ? v[1] / v[2] : 0.0;
+  const double2* __restrict__ zp = S.zp;
+  double pq[1] = {0.0};
+  for (int g = wg * kGrpPerWg + tid / kGrpLanes; g < S.ngrp;
+       g += S.nmul * kGrpPerWg) {
+    const int row0 = S.grp[g], nr = S.grp[g + 1] - row0;
+    double s[3];
+    group_product(S.rp, S.col, S.val, row0, nr, lane,
+                  [&](int c) {
+                    const double2 w = zp[c];
+                    return w.x + beta * w.y;
+                  },
+                  s);
+    if (lane < nr) {
+      const int i = row0 + lane;
+      const double2 w = zp[i];
+      const double pi = w.x + beta * w.y;
+      const double qi = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
+      S.p[i] = pi;
+      S.q[i] = qi;
+      pq[0] = pq[0] + pi * qi;
+    }
+  }
+  block_sums<1, kMulBlock>(pq, s_red);
+  if (tid == 0) S.part[S.off_pq() + wg] = pq[0];
+}
+
+template <bool BATCH>
+__global__ void __launch_bounds__(kRedBlock)
+    k_pcg_vec(const PcgSys one, const PcgSys* __restrict__ sys,
+              const int32_t* __restrict__ owner, int it,
+              int32_t* __restrict__ gate) {
+  __shared__ double s_red[2][kRedBlock / 64];
+  const int si =
+      BATCH ? __builtin_amdgcn_readfirstlane(owner[blockIdx.x]) : 0;
+  const PcgSys& S = BATCH ? sys[si] : one;
+  const int wg = blockIdx.x - S.vec0;
+  if (gate[2 * si + 1]) {
+    if (wg == 0 && threadIdx.x == 0) gate[2 * si] = 1;
+    return;
+  }
+  double v[2] = {0.0, 0.0};  // p.q and the last r.z
+  for (int i = threadIdx.x; i < S.nmul; i += kRedBlock)
+    v[0] = v[0] + S.part[S.off_pq() + i];
+  for (int i = threadIdx.x; i < S.nvec; i += kRedBlock)
+    v[1] = v[1] + S.part[S.off_rz((it - 1) & 1) + i];
+  block_sums<2, kRedBlock>(v, s_red);
+  const double alpha = v[1] / v[0];
+  v[0] = v[1] = 0.0;  // r.r and r.z
+  for (int i = wg * kRedBlock + threadIdx.x; i < S.n;
+       i += S.nvec * kRedBlock) {
+    const double pi = S.p[i];
+    S.x[i] = S.x[i] + alpha * pi;
+    const double ri = S.r[i] - alpha * S.q[i];
+    const double zi = ri / S.diag[i];
+    S.r[i] = ri;
+    S.zp[i] = make_double2(zi, pi);
+    v[0] = v[0] + ri * ri;
+    v[1] = v[1] + ri * zi;
+  }
+  block_sums<2, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {
+    S.part[S.off_rr() + wg] = v[0];
+    S.part[S.off_rz(it & 1) + wg] = v[1];
+  }
+}
+
+// Workgroups of one system's matrix and vector launches: a tile of groups
+// (rows) each up to the cap, then equal shares.  The caps bound the partial
+// sums that every workgroup of the next launch reads again.
+int pcg_mul_wgs(int ngrp) {
+  const int t = (ngrp + kGrpPerWg - 1) / kGrpPerWg;
+  if (t < 1) return 1;
+  const int per = (t + kPcgMaxMul - 1) / kPcgMaxMul;
+  return (t + per - 1) / per;
+}
+int pcg_vec_wgs(int n) {
+  const int t = (n + kRedBlock - 1) / kRedBlock;
+  return t < 1 ? 1 : t > kPcgMaxVec ? kPcgMaxVec : t;
+}
+
+// state: 2 nsys words, the gates behind them
+int launch_pcg_init(const PcgSys& one, hipStream_t s, int32_t* state,
+                    double* sc) {
+  hipLaunchKernelGGL(k_pcg_init<false>, dim3(one.nvec), dim3(kRedBlock), 0, s,
+                     one, nullptr, nullptr);
+  hipLaunchKernelGGL(k_pcg_init2<false>, dim3(1), dim3(kRedBlock), 0, s, one,
+                     nullptr, state, state + 2, sc);
+  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+}
+
+int launch_pcg_iter(const PcgSys& one, int it, int32_t* state, double* sc,
+                    hipStream_t s) {
+  hipLaunchKernelGGL(k_pcg_mul<false>, dim3(one.nmul), dim3(kMulBlock), 0, s,
+                     one, nullptr, nullptr, it, state, state + 2, sc);
+  if (it < one.maxit)
+    hipLaunchKernelGGL(k_pcg_vec<false>, dim3(one.nvec), dim3(kRedBlock), 0,
+                       s, one, nullptr, nullptr, it, state + 2);
+  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+}
+
+int launch_pcg_batch_init(const PcgBatch& b, int32_t* state, double* sc,
+                          hipStream_t s) {
+  if (b.nsys <= 0) return W3D_OK;
+  hipLaunchKernelGGL(k_pcg_init<true>, dim3(b.nvec), dim3(kRedBlock), 0, s,
+                     PcgSys{}, b.sys, b.vec_owner);
+  hipLaunchKernelGGL(k_pcg_init2<true>, dim3(b.nsys), dim3(kRedBlock), 0, s,
+                     PcgSys{}, b.sys, state, state + 2 * b.nsys, sc);
+  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+}
+
+int launch_pcg_batch_iter(const PcgBatch& b, int it, int last, int32_t* state,
+                          double* sc, hipStream_t s) {
+  if (b.nsys <= 0) return W3D_OK;
+  int32_t* gate = state + 2 * b.nsys;
+  hipLaunchKernelGGL(k_pcg_mul<true>, dim3(b.nmul), dim3(kMulBlock), 0, s,
+                     PcgSys{}, b.sys, b.mul_owner, it, state, gate, sc);
+  if (!last)
+    hipLaunchKernelGGL(k_pcg_vec<true>, dim3(b.nvec), dim3(kRedBlock), 0, s,
+                       PcgSys{}, b.sys, b.vec_owner, it, gate);
+  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+}
+
+// ---------------------------------------------------------------------
+// Jacobi-preconditioned BiCGStab (van der Vorst 1992, right
+// preconditioning) on the full CSR rows, FP64, three launches an iteration:
+//   k_bicg_v   the test and beta, p = r + beta (p - omega v) at the
+//              gathered columns (pairs (r / diag, (p - omega v) / diag)),
+//              v = A D^-1 p, partial (rh, v)
+//   k_bicg_t   alpha, s = r - alpha v at the gathered columns (pairs
+//              (r / diag, v / diag)), t = A D^-1 s, partial (t, s), (t, t)
+//   k_bicg_x   omega, x, r, the pairs of the next iteration, partial
+//              (rh, r), (r, r)
+// (9,360 equations: 113 us an iteration with a launch per operation and a
+// host read, 20 us so.)
+// As in the PCG above every workgroup forms the scalars from the partial
+// sums of the launches before (a fixed order: a solve is bitwise
+// repeatable) and the first one writes them to sc for later launches:
+// [0], [1] rho by iteration parity, [2] alpha, [3] omega, [4] (r, r),
+// [5] |b|.  gate[0..2] close the three launches; none reads a gate that it
+// writes.  A breakdown (a zero rho, (rh, v) or last omega) ends the solve
+// with x at the last iterate.
+// ---------------------------------------------------------------------
+constexpr int kBicgScalars = 8;
+enum { kBicgConv = 1, kBicgLimit = 2, kBicgBreak = 3, kBicgZero = 4,
+       kBicgNan = 5 };
+
+struct BicgSys {
+  RowGroups A;
+  const double* val;
+  const double* b;
+  double *x, *r, *rh, *p, *v, *s, *t, *dinv;
+  double2 *rp2;             // (r, p - omega v) / diag
+  double2 *rv2;             // (r, v) / diag
+  double *part;             // rv nmul, ts nmul, tt nmul, rho nvec, rr nvec
+  double *sc;
+  int32_t* state;           // done, iterations; then the gates
+  int32_t* gate;
+  double rtol;
+  int32_t n, nmul, nvec, maxit;
+};
+
+__global__ void __launch_bounds__(kRedBlock) k_bicg_init(const BicgSys S) {
+  __shared__ double s_red[1][kRedBlock / 64];
+  double v[1] = {0.0};
+  for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < S.n;
+       i += S.nvec * kRedBlock) {
+    // dinv holds the row's diagonal (0 when the pattern has none)
+    const double d = S.dinv[i], di = d != 0.0 ? 1.0 / d : 1.0;
+    const double bi = S.b[i];
+    S.dinv[i] = di;
+    S.x[i] = 0.0;
+    S.r[i] = bi;
+    S.rh[i] = bi;
+    S.rp2[i] = make_double2(bi * di, 0.0);
+    S.p[i] = 0.0;
+    S.v[i] = 0.0;
+    v[0] = v[0] + bi * bi;
+  }
+  block_sums<1, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {  // rh = r = b: rho and (r, r) are (b, b)
+    S.part[3 * S.nmul + blockIdx.x] = v[0];
+    S.part[3 * S.nmul + S.nvec + blockIdx.x] = v[0];
+  }
+}
+
+__global__ void __launch_bounds__(kRedBlock) k_bicg_init2(const BicgSys S) {
+  __shared__ double s_red[1][kRedBlock / 64];
+  double v[1] = {0.0};
+  for (int i = threadIdx.x; i < S.nvec; i += kRedBlock)
+    v[0] = v[0] + S.part[3 * S.nmul + i];
+  block_sums<1, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {
+    for (int k = 0; k < kBicgScalars; ++k) S.sc[k] = 0.0;
+    S.sc[4] = v[0];
+    S.sc[5] = sqrt(v[0]);
+    const int32_t end = sqrt(v[0]) == 0.0 ? kBicgZero : 0;
+    S.state[0] = end;
+    S.state[1] = 0;
+    S.gate[0] = S.gate[1] = S.gate[2] = end;
+  }
+}
+
+// the diagonal of every row (0 when absent)
+__global__ void __launch_bounds__(kMulBlock)
+    k_grp_diag(RowGroups A, const double* __restrict__ val,
+               double* __restrict__ diag) {
+  const int lane = threadIdx.x % kGrpLanes;
+  const int g = blockIdx.x * kGrpPerWg + threadIdx.x / kGrpLanes;
+  if (g >= A.ngrp) return;
+  const int row0 = A.grp[g], nr = A.grp[g + 1] - row0;
+  const int64_t k0 = A.rp[row0];
+  const int len = (int)(A.rp[row0 + 1] - k0);
+  double d[3] = {0.0, 0.0, 0.0};
+  for (int k = lane; k < len; k += kGrpLanes) {
+    const int j = A.col[k0 + k] - row0;
+    if (j == 0) d[0] = val[k0 + k];
+    if (j == 1 && nr > 1) d[1] = val[k0 + len + k];
+    if (j == 2 && nr > 2) d[2] = val[k0 + 2 * (int64_t)len + k];
+  }
+#pragma unroll
+  for (int off = kGrpLanes / 2; off >= 1; off >>= 1)
+#pragma unroll
+    for (int r = 0; r < 3; ++r) d[r] = d[r] + __shfl_xor(d[r], off, kGrpLanes);
+  if (lane < nr) diag[row0 + lane] = lane == 0 ? d[0] : lane == 1 ? d[1] : d[2];
+}
+
+__global__ void __launch_bounds__(kMulBlock)
+    k_bicg_v(const BicgSys S, int it) {
+  __shared__ double s_red[2][kMulBlock / 64];
+  if (S.gate[0]) return;
+  const int wg = blockIdx.x, tid = threadIdx.x, lane = tid % kGrpLanes;
+  double v[2] = {0.0, 0.0};  // rho, (r, r)
+  for (int i = tid; i < S.nvec; i += kMulBlock) {
+    v[0] = v[0] + S.part[3 * S.nmul + i];
+    v[1] = v[1] + S.part[3 * S.nmul + S.nvec + i];
+  }
+  block_sums<2, kMulBlock>(v, s_red);
+  const double rho = v[0], rho1 = S.sc[(it - 1) & 1], alpha1 = S.sc[2],
+               omega1 = S.sc[3];
+  int end = 0;
+  if (it > 0) {  // the residual of iteration it
+    if (!isfinite(v[1]))
+      end = kBicgNan;
+    else if (sqrt(v[1]) / S.sc[5] <= S.rtol)
+      end = kBicgConv;
+    else if (it >= S.maxit)
+      end = kBicgLimit;
+  }
+  if (!end && (rho == 0.0 || (it > 0 && (rho1 == 0.0 || omega1 == 0.0))))
+    end = kBicgBreak;
+  if (wg == 0 && tid == 0) {
+    S.sc[4] = v[1];
+    S.sc[it & 1] = rho;
+    if (end) {
+      S.state[0] = end;
+      S.state[1] = it;
+      S.gate[1] = S.gate[2] = 1;
+    }
+  }
+  if (end) return;
+  const double beta = it > 0 ? (rho / rho1) * (alpha1 / omega1) : 0.0;
+  const double2* __restrict__ w2 = S.rp2;
+  double dot[1] = {0.0};
+  for (int g = wg * kGrpPerWg + tid / kGrpLanes; g < S.A.ngrp;
+       g += S.nmul * kGrpPerWg) {
+    const int row0 = S.A.grp[g], nr = S.A.grp[g + 1] - row0;
+    double s[3];
+    group_product(S.A.rp, S.A.col, S.val, row0, nr, lane,
+                  [&](int c) {
+                    const double2 w = w2[c];
+                    return w.x + beta * w.y;
+                  },
+                  s);
+    if (lane < nr) {
+      const int i = row0 + lane;
+      const double ri = S.r[i], di = S.dinv[i];
+      const double vi = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
+      // p, v: the last iteration's on entry, this one's on exit
+      S.p[i] = ri + beta * (S.p[i] - omega1 * S.v[i]);
+      S.v[i] = vi;
+      S.rv2[i] = make_double2(ri * di, vi * di);
+      dot[0] = dot[0] + S.rh[i] * vi;
+    }
+  }
+  double d2[1] = {dot[0]};
+  block_sums<1, kMulBlock>(d2, s_red);
+  if (tid == 0) S.part[wg] = d2[0];
+}
+
+__global__ void __launch_bounds__(kMulBlock)
+    k_bicg_t(const BicgSys S, int it) {
+  __shared__ double s_red[2][kMulBlock / 64];
+  if (S.gate[1]) return;
+  const int wg = blockIdx.x, tid = threadIdx.x, lane = tid % kGrpLanes;
+  double rv[1] = {0.0};
+  for (int i = tid; i < S.nmul; i += kMulBlock) rv[0] = rv[0] + S.part[i];
+  block_sums<1, kMulBlock>(rv, s_red);
+  if (rv[0] == 0.0) {
+    if (wg == 0 && tid == 0) {
+      S.state[0] = kBicgBreak;
+      S.state[1] = it;
+      S.gate[2] = 1;
+    }
+    return;
+  }
+  const double alpha = S.sc[it & 1] / rv[0];
+  if (wg == 0 && tid == 0) S.sc[2] = alpha;
+  const double2* __restrict__ w2 = S.rv2;
+  double v[2] = {0.0, 0.0};  // (t, s), (t, t)
+  for (int g = wg * kGrpPerWg + tid / kGrpLanes; g < S.A.ngrp;
+       g += S.nmul * kGrpPerWg) {
+    const int row0 = S.A.grp[g], nr = S.A.grp[g + 1] - row0;
+    double s[3];
+    group_product(S.A.rp, S.A.col, S.val, row0, nr, lane,
+                  [&](int c) {
+                    const double2 w = w2[c];
+                    return w.x - alpha * w.y;
+                  },
+                  s);
+    if (lane < nr) {
+      const int i = row0 + lane;
+      const double ti = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
+      const double si = S.r[i] - alpha * S.v[i];
+      S.s[i] = si;
+      S.t[i] = ti;
+      v[0] = v[0] + ti * si;
+      v[1] = v[1] + ti * ti;
+    }
+  }
+  block_sums<2, kMulBlock>(v, s_red);
+  if (tid == 0) {
+    S.part[S.nmul + wg] = v[0];
+    S.part[2 * S.nmul + wg] = v[1];
+  }
+}
+
+__global__ void __launch_bounds__(kRedBlock) k_bicg_x(const BicgSys S) {
+  __shared__ double s_red[2][kRedBlock / 64];
+  const int wg = blockIdx.x;
+  if (S.gate[2]) {
+    if (wg == 0 && threadIdx.x == 0) S.gate[0] = S.gate[1] = 1;
+    return;
+  }
+  double v[2] = {0.0, 0.0};
+  for (int i = threadIdx.x; i < S.nmul; i += kRedBlock) {
+    v[0] = v[0] + S.part[S.nmul + i];
+    v[1] = v[1] + S.part[2 * S.nmul + i];
+  }
+  block_sums<2, kRedBlock>(v, s_red);
+  // (t, t) = 0: s is already the residual of x (a converged half step)
+  const double omega = v[1] != 0.0 ? v[0] / v[1] : 0.0, alpha = S.sc[2];
+  if (wg == 0 && threadIdx.x == 0) S.sc[3] = omega;
+  v[0] = v[1] = 0.0;  // (rh, r), (r, r)
+  for (int i = wg * kRedBlock + threadIdx.x; i < S.n;
+       i += S.nvec * kRedBlock) {
+    const double di = S.dinv[i], pi = S.p[i], si = S.s[i];
+    const double y = pi * di, z = si * di;
+    S.x[i] = (S.x[i] + alpha * y) + omega * z;
+    const double ri = si - omega * S.t[i];
+    S.r[i] = ri;
+    S.rp2[i] = make_double2(ri * di, (pi - omega * S.v[i]) * di);
+    v[0] = v[0] + S.rh[i] * ri;
+    v[1] = v[1] + ri * ri;
+  }
+  block_sums<2, kRedBlock>(v, s_red);
+  if (threadIdx.x == 0) {
+    S.part[3 * S.nmul + wg] = v[0];
+    S.part[3 * S.nmul + S.nvec + wg] = v[1];
+  }
+}
+
+int bicgstab_words(int n, int ngrp) {
+  return 11 * n + kBicgScalars + 4 + 3 * pcg_mul_wgs(ngrp) +
+         2 * pcg_vec_wgs(n);
+}
+
+int bicgstab(int n, const RowGroups& A, const double* val, const double* b,
+             double* x, double* work, double rtol, int maxit, int* iters,
+             double* relres, int32_t* const h[2], const hipEvent_t ev[2],
+             hipStream_t st) {
+  BicgSys S{};
+  S.A = A;
+  S.val = val;
+  S.b = b;
+  S.x = x;
+  S.rp2 = reinterpret_cast<double2*>(work);  // work: 16-byte aligned
+  S.rv2 = S.rp2 + n;
+  S.r = reinterpret_cast<double*>(S.rv2 + n);
+  S.rh = S.r + n;
+  S.p = S.rh + n;
+  S.v = S.p + n;
+  S.s = S.v + n;
+  S.t = S.s + n;
+  S.dinv = S.t + n;
+  S.sc = S.dinv + n;
+  S.state = reinterpret_cast<int32_t*>(S.sc + kBicgScalars);
+  S.gate = S.state + 2;
+  S.part = S.sc + kBicgScalars + 4;
+  S.rtol = rtol;
+  S.n = n;
+  S.nmul = pcg_mul_wgs(A.ngrp);
+  S.nvec = pcg_vec_wgs(n);
+  S.maxit = maxit;
+  const dim3 gm(S.nmul), tm(kMulBlock), gv(S.nvec), tv(kRedBlock);
+  if (A.ngrp > 0)
+    hipLaunchKernelGGL(k_grp_diag, dim3((A.ngrp + kGrpPerWg - 1) / kGrpPerWg),
+                       tm, 0, st, A, val, S.dinv);
+  hipLaunchKernelGGL(k_bicg_init, gv, tv, 0, st, S);
+  hipLaunchKernelGGL(k_bicg_init2, dim3(1), tv, 0, st, S);
+  const int32_t* state = nullptr;
+  const int rc = solve_poll(
+      [&](int it) {
+        hipLaunchKernelGGL(k_bicg_v, gm, tm, 0, st, S, it);
+        if (it < maxit) {
+          hipLaunchKernelGGL(k_bicg_t, gm, tm, 0, st, S, it);
+          hipLaunchKernelGGL(k_bicg_x, gv, tv, 0, st, S);
+        }
+        return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+      },
+      1, maxit, kPollChunk, S.state, h, ev, st, &state);
+  if (rc) return rc;
+  const int end = state[0];
+  *iters = state[1];
+  *relres = 0.0;
+  if (end == kBicgZero) return W3D_OK;
+  double v[2];
+  if (hipMemcpyAsync(v, S.sc + 4, sizeof v, hipMemcpyDeviceToHost, st) !=
+          hipSuccess ||
+      hipStreamSynchronize(st) != hipSuccess)
+    return W3D_ERR_DEVICE;
+  *relres = std::sqrt(v[0]) / v[1];
+  return end == kBicgConv ? W3D_OK : W3D_ERR_NUMERIC;
+}
 
 // the system owning global tile t (tile0 ascending, system 0 at tile 0)
 template <typename S>
@@ -191,174 +738,6 @@ __device__ __forceinline__ double sum_partials(const double* __restrict__ v,
   double t = 0.0;
   for (int i = threadIdx.x; i < n; i += kRedBlock) t = t + v[i];
   return block_sum(t, s_red);
-}
-
-__global__ void __launch_bounds__(kRedBlock)
-    k_pcg_init(const PcgSys* __restrict__ sys, int nsys,
-               double* __restrict__ part) {
-  __shared__ double s_red[kRedBlock];
-  const int si = owner(sys, nsys, blockIdx.x);
-  const PcgSys& S = sys[si];
-  const int t = blockIdx.x - S.tile0;
-  const int row = t * kTileRows + threadIdx.x;
-  double bb = 0.0, rz = 0.0;
-  if (threadIdx.x < kTileRows && row < S.n) {
-    const double bi = S.b[row];
-    const double zi = bi / S.diag[row];
-    S.x[row] = 0.0;
-    S.r[row] = bi;
-    S.p[row] = zi;
-    bb = bi * bi;
-    rz = bi * zi;
-  }
-  bb = block_sum(bb, s_red);
-  rz = block_sum(rz, s_red);
-  if (threadIdx.x == 0) {
-    double* P = part + 7 * (int64_t)S.tile0;
-    P[kPartBB * S.ntile + t] = bb;
-    P[(kPartRZ + 1) * S.ntile + t] = rz;  // the r.z of iteration -1
-  }
-}
-
-// one workgroup per system: |b|, and a zero right-hand side is solved
-__global__ void __launch_bounds__(kRedBlock)
-    k_pcg_init2(const PcgSys* __restrict__ sys, const double* __restrict__ part,
-                int32_t* __restrict__ state, double* __restrict__ sc) {
-  __shared__ double s_red[kRedBlock];
-  const PcgSys& S = sys[blockIdx.x];
-  const double* P = part + 7 * (int64_t)S.tile0;
-  const double bb = sum_partials(P + kPartBB * S.ntile, S.ntile, s_red);
-  if (threadIdx.x == 0) {
-    sc[2 * blockIdx.x] = sqrt(bb);
-    sc[2 * blockIdx.x + 1] = bb;
-    state[2 * blockIdx.x] = bb == 0.0 ? 1 : 0;
-    state[2 * blockIdx.x + 1] = 0;
-  }
-}
-
-// q = A p on the tile's rows (16 lanes per row) and the partial p.q
-__global__ void __launch_bounds__(kRedBlock)
-    k_pcg_spmv(const PcgSys* __restrict__ sys, int nsys, int it,
-               double* __restrict__ part, const int32_t* __restrict__ state) {
-  __shared__ double s_red[kRedBlock];
-  const int si = owner(sys, nsys, blockIdx.x);
-  if (state[2 * si]) return;
-  const PcgSys& S = sys[si];
-  const int t = blockIdx.x - S.tile0;
-  const int lane = threadIdx.x % kSpmvLanes;
-  constexpr int kRowsPerPass = kRedBlock / kSpmvLanes;
-  double pq = 0.0;
-  for (int k = threadIdx.x / kSpmvLanes; k < kTileRows; k += kRowsPerPass) {
-    const int row = t * kTileRows + k;
-    double v = 0.0;
-    if (row < S.n) {
-      for (int64_t j = S.rp[row] + lane; j < S.rp[row + 1]; j += kSpmvLanes)
-        v = v + S.val[j] * S.p[S.col[j]];
-    }
-#pragma unroll
-    for (int off = kSpmvLanes / 2; off >= 1; off >>= 1)
-      v = v + __shfl_xor(v, off, kSpmvLanes);
-    if (row < S.n && lane == 0) {
-      S.q[row] = v;
-      pq = pq + S.p[row] * v;
-    }
-  }
-  pq = block_sum(pq, s_red);
-  if (threadIdx.x == 0)
-    part[7 * (int64_t)S.tile0 + (kPartPQ + (it & 1)) * S.ntile + t] = pq;
-}
-
-// alpha = r.z / p.q; x += alpha p, r -= alpha q; partial r.r and r.z
-__global__ void __launch_bounds__(kRedBlock)
-    k_pcg_xr(const PcgSys* __restrict__ sys, int nsys, int it,
-             double* __restrict__ part, const int32_t* __restrict__ state) {
-  __shared__ double s_red[kRedBlock];
-  const int si = owner(sys, nsys, blockIdx.x);
-  if (state[2 * si]) return;
-  const PcgSys& S = sys[si];
-  const int t = blockIdx.x - S.tile0;
-  double* P = part + 7 * (int64_t)S.tile0;
-  const double pq =
-      sum_partials(P + (kPartPQ + (it & 1)) * S.ntile, S.ntile, s_red);
-  const double rz =
-      sum_partials(P + (kPartRZ + ((it - 1) & 1)) * S.ntile, S.ntile, s_red);
-  const double alpha = rz / pq;
-  const int row = t * kTileRows + threadIdx.x;
-  double rr = 0.0, rzn = 0.0;
-  if (threadIdx.x < kTileRows && row < S.n) {
-    S.x[row] = S.x[row] + alpha * S.p[row];
-    const double ri = S.r[row] - alpha * S.q[row];
-    S.r[row] = ri;
-    rr = ri * ri;
-    rzn = ri * (ri / S.diag[row]);
-  }
-  rr = block_sum(rr, s_red);
-  rzn = block_sum(rzn, s_red);
-  if (threadIdx.x == 0) {
-    P[(kPartRR + (it & 1)) * S.ntile + t] = rr;
-    P[(kPartRZ + (it & 1)) * S.ntile + t] = rzn;
-  }
-}
-
-// convergence |r| <= rtol |b| (or the iteration limit) ends the system;
-// otherwise p = D^-1 r + (r.z / r.z old) p.  Every workgroup of a system
-// reaches the same decision from the same partials; the first tile's
-// writes the state, which a sibling in this launch may or may not see:
-// either way it leaves p alone or updates a p that is no longer read.
-__global__ void __launch_bounds__(kRedBlock)
-    k_pcg_p(const PcgSys* __restrict__ sys, int nsys, int it,
-            const double* __restrict__ part,
-            int32_t* __restrict__ state, double* __restrict__ sc) {
-  __shared__ double s_red[kRedBlock];
-  const int si = owner(sys, nsys, blockIdx.x);
-  if (state[2 * si]) return;
-  const PcgSys& S = sys[si];
-  const int t = blockIdx.x - S.tile0;
-  const double* P = part + 7 * (int64_t)S.tile0;
-  const double rr =
-      sum_partials(P + (kPartRR + (it & 1)) * S.ntile, S.ntile, s_red);
-  const bool conv = sqrt(rr) <= S.rtol * sc[2 * si];
-  if (conv || it + 1 >= S.maxit) {
-    if (t == 0 && threadIdx.x == 0) {
-      state[2 * si] = conv ? 1 : 2;
-      state[2 * si + 1] = it + 1;
-      sc[2 * si + 1] = rr;
-    }
-    return;
-  }
-  const double rzn =
-      sum_partials(P + (kPartRZ + (it & 1)) * S.ntile, S.ntile, s_red);
-  const double rzo =
-      sum_partials(P + (kPartRZ + ((it - 1) & 1)) * S.ntile, S.ntile, s_red);
-  const double beta = rzn / rzo;
-  const int row = t * kTileRows + threadIdx.x;
-  if (threadIdx.x < kTileRows && row < S.n)
-    S.p[row] = S.r[row] / S.diag[row] + beta * S.p[row];
-}
-
-int launch_pcg_batch_init(const PcgSys* d_sys, int nsys, int ntile_total,
-                          double* part, int32_t* state, double* sc,
-                          hipStream_t s) {
-  if (nsys <= 0) return W3D_OK;
-  if (ntile_total > 0)
-    hipLaunchKernelGGL(k_pcg_init, dim3(ntile_total), dim3(kRedBlock), 0, s,
-                       d_sys, nsys, part);
-  hipLaunchKernelGGL(k_pcg_init2, dim3(nsys), dim3(kRedBlock), 0, s, d_sys,
-                     part, state, sc);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int launch_pcg_batch_iter(const PcgSys* d_sys, int nsys, int ntile_total,
-                          int it, double* part, int32_t* state, double* sc,
-                          hipStream_t s) {
-  if (nsys <= 0 || ntile_total <= 0) return W3D_OK;
-  hipLaunchKernelGGL(k_pcg_spmv, dim3(ntile_total), dim3(kRedBlock), 0, s,
-                     d_sys, nsys, it, part, state);
-  hipLaunchKernelGGL(k_pcg_xr, dim3(ntile_total), dim3(kRedBlock), 0, s,
-                     d_sys, nsys, it, part, state);
-  hipLaunchKernelGGL(k_pcg_p, dim3(ntile_total), dim3(kRedBlock), 0, s, d_sys,
-                     nsys, it, part, state, sc);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
 // ---------------------------------------------------------------------
@@ -497,62 +876,11 @@ int solver_csr_values(const double* diag, const double* coef, int neq,
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
-int solver_spmv(int n, const int64_t* rp, const int32_t* col,
-                const double* val, const double* x, double* y, hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_spmv, dim3(nblk((int64_t)n * 16, 256)), dim3(256), 0,
-                       s, n, rp, col, val, x, y);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-// out[0] = a . b, with part of >= solver_npart(n) doubles of scratch
-int solver_npart(int n) {
-  int np = (n + kRedBlock * 4 - 1) / (kRedBlock * 4);
-  return np < 1 ? 1 : (np > 1024 ? 1024 : np);
-}
-int solver_dot(int n, const double* a, const double* b, double* part,
-               double* out, hipStream_t s) {
-  int np = solver_npart(n);
-  hipLaunchKernelGGL(k_dot_partial, dim3(np), dim3(kRedBlock), 0, s, n, a, b,
-                     part);
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kRedBlock), 0, s, np,
-                     part, out);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int solver_jacobi(int n, const double* diag, const double* r, double* z,
-                  hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_jacobi, dim3(nblk(n, 256)), dim3(256), 0, s, n, diag,
-                       r, z);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int solver_update_p(int n, const double* z, const double* sc, double* p,
-                    hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_update_p, dim3(nblk(n, 256)), dim3(256), 0, s, n, z,
-                       sc, p);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int solver_update_xr(int n, const double* p, const double* q, const double* sc,
-                     double* x, double* r, hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_update_xr, dim3(nblk(n, 256)), dim3(256), 0, s, n, p,
-                       q, sc, x, r);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int solver_residual(int n, const double* b, double* r, hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_residual, dim3(nblk(n, 256)), dim3(256), 0, s, n, b,
-                       r);
-  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
-}
-
-int solver_shift(double* sc, hipStream_t s) {
-  hipLaunchKernelGGL(k_shift, dim3(1), dim3(1), 0, s, sc);
+int solver_spmv(const RowGroups& A, const double* val, const double* x,
+                double* y, hipStream_t s) {
+  if (A.ngrp > 0)
+    hipLaunchKernelGGL(k_grp_spmv, dim3(nblk(A.ngrp, kGrpPerWg)),
+                       dim3(kMulBlock), 0, s, A, val, x, y);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
