@@ -1295,9 +1295,15 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
 // elem_hist(span, hist, ngp) from (element 1, first Rp word of crystal 1,
 // point 1), so words of several elements of the block enter it.  At step
 // 1 those words are the values mm10 initialised in place.  Elements with
-// several crystals get zeros.  Finite strains: per element (below).  One
-// 64-lane workgroup per mm10 block.
+// several crystals get zeros.  Finite strains: per element (below).
+// kGradWgs 256-lane workgroups per mm10 block, each fitting the block's 27
+// words and writing its share of the points (a point per lane, so a word's
+// stores are contiguous over the lanes).  Bound by the latency of the
+// gather and fit, then by the 216 bytes a point: one 64-lane workgroup a
+// block, which wrote the 27,648 words of 128 bricks alone, took 58 us.
 // ---------------------------------------------------------------------
+constexpr int kGradWgs = 8;
+constexpr int kGradBlock = 256;
 __device__ double mm10_init_word(const DevModel& M, const BlockDesc& bd,
                                  int w, int i, int64_t q, int64_t SG) {
   const double* hn = M.hist_n + bd.hist_off;
@@ -1314,21 +1320,24 @@ __device__ double mm10_init_word(const DevModel& M, const BlockDesc& bd,
   return hn[w * SG + q];  // words mm10 does not initialise
 }
 
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(kGradBlock)
     k_mm10_grads(DevModel M, const int32_t* __restrict__ blks, int lo,
                  int hi, int step) {
-  const int b = blks[blockIdx.x];
+  const int b = blks[blockIdx.x / kGradWgs];
   if (b < lo || b >= hi) return;
   const BlockDesc bd = M.blocks[b];
   const GaussTable* gt = M.tables + bd.table;
   const int S = bd.span, G = bd.ngp, H = bd.hist;
   const int64_t SG = (int64_t)S * G;
   const int l = threadIdx.x;
+  // the first point (or, for finite strains, element) of this lane
+  const int first = (blockIdx.x % kGradWgs) * kGradBlock + l;
+  if (first - l >= (bd.geonl ? S : (int)SG)) return;  // uniform
   __shared__ double s_v[9 * kMaxGp];
   __shared__ double s_g[27];
   const double* hn = M.hist_n + bd.hist_off;
   if (bd.ncry == 1) {
-    for (int f = l; f < 9 * G; f += 64) {
+    for (int f = l; f < 9 * G; f += kGradBlock) {
       const int64_t L = (int64_t)(kMM10Common + 9) * S + f;
       const int i = (int)(L % S);
       const int w = (int)((L / S) % H);
@@ -1350,8 +1359,9 @@ __global__ void __launch_bounds__(64)
   __syncthreads();
   double* hn1 = M.hist_n1 + bd.hist_off;
   if (!bd.geonl) {
-    for (int64_t k = l; k < 27 * SG; k += 64)
-      hn1[(36 + k / SG) * SG + k % SG] = s_g[k / SG];
+    for (int q = first; q < (int)SG; q += kGradWgs * kGradBlock)
+#pragma unroll
+      for (int k = 0; k < 27; ++k) hn1[(36 + k) * SG + q] = s_g[k];
     return;
   }
   // finite strains (mm10_calc_grads' geonl branch): per element, the fit
@@ -1359,7 +1369,7 @@ __global__ void __launch_bounds__(64)
   // n+1]) taken to the current axes by the inverse (mm10_a_invert_33) of
   // the element's n = 0 Jacobian at its last point; zeros for several
   // crystals or a singular Jacobian
-  for (int i = l; i < S; i += 64) {
+  for (int i = first; i < S; i += kGradWgs * kGradBlock) {
     double gv[27];
 #pragma unroll
     for (int k = 0; k < 27; ++k) gv[k] = 0.0;
@@ -1425,8 +1435,8 @@ __global__ void __launch_bounds__(64)
 int launch_mm10_grads(const DevModel& M, const int32_t* d_blks, int nblks,
                       int lo, int hi, int step, hipStream_t s) {
   if (nblks > 0)
-    hipLaunchKernelGGL(k_mm10_grads, dim3(nblks), dim3(64), 0, s, M, d_blks,
-                       lo, hi, step);
+    hipLaunchKernelGGL(k_mm10_grads, dim3(nblks * kGradWgs), dim3(kGradBlock),
+                       0, s, M, d_blks, lo, hi, step);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
