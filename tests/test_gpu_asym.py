@@ -118,3 +118,58 @@ def test_bicgstab_solves_the_asymmetric_csr():
     assert np.abs(x - xr).max() <= 1e-8 * np.abs(xr).max()
     # bitwise repeatable
     assert np.array_equal(d.solve_bicgstab(b, rtol=1e-12, maxit=5000)[0], x)
+
+
+def _fan(n):
+    """n bricks around one edge: its two nodes' rows couple 12 n + 6
+    equations, of every element of the mesh."""
+    a = 2 * np.pi * np.arange(n) / n
+    b = a + np.pi / n
+    plan = [np.zeros((1, 2)), np.stack([np.cos(a), np.sin(a)], 1),
+            1.2 * np.stack([np.cos(b), np.sin(b)], 1)]
+    plan = np.concatenate(plan)
+    xyz = np.concatenate([np.c_[plan, np.full(len(plan), z)]
+                          for z in (0.0, 0.4)])
+    np_ = len(plan)
+    conn = []
+    for i in range(n):
+        q = {(-1, -1): 0, (1, -1): 1 + i, (1, 1): 1 + n + i,
+             (-1, 1): 1 + (i + 1) % n}
+        conn.append([1 + q[(x, y)] + (np_ if z > 0 else 0)
+                     for x, y, z in M.HEX8_NAT.astype(int)])
+    return M.Mesh(xyz, conn, _abi.W3D_L3DISOP)
+
+
+@pytest.mark.parametrize("n,span", [(2, 1), (3, 5), (5, 33), (6, 128)])
+def test_full_matrices_of_block_remainders(n, span):
+    """Batches and work items cut short by the block, and rows of nodes
+    with one, two or three free components."""
+    from warp3d_amd.model import BlockModel
+    m = M.box_hex8(n, jitter=0.05, seed=n)
+    cp = _abi.mm10_material(**RVE_MATERIAL)
+    arr = m.model(cp, auto_size=span,
+                  angles=M.random_orientations(m.noelem, seed=6))
+    cst = (np.random.default_rng(n).random(3 * m.nonode) < 0.3)
+    _compare(BlockModel(arr), O.OracleModel(arr), m, 0.004,
+             cst.astype(np.int32))
+
+
+@pytest.mark.parametrize("n", [20, 56, 57, 63])
+def test_rows_of_a_fan_of_bricks(n):
+    """Long rows (12 n + 6 entries): four waves a workgroup up to 682
+    entries, two from there to the longest row taken (768)."""
+    from warp3d_amd.model import BlockModel
+    m = _fan(n)
+    mat = _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0)
+    arr = m.model(mat, auto_size=16, bbar=0)
+    _compare(BlockModel(arr), O.OracleModel(arr), m, 0.002, None)
+
+
+def _compare(d, o, m, amp, cst):
+    assert_close(_drive(d, m, amp, cst), _drive(o, m, amp, cst),
+                 what="forces")
+    for b in range(1, o.nelblk + 1):
+        assert_close(d.get_ek_full(b), o.get_ek_full(b), what=f"Ke {b}")
+    rp, col, val = d.assemble_csr()
+    _, _, valo = o.assemble_csr(rp, col)
+    assert_close(val, valo, what="CSR values")

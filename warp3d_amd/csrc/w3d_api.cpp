@@ -1816,7 +1816,7 @@ int w3d_assemble_csr_dev(w3d_ctx* c, double* d_val) {
   prof_begin(c, W3D_PHASE_ASSEMBLE);
   rc = launch_assemble_full(c->d_ekf, c->d_fa_ebase, c->d_fa_atoff,
                             c->d_fa_at, c->d_fa_eqdof, c->d_fa_invptr,
-                            c->d_fa_ln, c->d_csr_rp, d_val, c->neqns,
+                            c->d_fa_ln, c->groups(), c->csr_maxrow, d_val,
                             c->stream);
   prof_end(c, W3D_PHASE_ASSEMBLE);
   if (rc) return fail(rc, "w3d_assemble_csr: kernel launch failed");

@@ -221,9 +221,10 @@ struct RowGroups {
   int32_t ngrp;
 };
 
-// Asymmetric assembly (w3d_asym.hip): full FP64 Ke of every element of
-// the work list into ekf (block b's elements from ekf_off[b], T*T words
-// each), and its gather into the values of the full CSR rows.
+// Asymmetric assembly: full FP64 Ke of every element of the work list into
+// ekf (block b's elements from ekf_off[b], T*T words each; w3d_tangent.hip),
+// and its gather into the values of the full CSR rows, the longest of which
+// has maxrow entries (w3d_asym.hip).
 int launch_tangent_full(const DevModel& M, const WorkItem* d_work,
                         const std::vector<int>& groups,
                         const std::vector<int>& gstart,
@@ -244,8 +245,8 @@ constexpr int kAsmNone = 0xFFFF;  // constrained column in the gather map
 int launch_assemble_full(const double* ekf, const int64_t* ebase,
                          const int64_t* atoff, const uint16_t* at,
                          const int32_t* eq_dof, const int64_t* inv_ptr,
-                         const int32_t* inv_ln, const int64_t* rp,
-                         double* val, int neq, hipStream_t s);
+                         const int32_t* inv_ln, const RowGroups& A,
+                         int maxrow, double* val, hipStream_t s);
 int launch_tangent_mfma(const DevModel& M, const WorkItem* d_work,
                         const std::vector<int>& groups,
                         const std::vector<int>& group_start,

@@ -31,6 +31,13 @@
 // gtg(a, b) = sum_p (g_a^T S g_b) w |J| of every node pair is a second,
 // smaller contraction on the matrix cores (k = (point, component)) whose
 // NN x NN result is added to the three component blocks as Ke is stored.
+//
+// Asymmetric assembly (FULL; gptns1.f:1513 bdbt_asym, gptns1.f:1371
+// drive_10_cnst, gptns1.f:1174 extract_D_symmetric): the same contraction
+// over every 16x16 tile, in the element's own dof order, with the whole
+// 6x6 [D] (mm10: the point's history words 1-36, unsymmetrised; mm01: its
+// cep).  Word col T + row is sum_k B(k, col) BD(k, row), so the B columns
+// are the A operand and lanes walk consecutive words.  FP64 only.
 #include <hip/hip_runtime.h>
 
 #include "w3d_geonl.h"
@@ -100,16 +107,21 @@ __host__ __device__ constexpr int tan_waves_per_eu(int nnode, bool geonl) {
 }
 
 template <int NN, int G, bool BBAR, typename T, bool GEONL = false,
-          bool TRN = false>
+          bool TRN = false, bool FULL = false>
 __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
     __attribute__((amdgpu_waves_per_eu(tan_waves_per_eu(NN, GEONL))))
     k_tangent_mfma(DevModel M, const WorkItem* __restrict__ work,
-                   T* __restrict__ ek_out) {
+                   T* __restrict__ ek_out,
+                   const int64_t* __restrict__ ekf_off) {
+  static_assert(!FULL || (sizeof(T) == 8 && !GEONL && !TRN),
+                "the full Ke is FP64, small displacements");
   constexpr int W = tan_mfma_waves(NN);   // waves per workgroup
   constexpr int EB = tan_batch(G, (int)sizeof(T));  // elements of a batch
   constexpr int TD = 3 * NN;              // element dofs
   constexpr int NTL = (TD + 15) / 16;     // 16-wide tiles per side
-  constexpr int NUP = NTL * (NTL + 1) / 2;  // upper tiles
+  // tiles of the contraction: the upper ones, or all of them
+  constexpr int NUP = FULL ? NTL * NTL : NTL * (NTL + 1) / 2;
+  constexpr int ND = FULL ? 36 : 21;      // [D] words of a point
   constexpr int NPG = (G + 3) / 4;        // 4-point groups (one k step each)
   using MF = Mfma<T>;
   using v4 = typename MF::v4;
@@ -127,7 +139,7 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
   // the batch's scaled [D] words (S3 on) share each wave's slab with the
   // nodal coordinates (S1-S2 only): one workgroup more per CU.  The slabs
   // are per wave, as the waves run their stages independently.
-  constexpr size_t kDBytes = sizeof(T) * EB * G * 21;
+  constexpr size_t kDBytes = sizeof(T) * EB * G * ND;
   constexpr size_t kCeBytes = sizeof(double) * EB * 3 * NN;
   constexpr size_t kSlab = (kDBytes > kCeBytes ? kDBytes : kCeBytes) / 8;
   __shared__ double s_dce[W][kSlab];
@@ -145,7 +157,7 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
   const int tid = threadIdx.x;
   const int wv = tid >> 6;   // wave of this lane
   // this wave's slab as [D] words and as coordinates
-  T(*s_dw)[G][21] = reinterpret_cast<T(*)[G][21]>(&s_dce[wv][0]);
+  T(*s_dw)[G][ND] = reinterpret_cast<T(*)[G][ND]>(&s_dce[wv][0]);
   double(*s_cew)[3][NN] = reinterpret_cast<double(*)[3][NN]>(&s_dce[wv][0]);
   const int l = tid & 63;    // lane in the wave
   const int q = l >> 4;      // point of the lane inside a 4-point group
@@ -161,11 +173,12 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
   // the lane's component in each tile's dof column
   int cmp[NTL];
 #pragma unroll
-  for (int t = 0; t < NTL; ++t) cmp[t] = (16 * t + cres) % 3;
+  for (int t = 0; t < NTL; ++t)
+    cmp[t] = FULL ? (16 * t + cres) / NN : (16 * t + cres) % 3;
   // small elements (at most 3 upper tiles): the word of each accumulator
   // value in the ranked upper triangle, or -1 below the diagonal or past
   // the last dof
-  constexpr bool kPreOff = NUP <= 3;
+  constexpr bool kPreOff = !FULL && NUP <= 3;
   int soff[kPreOff ? 4 * NUP : 1];
   if (kPreOff) {
 #pragma unroll
@@ -221,7 +234,7 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
     wave_sync();
     const bool pact = l < nb * G;   // the lane has a point of the batch
     // S2: node ranks; the Jacobian at every point (jacob1) and its inverse
-    for (int k = l; k < nb * NN; k += 64) {
+    for (int k = FULL ? nb * NN : l; k < nb * NN; k += 64) {
       const int e = k / NN, j = k % NN;
       const int mine = s_node[wv][e][j];
       int r = 0;
@@ -266,14 +279,26 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
       s_detw[wv][e][g] = dj;
     }
     wave_sync();
-    // this lane's point: the 21 words of its stored [D], coalesced over
+    // this lane's point: the words of its stored [D], coalesced over
     // the batch (word k of point (i, g) at k S G + i G + g); issued after
     // the Jacobians, which need many registers, and in flight during the
     // B-bar sums; lanes past the batch read its last point (in bounds) and drop it
     const int64_t pq = (int64_t)ie0 * G + (pact ? l : nb * G - 1);
-    double pd[21];
+    double pd[ND];
+    if (FULL && bd.model == W3D_MM10) {
+      const double* hd = M.hist_n1 + bd.hist_off + pq;
 #pragma unroll
-    for (int k = 0; k < 21; ++k) pd[k] = cep_b[k * SG + pq];
+      for (int k = 0; k < ND; ++k) pd[k] = hd[k * SG];
+    } else if (FULL) {
+      double lo[21];
+#pragma unroll
+      for (int k = 0; k < 21; ++k) lo[k] = cep_b[k * SG + pq];
+#pragma unroll
+      for (int k = 0; k < ND; ++k) pd[k] = lo[tri(k % 6, k / 6)];
+    } else {
+#pragma unroll
+      for (int k = 0; k < ND; ++k) pd[k] = cep_b[k * SG + pq];
+    }
     // S3: B-bar volume terms (lanes = element x node); [D] scaled by
     // w |J| (extract_D_symmetric) and by 1/6 for tetrahedra (adjust_cnst)
     if (BBAR)
@@ -330,7 +355,7 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
         for (int k = 0; k < 6; ++k) s_cs[wv][e][g][k] = (T)cs[k];
       } else {
 #pragma unroll
-        for (int k = 0; k < 21; ++k) {
+        for (int k = 0; k < ND; ++k) {
           double v = wdj * pd[k];
           if (tet) v = (1.0 / 6.0) * v;
           s_dw[e][g][k] = (T)v;
@@ -347,7 +372,7 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
 #pragma unroll
       for (int t = 0; t < NTL; ++t) {
         const int dp = 16 * t + cres;
-        jn[t] = dp < TD ? s_inv[wv][e][dp / 3] : -1;
+        jn[t] = dp >= TD ? -1 : FULL ? dp % NN : s_inv[wv][e][dp / 3];
       }
       // the contraction, four points per k step
       v4 acc[NUP];
@@ -429,8 +454,13 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
 #pragma unroll
         for (int r = 0; r < 6; ++r) {
           // BD(r, dof) = sum_m D(m, r) B(m, dof), bdbtgen order
-          const T d0 = dm[tri(0, r)], d1 = dm[tri(1, r)], d2 = dm[tri(2, r)],
-                  d3 = dm[tri(3, r)], d4 = dm[tri(4, r)], d5 = dm[tri(5, r)];
+          // (FULL: D(m, r) at word 6 r + m)
+          const T d0 = dm[FULL ? 6 * r : tri(0, r)],
+                  d1 = dm[FULL ? 6 * r + 1 : tri(1, r)],
+                  d2 = dm[FULL ? 6 * r + 2 : tri(2, r)],
+                  d3 = dm[FULL ? 6 * r + 3 : tri(3, r)],
+                  d4 = dm[FULL ? 6 * r + 4 : tri(4, r)],
+                  d5 = dm[FULL ? 6 * r + 5 : tri(5, r)];
           T bdv[NTL];
 #pragma unroll
           for (int t = 0; t < NTL; ++t)
@@ -438,7 +468,9 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
                      d3 * col[t][3] + d4 * col[t][4] + d5 * col[t][5];
 #pragma unroll
           for (int u = 0; u < NUP; ++u)
-            acc[u] = MF::mma(bdv[tile_i(u)], col[tile_j(u)][r], acc[u]);
+            acc[u] = FULL ? MF::mma(col[u / NTL][r], bdv[u % NTL], acc[u])
+                          : MF::mma(bdv[FULL ? 0 : tile_i(u)],
+                                    col[FULL ? 0 : tile_j(u)][r], acc[u]);
         }
       }
       if (GEONL) {
@@ -501,6 +533,18 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
           }
         }
         wave_sync();
+      }
+      if (FULL) {
+        T* out = ek_out + ekf_off[wi.blk] + (int64_t)ie * TD * TD;
+#pragma unroll
+        for (int u = 0; u < NUP; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int cw = 16 * (u / NTL) + MF::row(l, v);
+            const int rw = 16 * (u % NTL) + cres;
+            if (cw < TD && rw < TD) out[cw * TD + rw] = acc[u][v];
+          }
+        continue;
       }
       // the upper triangle straight from the accumulators, ranked
       // row-major: each store writes four runs of 16 consecutive words
@@ -584,7 +628,8 @@ int launch_tangent_mfma(const DevModel& M, const WorkItem* d_work,
 #define LAUNCH(NN, G, BB, T, GE, TR)                                          \
   hipLaunchKernelGGL((k_tangent_mfma<NN, G, BB, T, GE, TR>), grid,            \
                      dim3(64 * tan_mfma_waves(NN)), 0, s, M, w,               \
-                     precision == W3D_FP32 ? (T*)M.ek32 : (T*)M.ek64)
+                     precision == W3D_FP32 ? (T*)M.ek32 : (T*)M.ek64,         \
+                     (const int64_t*)nullptr)
 #define BY_TRN(NN, G, BB, T, GE)          \
   if (trn)                                \
     LAUNCH(NN, G, BB, T, GE, true);       \
@@ -607,6 +652,32 @@ int launch_tangent_mfma(const DevModel& M, const WorkItem* d_work,
 #undef X
 #undef BY_TRN
 #undef LAUNCH
+    if (!done) return W3D_ERR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
+}
+
+int launch_tangent_full(const DevModel& M, const WorkItem* d_work,
+                        const std::vector<int>& groups,
+                        const std::vector<int>& gstart,
+                        const std::vector<int>& gcount,
+                        const int64_t* d_ekf_off, double* d_ekf,
+                        hipStream_t s) {
+  for (size_t k = 0; k < groups.size(); ++k) {
+    if (gcount[k] == 0) continue;
+    if (groups[k] & 1) return W3D_ERR_UNSUPPORTED;  // finite strains
+    const WorkItem* w = d_work + gstart[k];
+    bool done = false;
+#define X(NN, G, BB)                                                        \
+  if (!done && (groups[k] >> 3) == (group_key(NN, G, BB) >> 3)) {           \
+    hipLaunchKernelGGL((k_tangent_mfma<NN, G, BB, double, false, false,     \
+                                       true>),                              \
+                       dim3(gcount[k]), dim3(64 * tan_mfma_waves(NN)), 0, s, \
+                       M, w, d_ekf, d_ekf_off);                             \
+    done = true;                                                            \
+  }
+    W3D_TAN_GROUPS(X)
+#undef X
     if (!done) return W3D_ERR_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
