@@ -1,0 +1,47 @@
+"""The symmetric assembly's segment map and gather at the sizes where a
+wave's 64 segments and its window of 192 contributions end: one element,
+rows of nodes with one, two or three free components, single segments of
+many contributions (a fan of bricks around one edge) and waves of several
+windows.  The matrix equals the oracle's assembly of the same blocks: the
+FP64 tangent within 1e-10, the FP32 one within 2e-6 of its own scale."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests._util import RTOL_FP64, assert_close, smooth_field
+from tests.test_gpu_asym import _fan
+from warp3d_amd import _abi
+from warp3d_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+MESHES = {
+    "one_hex8": lambda: M.box_hex8(1),
+    "one_tet10_cell": lambda: M.box_tet10(1),
+    "hex8": lambda: M.box_hex8(5, 4, 7, jitter=0.05, seed=1),
+    "hex20": lambda: M.box_hex20(2, 3, 2, jitter=0.05, seed=2),
+    "tet10": lambda: M.box_tet10(2, 2, 3, jitter=0.05, seed=3),
+    "fan_3": lambda: _fan(3),
+    "fan_12": lambda: _fan(12),
+    "fan_120": lambda: _fan(120),
+}
+
+
+@pytest.mark.parametrize("fixed", [0.0, 0.4])
+@pytest.mark.parametrize("kind", sorted(MESHES))
+def test_assembled_matrix(kind, fixed):
+    from warp3d_amd.model import BlockModel
+    m = MESHES[kind]()
+    mat = _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0)
+    arr = m.model(mat, auto_size=16)
+    d, o = BlockModel(arr), O.OracleModel(arr)
+    cst = (np.random.default_rng(5).random(3 * m.nonode) < fixed)
+    u, du = np.zeros(3 * m.nonode), smooth_field(m, 0.002, seed=2)
+    for x in (d, o):
+        x.pattern(cst.astype(np.int32))
+        x.recover(1, 1, u, du)
+    o.tangent(1, 1)
+    ko = np.concatenate(o.assemble_vss())
+    for prec, rtol in ((_abi.W3D_FP64, RTOL_FP64), (_abi.W3D_FP32, 2e-6)):
+        d.tangent(1, 1, prec)
+        assert_close(np.concatenate(d.assemble_vss()), ko, rtol, kind)

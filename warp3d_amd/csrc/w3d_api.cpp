@@ -580,13 +580,15 @@ int create_impl(w3d_ctx* c, const w3d_model* m) {
     std::vector<double> xyz(m->c, m->c + 3 * (int64_t)m->nonode);
     if ((rc = upload(&c->d_coords, xyz))) return rc;
   }
+  // (the Ke arrays two words longer: the assembly loads three words of
+  // every contribution)
   struct A {
     double** p;
     int64_t n;
   } arrs[] = {{&c->d_stress_n, 9 * q},  {&c->d_stress_n1, 9 * q},
               {&c->d_strain_n, 6 * q},  {&c->d_strain_n1, 6 * q},
               {&c->d_hist_n, h},        {&c->d_hist_n1, h},
-              {&c->d_cep, 21 * q},      {&c->d_ek64, ek},
+              {&c->d_cep, 21 * q},      {&c->d_ek64, ek + 2},
               {&c->d_einfvec, fv},      {&c->d_evol, c->noelem},
               {&c->d_u, 3 * (int64_t)c->nonode},
               {&c->d_du, 3 * (int64_t)c->nonode},
@@ -610,8 +612,8 @@ int create_impl(w3d_ctx* c, const w3d_model* m) {
     HIPCHK(hipMemset(c->d_u_t, 0, 3 * (size_t)c->nonode * sizeof(double)));
     HIPCHK(hipMemset(c->d_du_t, 0, 3 * (size_t)c->nonode * sizeof(double)));
   }
-  if ((rc = dalloc(&c->d_ek32, ek))) return rc;
-  HIPCHK(hipMemset(c->d_ek32, 0, std::max<int64_t>(ek, 1) * sizeof(float)));
+  if ((rc = dalloc(&c->d_ek32, ek + 2))) return rc;
+  HIPCHK(hipMemset(c->d_ek32, 0, (ek + 2) * sizeof(float)));
   if ((rc = dalloc(&c->d_flags, 4))) return rc;
   HIPCHK(hipMemset(c->d_flags, 0, 4 * sizeof(int32_t)));
   if ((rc = dalloc(&c->d_counter, 4))) return rc;

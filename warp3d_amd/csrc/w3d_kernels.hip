@@ -850,13 +850,26 @@ __global__ void k_energy_reduce(const double* __restrict__ en_wg,
 }
 
 // Row-by-row assembly (assem_a_row, assemble_code.f:785) over the segment
-// map: one thread per segment (a diagonal, or a run of one row's
-// coefficients in the components of one column node).  The wave finds its
-// segments' first contribution and first output by prefix sums of the
-// headers from the wave's two base offsets.  Each output sums its
-// contributions in FP64 in the reference's order (elements on the row's
-// node, then erow, then ecol occurrences).  Outputs 0 .. neq-1 are the
-// diagonal, the rest the coefficients right of the diagonal.
+// map: a wave takes 64 segments (a diagonal, or a run of one row's
+// coefficients in the components of one column node) and finds their
+// first contribution and first output by one prefix sum of the headers from
+// its two base offsets.  Each output sums its contributions in FP64 in the
+// reference's order (elements on the row's node, then erow, then ecol
+// occurrences).  Outputs 0 .. neq-1 are the diagonal, the rest the
+// coefficients right of the diagonal.
+//
+// Bound by the Ke words' gather (three words a contribution out of lines
+// that neighbouring nodes share), so the loads are spread over the lanes: a
+// lane loads one contribution of the wave's contiguous list, all of a
+// window's loads in flight together and every lane at work, and leaves its
+// three words in LDS, where the lane of the segment sums them in order; the
+// outputs go through LDS too and leave as one contiguous run.  A lane that
+// walked its own segment's list (up to eight contributions, three on
+// average) loaded word by word at a third of the lanes: 308 -> 171 us on
+// 216,000 bricks in FP32 (2.7 TB/s of Ke words and outputs), 163 -> 97 us on
+// 15,600 quadratic bricks in FP64 (3.7 TB/s).  The window of 192 is what the
+// 64 segments of such meshes list on average; 256 and 320 cost FP64 its
+// waves a CU (119 and 131 us on the quadratic bricks).
 __device__ inline int wave_incl_scan(int x, int lane) {
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -866,39 +879,83 @@ __device__ inline int wave_incl_scan(int x, int lane) {
   return x;
 }
 
+// three consecutive Ke words, loaded together at the alignment of one
 template <typename KT>
-__global__ void __launch_bounds__(256)
+struct Ke3 {
+  KT w[3];
+};
+constexpr int kAsmVssWaves = 4;    // waves of a workgroup
+constexpr int kAsmVssWindow = 192; // contributions in LDS, a multiple of 64
+
+template <typename KT>
+__global__ void __launch_bounds__(64 * kAsmVssWaves)
     k_assemble(const KT* __restrict__ ek, const uint16_t* __restrict__ hdr,
                const uint32_t* __restrict__ src,
                const int64_t* __restrict__ wbase, int64_t nseg, int64_t neq,
                double* __restrict__ diag, double* __restrict__ coef) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
+  constexpr int U = kAsmVssWindow / 64;
+  // a window's words, then the wave's (at most 192) outputs
+  constexpr int kIn = 3 * kAsmVssWindow * (int)sizeof(KT), kOut = 192 * 8;
+  __shared__ double s_all[kAsmVssWaves][(kIn > kOut ? kIn : kOut) / 8];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t w = (int64_t)blockIdx.x * kAsmVssWaves + wv;
+  if (w * 64 >= nseg) return;  // uniform across the wave
+  const int64_t t = w * 64 + lane;
+  KT* in = reinterpret_cast<KT*>(s_all[wv]);
+  double* out = s_all[wv];
   const int h = t < nseg ? hdr[t] : 0;
-  const int n = h & 255, mask = (h >> 8) & 7;
-  const int len = __popc(mask);
-  const int n_ex = wave_incl_scan(n, lane) - n;
-  const int l_ex = wave_incl_scan(len, lane) - len;
-  if (t >= nseg) return;
-  const int64_t w = t >> 6;
-  const int64_t so = wbase[2 * w] + n_ex;
-  int64_t oo = wbase[2 * w + 1] + l_ex;
+  const int n = h & 255, mask = (h >> 8) & 7, len = __popc(mask);
+  // contributions (at most 64 * 255) and outputs scanned together
+  const int incl = wave_incl_scan(n | len << 16, lane);
+  const int tot = __builtin_amdgcn_readlane(incl, 63);
+  const int ntot = tot & 0xffff, ltot = tot >> 16;
+  const int n1 = incl & 0xffff, n0 = n1 - n, l0 = (incl >> 16) - len;
+  const int64_t so = wbase[2 * w], oo = wbase[2 * w + 1];
   double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int k = 0; k < n; ++k) {
-    const uint32_t b = src[so + k];
-    if (mask & 1) s0 = s0 + (double)ek[b];
-    if (mask & 2) s1 = s1 + (double)ek[b + 1];
-    if (mask & 4) s2 = s2 + (double)ek[b + 2];
-  }
-  const double v[3] = {s0, s1, s2};
+  for (int c0 = 0; c0 < ntot; c0 += kAsmVssWindow) {
+    const int m = ntot - c0 < kAsmVssWindow ? ntot - c0 : kAsmVssWindow;
+    uint32_t b[U];
+    Ke3<KT> v[U];
+    // lanes past the window's end load its last contribution again; the
+    // words past a single-component one are in the padded array and unused
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    if (!(mask >> c & 1)) continue;
-    if (oo < neq)
-      diag[oo] = v[c];
+    for (int j = 0; j < U; ++j) {
+      const int k = 64 * j + lane;
+      b[j] = src[so + c0 + (k < m ? k : m - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+      v[j] = *reinterpret_cast<const Ke3<KT>*>(ek + b[j]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int k = 64 * j + lane;
+      if (k < m) {
+        in[3 * k] = v[j].w[0];
+        in[3 * k + 1] = v[j].w[1];
+        in[3 * k + 2] = v[j].w[2];
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int ka = (n0 > c0 ? n0 : c0) - c0;
+    const int ke = (n1 < c0 + m ? n1 : c0 + m) - c0;
+    for (int k = ka; k < ke; ++k) {
+      s0 = s0 + (double)in[3 * k];
+      s1 = s1 + (double)in[3 * k + 1];
+      s2 = s2 + (double)in[3 * k + 2];
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  int o = l0;
+  if (mask & 1) out[o++] = s0;
+  if (mask & 2) out[o++] = s1;
+  if (mask & 4) out[o++] = s2;
+  __builtin_amdgcn_wave_barrier();
+  for (int k = lane; k < ltot; k += 64) {
+    if (oo + k < neq)
+      diag[oo + k] = out[k];
     else
-      coef[oo - neq] = v[c];
-    ++oo;
+      coef[oo + k - neq] = out[k];
   }
 }
 
@@ -1008,14 +1065,16 @@ int launch_assemble(const double* ek64, const float* ek32, int fp32,
                     const uint16_t* hdr, const uint32_t* src,
                     const int64_t* wbase, int64_t nseg, int64_t neq,
                     double* diag, double* coef, hipStream_t s) {
-  const int64_t nb = (nseg + 255) / 256;
+  const int64_t nb = (nseg + 64 * kAsmVssWaves - 1) / (64 * kAsmVssWaves);
   if (nb > 0) {
     if (fp32)
-      hipLaunchKernelGGL(k_assemble<float>, dim3((unsigned)nb), dim3(256), 0,
-                         s, ek32, hdr, src, wbase, nseg, neq, diag, coef);
+      hipLaunchKernelGGL(k_assemble<float>, dim3((unsigned)nb),
+                         dim3(64 * kAsmVssWaves), 0, s, ek32, hdr, src, wbase,
+                         nseg, neq, diag, coef);
     else
-      hipLaunchKernelGGL(k_assemble<double>, dim3((unsigned)nb), dim3(256), 0,
-                         s, ek64, hdr, src, wbase, nseg, neq, diag, coef);
+      hipLaunchKernelGGL(k_assemble<double>, dim3((unsigned)nb),
+                         dim3(64 * kAsmVssWaves), 0, s, ek64, hdr, src, wbase,
+                         nseg, neq, diag, coef);
   }
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
