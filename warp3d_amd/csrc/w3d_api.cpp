@@ -157,46 +157,10 @@ void build_runs(w3d_ctx* c) {
   }
 }
 
-// Pinned slots of 8 doubles, one per context: contexts share slabs of 64
-// slots, so that making one costs no pinned allocation of its own (set-up
-// of a 1,000-brick context 0.40 ms with and without); a slab without a slot
-// in use is given back.
-struct PollSlab {
-  double* base;
-  uint64_t used;
-};
-std::mutex g_poll_mu;
-std::vector<PollSlab> g_poll_slabs;
-
-double* poll_slot() {
-  std::lock_guard<std::mutex> lk(g_poll_mu);
-  for (PollSlab& s : g_poll_slabs)
-    if (~s.used) {
-      const int k = __builtin_ctzll(~s.used);
-      s.used |= 1ull << k;
-      return s.base + 8 * k;
-    }
-  PollSlab s{nullptr, 1};
-  if (hipHostMalloc((void**)&s.base, 64 * 8 * sizeof(double),
-                    hipHostMallocPortable) != hipSuccess)
-    return nullptr;
-  g_poll_slabs.push_back(s);
-  return s.base;
-}
-
-void poll_slot_free(double* p) {
-  if (!p) return;
-  std::lock_guard<std::mutex> lk(g_poll_mu);
-  for (size_t i = 0; i < g_poll_slabs.size(); ++i) {
-    PollSlab& s = g_poll_slabs[i];
-    if (p < s.base || p >= s.base + 64 * 8) continue;
-    s.used &= ~(1ull << ((p - s.base) / 8));
-    if (!s.used) {
-      (void)hipHostFree(s.base);
-      g_poll_slabs.erase(g_poll_slabs.begin() + i);
-    }
-    return;
-  }
+// A context's pinned image: a solve's scalars and states (8 words), then
+// what a recovery leaves for the host (launch_recover_end).
+size_t pin_words(const w3d_ctx* c) {
+  return 8 + kBlkSums * (size_t)c->nelblk + 2;
 }
 
 void free_ctx(w3d_ctx* c) {
@@ -241,8 +205,8 @@ void free_ctx(w3d_ctx* c) {
     c->poll_ev[k] = nullptr;
     c->h_poll[k] = nullptr;
   }
-  poll_slot_free(c->h_poll_sc);
-  c->h_poll_sc = nullptr;
+  if (c->h_poll_sc) (void)hipHostFree(c->h_poll_sc);
+  c->h_poll_sc = c->h_rec = nullptr;
   if (c->stream) hipStreamDestroy(c->stream);
   c->stream = nullptr;
 }
@@ -527,8 +491,13 @@ int create_impl(w3d_ctx* c, const w3d_model* m) {
   // ---- device ----
   HIPCHK(hipSetDevice(c->device));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  c->h_poll_sc = poll_slot();
-  if (!c->h_poll_sc) return fail(W3D_ERR_NOMEM, "w3d_create: pinned memory");
+  if (hipHostMalloc((void**)&c->h_poll_sc, pin_words(c) * sizeof(double),
+                    hipHostMallocPortable | hipHostMallocCoherent) !=
+      hipSuccess) {
+    c->h_poll_sc = nullptr;
+    return fail(W3D_ERR_NOMEM, "w3d_create: pinned memory");
+  }
+  c->h_rec = c->h_poll_sc + 8;
   for (int k = 0; k < 2; ++k) {
     c->h_poll[k] = reinterpret_cast<int32_t*>(c->h_poll_sc + 4 + k);
     HIPCHK(hipEventCreateWithFlags(&c->poll_ev[k], hipEventDisableTiming));
@@ -744,9 +713,10 @@ int enqueue_block_recover(w3d_ctx* c, int b, hipStream_t s, int step,
                           c->d_en_wg, 1, s);
   }
   if (!rc && want_energy)
-    rc = launch_energy_reduce(c->d_en_wg, c->d_blk_wfirst + b,
-                              c->d_blk_wcount + b, 1,
-                              c->d_blk_sums + kBlkSums * b, s);
+    rc = launch_recover_end(nullptr, nullptr, nullptr, 0, nullptr, c->d_en_wg,
+                            c->d_blk_wfirst + b, c->d_blk_wcount + b, 1,
+                            c->d_blk_sums + kBlkSums * b, nullptr, nullptr,
+                            s);
   return rc;
 }
 
@@ -758,15 +728,6 @@ int flags_status(const int32_t* f, int step) {
     return fail(W3D_ERR_NUMERIC, "non-positive deformation Jacobian at step 1");
   if (f[1] || f[3]) return W3D_CUT_STEP;
   return W3D_OK;
-}
-
-int check_flags(w3d_ctx* c, int step) {
-  int32_t f[4];
-  HIPCHK(hipMemcpyAsync(f, c->d_flags, sizeof f, hipMemcpyDeviceToHost,
-                        c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  prof_collect(c);
-  return flags_status(f, step);
 }
 
 int recover_lists(w3d_ctx* c, RecoverLists& L) {
@@ -793,13 +754,10 @@ int enqueue_recover_stage(w3d_ctx* c, const RecoverLists& L, int stage,
       if (!d_u)
         return fail(W3D_ERR_ARG,
                     "recover: finite strains need the displacements u");
-      const size_t nb = 3 * (size_t)c->nonode * sizeof(double);
-      HIPCHK(hipMemcpyAsync(c->d_u_t, d_u, nb, hipMemcpyDeviceToDevice,
-                            c->stream));
-      HIPCHK(hipMemcpyAsync(c->d_du_t, d_du, nb, hipMemcpyDeviceToDevice,
-                            c->stream));
     }
-    rc = launch_fill_i32(c->d_flags, 4, 0, c->stream);
+    rc = launch_recover_begin(c->d_flags,
+                              c->has_geonl ? 3 * (int64_t)c->nonode : 0, d_u,
+                              d_du, c->d_u_t, c->d_du_t, c->stream);
     if (rc) return fail(rc, "recover: flag reset launch failed");
     c->last_step = step;
     prof_begin(c, W3D_PHASE_RECOVER);
@@ -827,17 +785,26 @@ int enqueue_recover_stage(w3d_ctx* c, const RecoverLists& L, int stage,
                           c->stream);
       prof_end(c, W3D_PHASE_RECOVER);
     }
+    // the forces, the energy sums and the host's image in one launch (while
+    // phases are timed the forces in a launch of their own)
+    const int nsum = sums && want_energy ? c->nelblk : 0;
+    const bool apart = c->profiling && !c->capturing && (nsum || L.host);
     if (!rc && d_ifv) {
       prof_begin(c, W3D_PHASE_IFV);
-      rc = launch_ifv_gather(c->d_einfvec, c->d_inv_ptr, c->d_inv_off,
-                             c->nonode, d_ifv, c->stream);
+      rc = launch_recover_end(c->d_einfvec, c->d_inv_ptr, c->d_inv_off,
+                              c->nonode, d_ifv, c->d_en_wg, c->d_blk_wfirst,
+                              c->d_blk_wcount, apart ? 0 : nsum,
+                              c->d_blk_sums, c->d_flags,
+                              apart ? nullptr : L.host, c->stream);
       prof_end(c, W3D_PHASE_IFV);
       if (rc) return fail(rc, "recover: ifv gather launch failed");
     }
-    if (!rc && sums && want_energy) {
+    if (!rc && (nsum || L.host) && (apart || !d_ifv)) {
       prof_begin(c, W3D_PHASE_ENERGY);
-      rc = launch_energy_reduce(c->d_en_wg, c->d_blk_wfirst, c->d_blk_wcount,
-                                c->nelblk, c->d_blk_sums, c->stream);
+      rc = launch_recover_end(nullptr, nullptr, nullptr, 0, nullptr,
+                              c->d_en_wg, c->d_blk_wfirst, c->d_blk_wcount,
+                              nsum, c->d_blk_sums, c->d_flags, L.host,
+                              c->stream);
       prof_end(c, W3D_PHASE_ENERGY);
       if (rc) return fail(rc, "recover: energy reduction launch failed");
     }
@@ -891,17 +858,16 @@ int enqueue_csr_values(w3d_ctx* c, const double* d_diag,
 }
 
 // After the stream: energy and plastic work from the per-block sums (block
-// order), then the flags.
+// order), then the flags, both from the context's pinned image.
 int finish_recover(w3d_ctx* c, int step, int iter, double* energy,
                    double* plastic_work) {
+  HIPCHK(hipStreamSynchronize(c->stream));
   double en = 0.0, pw = 0.0, fa = 0.0;
+  int nsum = 0;
   if ((energy || plastic_work) && iter > 0) {
-    std::vector<double> sums(kBlkSums * (size_t)c->nelblk);
-    HIPCHK(hipMemcpyAsync(sums.data(), c->d_blk_sums,
-                          sums.size() * sizeof(double),
-                          hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int b = 0; b < c->nelblk; ++b) {
+    nsum = c->nelblk;
+    const double* sums = c->h_rec;
+    for (int b = 0; b < nsum; ++b) {
       en = en + sums[kBlkSums * b];
       pw = pw + sums[kBlkSums * b + 1];
       fa = fa + sums[kBlkSums * b + 2];
@@ -911,7 +877,10 @@ int finish_recover(w3d_ctx* c, int step, int iter, double* energy,
   }
   if (energy) *energy = en;
   if (plastic_work) *plastic_work = pw;
-  return check_flags(c, step);
+  prof_collect(c);
+  int32_t f[4];
+  std::memcpy(f, c->h_rec + kBlkSums * nsum, sizeof f);
+  return flags_status(f, step);
 }
 
 int recover_impl(w3d_ctx* c, int step, int iter, int extrapolated,
@@ -921,6 +890,7 @@ int recover_impl(w3d_ctx* c, int step, int iter, int extrapolated,
   HIPCHK(hipSetDevice(c->device));
   RecoverLists L;
   int rc = recover_lists(c, L);
+  L.host = c->h_rec;
   if (!rc)
     rc = enqueue_recover(c, L, step, iter, extrapolated, d_u, d_du, d_ifv,
                          energy || plastic_work, first_blk, nblk);
@@ -1184,8 +1154,9 @@ int w3d_assemble_ifv(w3d_ctx* c, double* ifv, double* sum_ifv,
                      int64_t* num_term_ifv) {
   if (!c) return fail(W3D_ERR_ARG, "w3d_assemble_ifv: null context");
   HIPCHK(hipSetDevice(c->device));
-  int rc = launch_ifv_gather(c->d_einfvec, c->d_inv_ptr, c->d_inv_off,
-                             c->nonode, c->d_ifv, c->stream);
+  int rc = launch_recover_end(c->d_einfvec, c->d_inv_ptr, c->d_inv_off,
+                              c->nonode, c->d_ifv, nullptr, nullptr, nullptr,
+                              0, nullptr, nullptr, nullptr, c->stream);
   if (rc) return fail(rc, "w3d_assemble_ifv: launch failed");
   if (ifv)
     HIPCHK(hipMemcpyAsync(ifv, c->d_ifv, 3 * (size_t)c->nonode * 8,
@@ -1638,17 +1609,17 @@ static int finish_pattern(w3d_ctx* c, int32_t* neqns_out,
     if ((rc = upload(&c->d_csr_vidx, vidx))) return rc;
     if ((rc = dalloc(&c->d_csr_val, nnz))) return rc;
     // rows in groups that share their columns: the consecutive equations
-    // of one node
+    // of one node (a row's columns compared with the row before it)
+    std::vector<uint8_t> same(neq > 0 ? neq : 1, 0);
+#pragma omp parallel for schedule(static)
+    for (int r = 1; r < neq; ++r)
+      same[r] = c->eqn_node_map[r] == c->eqn_node_map[r - 1] &&
+                rp[r + 1] - rp[r] == rp[r] - rp[r - 1] &&
+                std::equal(col.begin() + rp[r], col.begin() + rp[r + 1],
+                           col.begin() + rp[r - 1]);
     std::vector<int32_t> grp{0};
-    for (int r = 1; r < neq; ++r) {
-      const int g = grp.back();
-      const bool same =
-          r - g < 3 && c->eqn_node_map[r] == c->eqn_node_map[g] &&
-          rp[r + 1] - rp[r] == rp[g + 1] - rp[g] &&
-          std::equal(col.begin() + rp[r], col.begin() + rp[r + 1],
-                     col.begin() + rp[g]);
-      if (!same) grp.push_back(r);
-    }
+    for (int r = 1; r < neq; ++r)
+      if (!same[r] || r - grp.back() >= 3) grp.push_back(r);
     c->csr_ngrp = neq > 0 ? (int)grp.size() : 0;
     grp.push_back(neq);
     dfree(c->d_csr_grp);
@@ -2253,6 +2224,7 @@ int w3d_iteration_dev(w3d_ctx* c, int32_t step, int32_t iter,
     RecoverLists L;
     int rc = recover_lists(c, L);  // the resident lists
     if (rc) return rc;
+    L.host = c->h_rec;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
     rc = enqueue_recover(c, L, step_c, iter_c, extrapolated ? 1 : 0, d_u, d_du,

@@ -209,6 +209,7 @@ struct w3d_ctx {
   // solve allocates nothing
   int32_t* h_poll[2] = {};
   double* h_poll_sc = nullptr;
+  double* h_rec = nullptr;  // what a recovery leaves for the host
   hipEvent_t poll_ev[2] = {};
   // BiCGStab of the asymmetric CSR: b, x and the work vectors, allocated
   // with the gather map, once per pattern
@@ -283,6 +284,8 @@ struct RecoverLists {
   const WorkItem* d_w = nullptr;
   const WorkItem* d_wm = nullptr;
   int nwm = 0;
+  // the pinned image stage 3 writes for finish_recover (NULL: none)
+  double* host = nullptr;
   std::vector<int> sg, ss, sn;
 };
 

@@ -197,12 +197,19 @@ int launch_fill_i32(int32_t* d, int n, int32_t v, hipStream_t s);
 // index lies in [lo, hi) (rknstr_finish_cp), one workgroup per block.
 int launch_mm10_grads(const DevModel& M, const int32_t* d_blks, int nblks,
                       int lo, int hi, int step, hipStream_t s);
-int launch_ifv_gather(const double* einfvec, const int64_t* inv_ptr,
-                      const int64_t* inv_off, int nonode, double* ifv,
-                      hipStream_t s);
-int launch_energy_reduce(const double* en_wg, const int32_t* blk_wfirst,
-                         const int32_t* blk_wcount, int nblk,
-                         double* blk_sums, hipStream_t s);
+// The start of a recovery: flags cleared, and n words of u and du copied
+// to u_t and du_t (n = 0: none).  Its end, in one launch: the structure
+// forces into ifv (NULL: not formed), the sums of nblk blocks into blk_sums
+// and, where host is given (pinned, kBlkSums nblk + 2 words), those sums and
+// the four flags into it.
+int launch_recover_begin(int32_t* flags, int64_t n, const double* u,
+                         const double* du, double* u_t, double* du_t,
+                         hipStream_t s);
+int launch_recover_end(const double* einfvec, const int64_t* inv_ptr,
+                       const int64_t* inv_off, int nonode, double* ifv,
+                       const double* en_wg, const int32_t* blk_wfirst,
+                       const int32_t* blk_wcount, int nblk, double* blk_sums,
+                       const int32_t* flags, double* host, hipStream_t s);
 // Assembly over the segment map built by w3d_pattern: per segment a
 // header (contributions | component mask << 8), its contributions' first
 // Ke words in src, and per 64 segments the index of the first contribution

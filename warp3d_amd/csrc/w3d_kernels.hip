@@ -12,6 +12,8 @@
 //   assem_by_row.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "w3d_geonl.h"
 #include "w3d_internal.h"
 
@@ -811,42 +813,98 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------
 // Gathers (deterministic: each output sums its inputs in a fixed order)
 // ---------------------------------------------------------------------
-__global__ void k_ifv_gather(const double* __restrict__ einfvec,
-                             const int64_t* __restrict__ inv_ptr,
-                             const int64_t* __restrict__ inv_off, int nonode,
-                             double* __restrict__ ifv) {
-  const int n = (int)xcd_block(blockIdx.x, gridDim.x) * blockDim.x +
-                threadIdx.x;
-  if (n >= nonode) return;
+// Terms whose loads are in flight together in the ordered sums below.
+constexpr int kGatherAhead = 8;
+
+// The force of node n: its (node, element) pairs in inverse-incidence
+// order, their loads kGatherAhead pairs ahead of the sums (a chain of two
+// dependent loads a pair took 14.8 us on tetrahedra, 24 pairs a node; now 7.4).
+__device__ inline void ifv_node(const double* __restrict__ einfvec,
+                                const int64_t* __restrict__ inv_ptr,
+                                const int64_t* __restrict__ inv_off, int n,
+                                double* __restrict__ ifv) {
   double fx = 0.0, fy = 0.0, fz = 0.0;
-  for (int64_t p = inv_ptr[n]; p < inv_ptr[n + 1]; ++p) {
-    int64_t o = inv_off[p];  // the node's 3 contiguous force words
-    fx = fx + einfvec[o];
-    fy = fy + einfvec[o + 1];
-    fz = fz + einfvec[o + 2];
+  const int64_t p1 = inv_ptr[n + 1];
+  for (int64_t p = inv_ptr[n]; p < p1; p += kGatherAhead) {
+    int64_t o[kGatherAhead];  // the node's 3 contiguous force words
+    double x[kGatherAhead], y[kGatherAhead], z[kGatherAhead];
+#pragma unroll
+    for (int k = 0; k < kGatherAhead; ++k)
+      o[k] = inv_off[p + k < p1 ? p + k : p1 - 1];
+#pragma unroll
+    for (int k = 0; k < kGatherAhead; ++k) {
+      x[k] = einfvec[o[k]];
+      y[k] = einfvec[o[k] + 1];
+      z[k] = einfvec[o[k] + 2];
+    }
+#pragma unroll
+    for (int k = 0; k < kGatherAhead; ++k) {
+      const bool in = p + k < p1;  // (a sum is never -0, so + 0 is exact)
+      fx = fx + (in ? x[k] : 0.0);
+      fy = fy + (in ? y[k] : 0.0);
+      fz = fz + (in ? z[k] : 0.0);
+    }
   }
   ifv[3 * n] = fx;
   ifv[3 * n + 1] = fy;
   ifv[3 * n + 2] = fz;
 }
 
-// Per-block internal energy, plastic work and sum of |element force|: the
-// block's chunk sums in element order (one thread per block).
-__global__ void k_energy_reduce(const double* __restrict__ en_wg,
-                                const int32_t* __restrict__ wfirst,
-                                const int32_t* __restrict__ wcount, int nblk,
-                                double* __restrict__ sums) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nblk) return;
-  double en = 0.0, pw = 0.0, fa = 0.0;
-  for (int w = wfirst[b]; w < wfirst[b] + wcount[b]; ++w) {
-    en = en + en_wg[kBlkSums * w];
-    pw = pw + en_wg[kBlkSums * w + 1];
-    fa = fa + en_wg[kBlkSums * w + 2];
+// Internal energy, plastic work and sum of |element force| of block b: its
+// chunk sums in element order.
+__device__ inline void block_sums(const double* __restrict__ en_wg,
+                                  int wfirst, int wcount, double (&s)[3]) {
+  s[0] = s[1] = s[2] = 0.0;
+  for (int w = 0; w < wcount; w += kGatherAhead) {
+    double v[kGatherAhead][kBlkSums];
+#pragma unroll
+    for (int k = 0; k < kGatherAhead; ++k) {
+      const int i = wfirst + (w + k < wcount ? w + k : wcount - 1);
+#pragma unroll
+      for (int j = 0; j < kBlkSums; ++j) v[k][j] = en_wg[kBlkSums * i + j];
+    }
+#pragma unroll
+    for (int k = 0; k < kGatherAhead; ++k)
+#pragma unroll
+      for (int j = 0; j < kBlkSums; ++j)
+        s[j] = s[j] + (w + k < wcount ? v[k][j] : 0.0);
   }
-  sums[kBlkSums * b] = en;
-  sums[kBlkSums * b + 1] = pw;
-  sums[kBlkSums * b + 2] = fa;
+}
+
+// The end of a recovery: workgroups 0 .. ngather-1 sum the structure
+// forces, the others the blocks' energies (a thread per block) into sums
+// and, with the recovery flags, into the host image (pinned memory the
+// device writes: nblk blocks of kBlkSums words, then the four flags).  The
+// two have no input in common, so they share a launch.
+__global__ void __launch_bounds__(256)
+    k_recover_end(const double* __restrict__ einfvec,
+                  const int64_t* __restrict__ inv_ptr,
+                  const int64_t* __restrict__ inv_off, int nonode,
+                  double* __restrict__ ifv, int ngather,
+                  const double* __restrict__ en_wg,
+                  const int32_t* __restrict__ wfirst,
+                  const int32_t* __restrict__ wcount, int nblk,
+                  double* __restrict__ sums,
+                  const int32_t* __restrict__ flags,
+                  double* __restrict__ host) {
+  if ((int)blockIdx.x < ngather) {
+    const int n =
+        (int)xcd_block(blockIdx.x, ngather) * blockDim.x + threadIdx.x;
+    if (n < nonode) ifv_node(einfvec, inv_ptr, inv_off, n, ifv);
+    return;
+  }
+  const int b = (blockIdx.x - ngather) * blockDim.x + threadIdx.x;
+  if (b < nblk) {
+    double s[3];
+    block_sums(en_wg, wfirst[b], wcount[b], s);
+#pragma unroll
+    for (int j = 0; j < kBlkSums; ++j) {
+      sums[kBlkSums * b + j] = s[j];
+      if (host) host[kBlkSums * b + j] = s[j];
+    }
+  }
+  if (host && b < 4)
+    reinterpret_cast<int32_t*>(host + kBlkSums * nblk)[b] = flags[b];
 }
 
 // Row-by-row assembly (assem_a_row, assemble_code.f:785) over the segment
@@ -1041,23 +1099,39 @@ int launch_fill_i32(int32_t* d, int n, int32_t v, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
-int launch_ifv_gather(const double* einfvec, const int64_t* inv_ptr,
-                      const int64_t* inv_off, int nonode, double* ifv,
-                      hipStream_t s) {
-  int nb = (nonode + 255) / 256;
-  if (nb > 0)
-    hipLaunchKernelGGL(k_ifv_gather, dim3(nb), dim3(256), 0, s, einfvec,
-                       inv_ptr, inv_off, nonode, ifv);
+// The start of a recovery: its four flags cleared and, for finite strains,
+// the displacements kept for the tangent (n words each).
+__global__ void k_recover_begin(int32_t* __restrict__ flags, int64_t n,
+                                const double* u, const double* du,
+                                double* u_t, double* du_t) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < 4) flags[k] = 0;
+  if (k < n) {
+    u_t[k] = u[k];
+    du_t[k] = du[k];
+  }
+}
+
+int launch_recover_begin(int32_t* flags, int64_t n, const double* u,
+                         const double* du, double* u_t, double* du_t,
+                         hipStream_t s) {
+  const int64_t nb = n > 256 ? (n + 255) / 256 : 1;
+  hipLaunchKernelGGL(k_recover_begin, dim3((unsigned)nb), dim3(256), 0, s,
+                     flags, n, u, du, u_t, du_t);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
-int launch_energy_reduce(const double* en_wg, const int32_t* wfirst,
-                         const int32_t* wcount, int nblk, double* sums,
-                         hipStream_t s) {
-  int nb = (nblk + 63) / 64;
-  if (nb > 0)
-    hipLaunchKernelGGL(k_energy_reduce, dim3(nb), dim3(64), 0, s, en_wg,
-                       wfirst, wcount, nblk, sums);
+int launch_recover_end(const double* einfvec, const int64_t* inv_ptr,
+                       const int64_t* inv_off, int nonode, double* ifv,
+                       const double* en_wg, const int32_t* blk_wfirst,
+                       const int32_t* blk_wcount, int nblk, double* blk_sums,
+                       const int32_t* flags, double* host, hipStream_t s) {
+  const int ng = ifv ? (nonode + 255) / 256 : 0;
+  const int ns = nblk > 0 || host ? std::max(1, (nblk + 255) / 256) : 0;
+  if (ng + ns > 0)
+    hipLaunchKernelGGL(k_recover_end, dim3(ng + ns), dim3(256), 0, s, einfvec,
+                       inv_ptr, inv_off, nonode, ifv, ng, en_wg, blk_wfirst,
+                       blk_wcount, nblk, blk_sums, flags, host);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 
