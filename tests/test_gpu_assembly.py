@@ -45,3 +45,24 @@ def test_assembled_matrix(kind, fixed):
     for prec, rtol in ((_abi.W3D_FP64, RTOL_FP64), (_abi.W3D_FP32, 2e-6)):
         d.tangent(1, 1, prec)
         assert_close(np.concatenate(d.assemble_vss()), ko, rtol, kind)
+
+
+@pytest.mark.parametrize("n", [11, 15, 19, 24])
+def test_tangent_work_items(n):
+    """The tangent's work items of 4, 8, 16 and 32 bricks (256 compute
+    units), in blocks whose last item is short."""
+    from warp3d_amd.model import BlockModel
+    m = M.box_hex8(n, jitter=0.05, seed=n)
+    mat = _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0)
+    arr = m.model(mat, auto_size=61)
+    d, o = BlockModel(arr), O.OracleModel(arr)
+    u, du = np.zeros(3 * m.nonode), smooth_field(m, 0.002, seed=2)
+    for x in (d, o):
+        x.recover(1, 1, u, du)
+    o.tangent(1, 1)
+    for prec, rtol in ((_abi.W3D_FP64, RTOL_FP64), (_abi.W3D_FP32, 2e-6)):
+        d.tangent(1, 1, prec)
+        which = _abi.ESTIFF
+        for b in range(1, o.nelblk + 1, 7):
+            assert_close(d.get_block_state(b, which),
+                         o.get_block_state(b, which), rtol, f"block {b}")

@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -88,15 +89,28 @@ void build_work(const w3d_ctx* c, bool tangent, std::vector<WorkItem>& items,
                 std::vector<int>& groups, std::vector<int>& start,
                 std::vector<int>& count) {
   std::vector<std::pair<int, WorkItem>> all;
+  auto key_of = [&](const BlockDesc& B) {
+    return group_key(B.nnode, B.ngp, B.bbar,
+                     !tangent && B.model == W3D_MM10, B.geonl,
+                     tangent && B.trn);
+  };
+  std::map<int, int64_t> nelem;  // elements of each kernel group
+  for (const BlockDesc& B : c->blocks) nelem[key_of(B)] += B.span;
   for (int b = 0; b < c->nelblk; ++b) {
     const BlockDesc& B = c->blocks[b];
-    int key = group_key(B.nnode, B.ngp, B.bbar,
-                        !tangent && B.model == W3D_MM10, B.geonl,
-                        tangent && B.trn);
+    const int key = key_of(B);
     int E = tangent ? tan_mfma_chunk(B.nnode) : rec_elems(B.ngp);
-    if (tangent)
+    if (tangent) {
+      // a group of less than three workgroups on two compute units takes
+      // smaller items, down to an element a wave (tangent of 1,000 bricks,
+      // FP64: 26.3 us in items of 32, 15.3 of 16, 9.7 of 4; of 10,296
+      // tetrahedra 28.1 us of 32, 22.3 of 16, 26.5 of 8); larger groups lose
+      // by it (14,400 bricks, FP32: 29.3 us of 32, 33.9 of 16)
+      while (E > tan_mfma_waves(B.nnode) && nelem[key] / E < 3 * c->n_cu / 2)
+        E /= 2;
       for (const auto& kc : c->tan_chunk)
         if (kc.first == key) E = kc.second;
+    }
     for (int f = 0; f < B.span; f += E) {
       WorkItem w;
       w.blk = b;

@@ -201,9 +201,12 @@ __global__ void __launch_bounds__(64 * tan_mfma_waves(NN))
   if (tid < G) s_w[tid] = gt->w[tid];
   __syncthreads();
 
-  // each wave takes batches of EB consecutive elements of the work item
-  for (int b0 = wv * EB; b0 < wi.count; b0 += W * EB) {
-    const int nb = wi.count - b0 < EB ? wi.count - b0 : EB;
+  // each wave takes batches of consecutive elements of the work item: EB of
+  // them, or an equal share of a smaller item
+  const int share = (wi.count + W - 1) / W;
+  const int eb = share < EB ? share : EB;
+  for (int b0 = wv * eb; b0 < wi.count; b0 += W * eb) {
+    const int nb = wi.count - b0 < eb ? wi.count - b0 : eb;
     const int ie0 = wi.first + b0;
     wave_sync();
     // S1: nodes and coordinates of the batch (lanes = element x node)
