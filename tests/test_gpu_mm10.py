@@ -160,3 +160,17 @@ def test_mm10_cut_step_status(W):
     _, _, _, rco = orc.recover(2, 1, u, du)
     _, _, _, rcd = dev.recover(2, 1, u, du)
     assert rco == rcd == _abi.W3D_CUT_STEP
+
+
+@pytest.mark.parametrize("span,ncry,n,m_exp", [
+    (1, 1, 20.0, 1.0), (2, 3, 17.5, 1.3), (3, 1, 10.0, 5.0),
+    (9, 2, 20.0, 1.0), (27, 1, 17.5, 2.0)])
+def test_mm10_parts_and_exponents(W, span, ncry, n, m_exp):
+    """Work items whose last part has 8 to 16 points, several crystals, and
+    exponents that take pow as well as repeated squaring."""
+    m = M.box_hex8(3, jitter=0.1, seed=span)
+    ang = M.random_orientations(m.noelem, seed=7, per_element=ncry)
+    mat = cubic_fcc(ncrystals=ncry, harden_n=n, voce_m=m_exp)
+    arr = m.model(mat, auto_size=span, angles=ang, angle_stride=ncry)
+    run(W.BlockModel(arr), O.OracleModel(arr), m, ncry=ncry,
+        tag=f"span {span}")

@@ -19,6 +19,10 @@ SOURCES = ["w3d_api.cpp", "w3d_elements.cpp", "w3d_mm10_setup.cpp",
            "w3d_kernels.hip", "w3d_tangent.hip", "w3d_mm10.hip",
            "w3d_solver.hip", "w3d_serve.cpp", "w3d_asym.hip"]
 
+# The crystal update's loops hold all their registers can: constants and
+# addresses hoisted out of them only came back as spills.
+FLAGS = {"w3d_mm10.hip": ["-mllvm", "-disable-machine-licm"]}
+
 
 def hipcc():
     for cand in (os.environ.get("HIPCC"), "/opt/rocm/bin/hipcc",
@@ -41,8 +45,8 @@ def build(verbose=False, jobs=8):
     for src in SOURCES:
         obj = os.path.join(objdir, src + ".o")
         objs.append(obj)
-        cmd = [cc] + common + ["-x", "hip", "-c", os.path.join(CSRC, src),
-                               "-o", obj]
+        cmd = [cc] + common + FLAGS.get(src, []) + [
+            "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE,

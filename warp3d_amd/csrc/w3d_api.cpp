@@ -603,8 +603,8 @@ int create_impl(w3d_ctx* c, const w3d_model* m) {
   HIPCHK(hipMemset(c->d_counter, 0, 4 * sizeof(int32_t)));
   HIPCHK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount,
                                c->device));
-  // persistent mm10: one wave per SIMD fits (registers), four per CU
-  c->mm10_grid = 4 * std::max(c->n_cu, 1);
+  // persistent mm10: two waves per SIMD fit (registers), eight per CU
+  c->mm10_grid = 8 * std::max(c->n_cu, 1);
   {
     std::vector<WorkItem> items;
     build_work(c, false, items, c->rec_groups, c->rec_start, c->rec_count);

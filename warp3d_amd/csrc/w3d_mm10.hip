@@ -1,5 +1,5 @@
 // w3d_mm10.hip -- gfx950 kernel of the mm10 crystal-plasticity update
-// (Voce hardening, 12 fcc or bcc slip systems), one thread per Gauss point.
+// (Voce hardening, 12 fcc or bcc slip systems), four lanes per Gauss point.
 //
 // Reference routines restated (file:line under the reference's src/):
 //   rstgp1.f:4327 drive_10_update ([R n+1] of the polar decomposition for
@@ -19,13 +19,15 @@
 //   sign(slip) factor on its rate term, :1978-1983, kept as written).
 //
 // Every array of the local problem has compile-time indices, so the whole
-// solve stays in registers; the pivoting of the small LU factorisations is
-// done with selects instead of indexed row swaps.  Operation order follows
-// the reference loop by loop (LAPACK/BLAS calls in their unblocked
-// reference-BLAS order), except that each slip system's resolved shear is
-// formed once per residual evaluation and reused (bitwise the value the
-// reference recomputes).
+// solve stays in registers; the pivoting of the small eliminations is done
+// with selects instead of indexed row swaps.  Operation order follows the
+// reference, except that sums over the slip systems run as three systems a
+// lane and two exchanges in the quad, that C (D - dbar) is C D less the
+// systems' C ms, and that each system's resolved shear and its power are
+// formed once per residual or Jacobian and reused.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "w3d_internal.h"
 
@@ -33,6 +35,14 @@ namespace w3d {
 namespace {
 
 constexpr int NS = 12;
+// Four lanes (a quad) share a point: lane `sub` of the quad owns the slip
+// systems 3 sub .. 3 sub + 2 and, of a matrix, the columns sub, sub + 4 (and
+// sub + 8).  Sums over the systems are a partial sum of the lane's three and
+// two exchanges inside the quad, which leave the same bits in all four
+// lanes, so a quad's lanes always branch together.
+constexpr int NSL = 3;            // systems of a lane
+constexpr int kLanes = 64;
+constexpr int kPts = kLanes / 4;  // points of a wave
 
 struct Props {
   const CrystalDev* cr;
@@ -41,31 +51,69 @@ struct Props {
   int miter, alter_mode, angle_type;
 };
 
-// crystal_state of one crystal (the Voce subset).  The slip tensors
+// A lane's part of crystal_state (the Voce subset).  The slip tensors
 // (mm10_setup's ms, qc) depend only on the plastic rotation at n and R n+1,
-// so every sub-step shares one copy.
-// The rotated ms live in LDS, one column per lane (word w of lane t at
-// g[w * kLanes + t]), so that the local problem's registers stay free; qs
-// is formed where it is used from the crystal's reference vectors and the
-// 3x3 rotation rw (mm10_rt2rvw), which keeps the LDS of a workgroup at
-// 72 words a lane (four one-wave workgroups per compute unit).
-constexpr int kLanes = 64;
-constexpr int kGeoWords = 72;
+// so every sub-step shares one copy: ms and qc of the lane's systems, and
+// their products C ms, which every residual and Jacobian takes (in LDS, word
+// w of lane t at cms[w * kLanes + t]), and sigma_n + C D of the increment (LDS
+// too, word w of point t at trial[w * kPts + t]).
 struct CState {
-  double D[6];
+  double* trial;
   double tt_rate, tinc, dg;
-  const double* g;           // 72 ms words, lane-strided
-  const double (*q0)[3];     // reference qs of the 12 systems
-  double rw[9];              // RT2RVW(R Rp_n^T), column-major
-  __device__ double ms(int i, int k) const { return g[(6 * i + k) * kLanes]; }
-  // the lattice-spin vector of system i: rw q0[i] (mv3); qc of the
-  // reference, or qs for a state whose rw is RT2RVW(Rp_n^T)
-  __device__ void qs3(int i, double* q) const {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      q[k] = rw[k] * q0[i][0] + rw[k + 3] * q0[i][1] + rw[k + 6] * q0[i][2];
-  }
+  double ms[NSL][6];
+  double q[NSL][3];
+  const double* cms;
+  int sub;
+  __device__ double cm(int j, int r) const { return cms[(6 * j + r) * kLanes]; }
 };
+
+template <int CTRL>
+__device__ inline int qperm(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ inline double qperm(double v) {
+  return __hiloint2double(qperm<CTRL>(__double2hiint(v)),
+                          qperm<CTRL>(__double2loint(v)));
+}
+// the quad's exchanges: with the neighbour (1 0 3 2), across (2 3 0 1)
+constexpr int kDppNext = 0xB1, kDppCross = 0x4E;
+template <typename T>
+__device__ inline T qsum(T v) {
+  v = v + qperm<kDppNext>(v);
+  return v + qperm<kDppCross>(v);
+}
+// the value of the quad's lane S
+template <int S, typename T>
+__device__ inline T qbcast(T v) {
+  return qperm<S * 0x55>(v);
+}
+// the argument of the lane's own number
+__device__ inline double qpick(int sub, double a, double b, double c,
+                               double d) {
+  const double lo = sub & 1 ? b : a, hi = sub & 1 ? d : c;
+  return sub & 2 ? hi : lo;
+}
+
+// a value that is the same in every lane, in scalar registers
+__device__ inline int uniform(int v) {
+  return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ inline double uniform(double v) {
+  return __hiloint2double(uniform(__double2hiint(v)),
+                          uniform(__double2loint(v)));
+}
+__device__ inline int64_t uniform(int64_t v) {
+  return (int64_t)(uint32_t)uniform((int)v) |
+         (int64_t)uniform((int)(v >> 32)) << 32;
+}
+
+// Orders a wave's own LDS traffic (its quads exchange through their slabs).
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 __device__ inline double sgn(double x) { return x >= 0.0 ? 1.0 : -1.0; }
 
@@ -73,24 +121,9 @@ __device__ inline double sgn(double x) { return x >= 0.0 ? 1.0 : -1.0; }
 // in [0, 127] (the rate and Voce exponents of practice, e.g. n = 20, m = 1
 // or 5: some ulps from the correctly rounded power, far inside the local
 // solve's tolerances), ocml's pow otherwise.  y is a material constant, so
-// the branch is uniform.
-__device__ inline double vpow(double x, double y) {
-  const int k = (int)y;
-  if ((double)k == y && k >= 0 && k < 128) {
-    double r = 1.0, b = x;
-#pragma unroll
-    for (int i = 0; i < 7; ++i) {
-      if (k >> i & 1) r = r * b;
-      if ((k >> i) > 1) b = b * b;
-    }
-    return r;
-  }
-  return pow(x, y);
-}
-
-// vpow over an array, in place: the exponent's bits are tested once for all
-// N values (uniform branches around straight runs of N products); every
-// value takes the products vpow takes.
+// the branch is uniform.  Over an array, in place: the exponent's bits are
+// tested once for all N values (uniform branches around straight runs of N
+// products).
 template <int N>
 __device__ inline void vpow_arr(double* v, double y) {
   const int k = (int)y;
@@ -115,6 +148,10 @@ __device__ inline void vpow_arr(double* v, double y) {
 #pragma unroll
     for (int j = 0; j < N; ++j) v[j] = pow(v[j], y);
   }
+}
+__device__ inline double vpow(double x, double y) {
+  vpow_arr<1>(&x, y);
+  return x;
 }
 
 // [b] c with b 3x3 column-major
@@ -183,78 +220,80 @@ __device__ inline void rt2rvw(const double* rt, double* rv) {
 #undef RT
 }
 
-// LU with partial pivoting (first largest |pivot|) and the solve of
-// nrhs right-hand sides, column-major with leading dimension N.  The
-// eliminations and substitutions do not skip zero multipliers as LAPACK's
-// loops do: across a wave the skip would be a divergent branch that saves
-// nothing, and adding a zero product changes no value (signed zeros
-// aside).
-template <int N, int NRHS>
-__device__ inline void lu_solve(double* a, double* b) {
-  int piv[N];
-  double rp[N];  // the pivots' reciprocals, for the back substitution
+// Gaussian elimination with partial pivoting (first largest |pivot|) of the
+// N columns the quad holds (column c in lane c & 3, slot c >> 2), with the
+// right-hand sides among the remaining slots.  A column's owner finds its
+// pivot and multipliers and the quad takes them from it; entries below the
+// diagonal of finished columns are left as they fall, nothing reads them.
+// rp: the pivots' reciprocals.  The eliminations do not skip zero
+// multipliers as LAPACK's loops do (a divergent branch that saves nothing;
+// adding a zero product changes no value, signed zeros aside).
+template <int N, int SLOTS, int J = 0>
+__device__ inline void quad_eliminate(double (&A)[SLOTS][7], double (&rp)[N]) {
+  if constexpr (J < N) {
+    double* col = A[J >> 2];
+    int p = J;
+    double amax = fabs(col[J]);
 #pragma unroll
-  for (int j = 0; j < N; ++j) {
-    int p = j;
-    double amax = fabs(a[j + N * j]);
-#pragma unroll
-    for (int i = j + 1; i < N; ++i) {
-      double v = fabs(a[i + N * j]);
+    for (int i = J + 1; i < N; ++i) {
+      const double v = fabs(col[i]);
       if (v > amax) {
         amax = v;
         p = i;
       }
     }
-    piv[j] = p;
+    p = qbcast<(J & 3)>(p);
 #pragma unroll
-    for (int i = j + 1; i < N; ++i) {
-      if (i == p) {
+    for (int i = J + 1; i < N; ++i) {
+      const bool sw = i == p;
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-          double t = a[j + N * k];
-          a[j + N * k] = a[i + N * k];
-          a[i + N * k] = t;
-        }
+      for (int s = 0; s < SLOTS; ++s) {
+        const double a = A[s][J], b = A[s][i];
+        A[s][J] = sw ? b : a;
+        A[s][i] = sw ? a : b;
       }
     }
-    const double r = 1.0 / a[j + N * j];
-    rp[j] = r;
+    const double r = 1.0 / col[J];
+    rp[J] = qbcast<(J & 3)>(r);
 #pragma unroll
-    for (int i = j + 1; i < N; ++i) a[i + N * j] = a[i + N * j] * r;
+    for (int i = J + 1; i < N; ++i) {
+      const double m = qbcast<(J & 3)>(col[i] * r);
 #pragma unroll
-    for (int k = j + 1; k < N; ++k) {
-      double t = -a[j + N * k];
-#pragma unroll
-      for (int i = j + 1; i < N; ++i)
-        a[i + N * k] = a[i + N * k] + a[i + N * j] * t;
+      for (int s = 0; s < SLOTS; ++s) A[s][i] = A[s][i] - m * A[s][J];
     }
+    quad_eliminate<N, SLOTS, J + 1>(A, rp);
   }
+}
+
+// Back substitution of NY right-hand sides of every lane against the
+// eliminated columns.
+template <int N, int SLOTS, int NY, int K = N - 1>
+__device__ inline void quad_backsub(const double (&A)[SLOTS][7],
+                                    const double (&rp)[N],
+                                    double (&y)[NY][N]) {
+  if constexpr (K >= 0) {
 #pragma unroll
-  for (int c = 0; c < NRHS; ++c) {
-    double* x = b + N * c;
+    for (int c = 0; c < NY; ++c) y[c][K] = y[c][K] * rp[K];
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
+    for (int i = 0; i < K; ++i) {
+      const double u = qbcast<(K & 3)>(A[K >> 2][i]);
 #pragma unroll
-      for (int i = j + 1; i < N; ++i) {
-        if (i == piv[j]) {
-          double t = x[j];
-          x[j] = x[i];
-          x[i] = t;
-        }
-      }
+      for (int c = 0; c < NY; ++c) y[c][i] = y[c][i] - y[c][K] * u;
     }
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-#pragma unroll
-      for (int i = k + 1; i < N; ++i) x[i] = x[i] - x[k] * a[i + N * k];
-    }
-#pragma unroll
-    for (int k = N - 1; k >= 0; --k) {
-      x[k] = x[k] * rp[k];
-#pragma unroll
-      for (int i = 0; i < k; ++i) x[i] = x[i] - x[k] * a[i + N * k];
-    }
+    quad_backsub<N, SLOTS, NY, K - 1>(A, rp, y);
   }
+}
+
+// A x = b, b the last column (lane 3, slot 1); x in all four lanes.
+template <int N>
+__device__ inline void quad_solve(double (&A)[2][7], double (&x)[N]) {
+  double rp[N], y[1][N];
+  quad_eliminate<N, 2>(A, rp);
+#pragma unroll
+  for (int i = 0; i < N; ++i) y[0][i] = qbcast<3>(A[1][i]);
+  quad_backsub<N, 2, 1>(A, rp, y);
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = y[0][i];
 }
 
 // DPOSV('U', 6, 1) with the stiffness
@@ -292,13 +331,32 @@ __device__ inline void chol_solve6(const double* __restrict__ ain, double* b) {
   }
 }
 
-// mm10_setup: effective strain increment (k_0 = 0: no geometric hardening)
-__device__ inline void setup(const Props& p, CState& s) {
+// mm10_setup of an increment D over tinc: effective strain increment (k_0 =
+// 0: no geometric hardening)
+__device__ inline void setup(const Props& p, CState& s, const double* D,
+                             double tinc) {
   const double twothirds = 2.0 / 3.0;
-  double t1 = s.D[0] * s.D[0] + s.D[1] * s.D[1] + s.D[2] * s.D[2];
-  double t2 = s.D[3] * s.D[3] + s.D[4] * s.D[4] + s.D[5] * s.D[5];
+  double t1 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
+  double t2 = D[3] * D[3] + D[4] * D[4] + D[5] * D[5];
+  s.tinc = tinc;
   s.dg = sqrt(twothirds * (t1 + 0.5 * t2));
-  if (p.alter_mode) s.dg = p.eps_dot_0_y * s.tinc;
+  if (p.alter_mode) s.dg = p.eps_dot_0_y * tinc;
+}
+
+// the trial stress sigma_n + C D of the increment
+__device__ inline void set_trial(const Props& p, CState& s, const double* D,
+                                 const double* sn, int64_t stride) {
+  const double* C = p.cr->C;
+  double t[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) t[i] = C[i] * D[0];
+#pragma unroll
+  for (int j = 1; j < 6; ++j)
+#pragma unroll
+    for (int i = 0; i < 6; ++i) t[i] = t[i] + C[i + 6 * j] * D[j];
+  // (the quad's lanes hold the same values; each writes them)
+#pragma unroll
+  for (int i = 0; i < 6; ++i) s.trial[i * kPts] = sn[i * stride] + t[i];
 }
 
 // mm10_a_mult_type_1: a = b c (3x3 column-major), the reference's order
@@ -311,49 +369,59 @@ __device__ inline void mul33(double* a, const double* b, const double* c) {
                      b[i + 6] * c[2 + 3 * j];
 }
 
-// mm10_setup: the slip tensors rotated by the plastic rotation at n.  The
-// rotation kept in the state (rw) is the one of qc, RT2RVW(R Rp_n^T)
-// (mm10_a.f:891-892); with small strains (rot null, R = I) R Rp_n^T is
-// Rp_n^T exactly and qc equals qs.  rot: the point's [R n+1], column-major
-// at rot[k * SG].
+// mm10_setup: the lane's slip tensors rotated by the plastic rotation at n,
+// and their products with the stiffness.  The vectors kept in the state are
+// qc, by RT2RVW(R Rp_n^T) (mm10_a.f:891-892); with small strains (rot null,
+// R = I) R Rp_n^T is Rp_n^T exactly and qc equals qs.  rot: the point's
+// [R n+1], column-major at rot[k * SG].
 __device__ inline void slip_geometry(const Props& p, const double* Rpn,
-                                     double* gl, CState& s,
+                                     double* cms, CState& s,
                                      const double* rot, int64_t SG) {
-  double tn[9], RE[36];
+  double tn[9], rw[9];
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) tn[i + 3 * j] = Rpn[j + 3 * i];
-  rt2rve(tn, RE);
   if (rot) {
     double R[9], w[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) R[k] = rot[k * SG];
     mul33(w, R, tn);
-    rt2rvw(w, s.rw);
+    rt2rvw(w, rw);
   } else {
-    rt2rvw(tn, s.rw);
+    rt2rvw(tn, rw);
   }
-  s.q0 = p.cr->qs;
+  {
+    double RE[36];
+    rt2rve(tn, RE);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    const double* m0 = p.cr->ms[i];
-    double m[6];
+    for (int i = 0; i < NSL; ++i) {
+      const double* m0 = p.cr->ms[NSL * s.sub + i];
+      mv3(s.q[i], rw, p.cr->qs[NSL * s.sub + i]);
 #pragma unroll
-    for (int r = 0; r < 6; ++r) m[r] = RE[r] * m0[0];
+      for (int r = 0; r < 6; ++r) s.ms[i][r] = RE[r] * m0[0];
 #pragma unroll
-    for (int j = 1; j < 6; ++j)
+      for (int j = 1; j < 6; ++j)
 #pragma unroll
-      for (int r = 0; r < 6; ++r) m[r] = m[r] + RE[r + 6 * j] * m0[j];
-#pragma unroll
-    for (int r = 0; r < 6; ++r) gl[(6 * i + r) * kLanes] = m[r];
+        for (int r = 0; r < 6; ++r)
+          s.ms[i][r] = s.ms[i][r] + RE[r + 6 * j] * m0[j];
+    }
   }
-  s.g = gl;
-}
-
-__device__ inline double rs_of(const CState& s, const double* x, int i) {
-  return x[0] * s.ms(i, 0) + x[1] * s.ms(i, 1) + x[2] * s.ms(i, 2) +
-         x[3] * s.ms(i, 3) + x[4] * s.ms(i, 4) + x[5] * s.ms(i, 5);
+  const double* C = p.cr->C;
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    double c[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) c[j] = C[r + 6 * j];
+#pragma unroll
+    for (int i = 0; i < NSL; ++i) {
+      double v = c[0] * s.ms[i][0];
+#pragma unroll
+      for (int j = 1; j < 6; ++j) v = v + c[j] * s.ms[i][j];
+      cms[(6 * i + r) * kLanes] = v;
+    }
+  }
+  s.cms = cms;
 }
 
 __device__ inline void symsw(const double* s, const double* w, double* sw) {
@@ -365,76 +433,66 @@ __device__ inline void symsw(const double* s, const double* w, double* sw) {
   sw[5] = 0.5 * (w[1] * (s[0] - s[2]) + w[0] * s[3] - w[2] * s[4]);
 }
 
-// resolved shears and slip increments at x (stress) and tau
+// resolved shears, (|rs| / tau)^(n-1) and slip increments of the lane's
+// systems at x (stress) and tau
 __device__ inline void slips(const Props& p, const CState& s, const double* x,
-                             double tt, double* rs, double* gam) {
-  // one reciprocal of tau for the twelve quotients (a few ulps from the
-  // quotients themselves, far inside the local solve's tolerances)
+                             double tt, double* rs, double* pw, double* gam) {
+  // one reciprocal of tau for the quotients (a few ulps from the quotients
+  // themselves, far inside the local solve's tolerances)
   const double itt = 1.0 / tt, dgt = s.dg * itt;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    rs[i] = rs_of(s, x, i);
-    gam[i] = fabs(rs[i] * itt);
+  for (int i = 0; i < NSL; ++i) {
+    rs[i] = x[0] * s.ms[i][0] + x[1] * s.ms[i][1] + x[2] * s.ms[i][2] +
+            x[3] * s.ms[i][3] + x[4] * s.ms[i][4] + x[5] * s.ms[i][5];
+    pw[i] = fabs(rs[i] * itt);
   }
-  vpow_arr<NS>(gam, p.rate_n - 1.0);
+  vpow_arr<NSL>(pw, p.rate_n - 1.0);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) gam[i] = dgt * gam[i] * rs[i];
+  for (int i = 0; i < NSL; ++i) gam[i] = dgt * pw[i] * rs[i];
 }
 
-// form_wp (with qc) and form_wbarp (with qs: a state whose rw is that
-// of Rp_n^T)
+// form_wp: the spin of all systems, qc weighted by slip and diffusion
 __device__ inline void form_w(const Props& p, const CState& s,
                               const double* rs, const double* gam, double* w) {
   w[0] = w[1] = w[2] = 0.0;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    double q[3];
-    s.qs3(i, q);
+  for (int i = 0; i < NSL; ++i) {
+    const double c = rs[i] * s.tinc * p.iD_v + gam[i];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) w[k] = w[k] + gam[i] * q[k];
-    double c = rs[i] * s.tinc * p.iD_v;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) w[k] = w[k] + c * q[k];
+    for (int k = 0; k < 3; ++k) w[k] = w[k] + c * s.q[i][k];
   }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) w[k] = qsum(w[k]);
 }
 
-// formR1 at x with tau tt, from the slips (rs, gam) at (x, tt)
+// formR1 at x, from the lane's slips (rs, gam) there: x - sigma_n -
+// C (D - dbar) + 2 sym(x) w, with C dbar summed from the systems' C ms
 __device__ inline void formR1_slips(const Props& p, const CState& s,
-                                    const double* sn, const double* x,
+                                    const double* x,
                                     const double* rs, const double* gam,
                                     double* R1) {
-  double dbar[6], wp[3], sw[6], w1[6];
+  double cd[6], wp[3], sw[6];
 #pragma unroll
-  for (int k = 0; k < 6; ++k) dbar[k] = 0.0;
+  for (int k = 0; k < 6; ++k) cd[k] = 0.0;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    double c = rs[i] * s.tinc * p.iD_v + gam[i];
+  for (int i = 0; i < NSL; ++i) {
+    const double c = rs[i] * s.tinc * p.iD_v + gam[i];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) dbar[k] = dbar[k] + c * s.ms(i, k);
+    for (int k = 0; k < 6; ++k) cd[k] = cd[k] + c * s.cm(i, k);
   }
   form_w(p, s, rs, gam, wp);
   symsw(x, wp, sw);
 #pragma unroll
-  for (int k = 0; k < 6; ++k) w1[k] = s.D[k] - dbar[k];
-  const double* C = p.cr->C;
-  double w2[6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) w2[i] = C[i] * w1[0];
-#pragma unroll
-  for (int j = 1; j < 6; ++j)
-#pragma unroll
-    for (int i = 0; i < 6; ++i) w2[i] = w2[i] + C[i + 6 * j] * w1[j];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) R1[k] = x[k] - sn[k] - w2[k] + 2.0 * sw[k];
+  for (int k = 0; k < 6; ++k)
+    R1[k] = x[k] - (s.trial[k * kPts] - qsum(cd[k])) + 2.0 * sw[k];
 }
 
 // formR1 at x with tau tt
 __device__ inline void formR1(const Props& p, const CState& s,
-                              const double* sn, const double* x, double tt,
-                              double* R1) {
-  double rs[NS], gam[NS];
-  slips(p, s, x, tt, rs, gam);
-  formR1_slips(p, s, sn, x, rs, gam, R1);
+                              const double* x, double tt, double* R1) {
+  double rs[NSL], pw[NSL], gam[NSL];
+  slips(p, s, x, tt, rs, pw, gam);
+  formR1_slips(p, s, x, rs, gam, R1);
 }
 
 // h_voche (tau_l = 0)
@@ -444,142 +502,127 @@ __device__ inline double h_voche(const Props& p, const double* gam, double tt,
   double ht = 1.0 - (tt - p.tau_y) / p.tau_v + 0.0 / (tt - p.tau_y);
   double f = vpow(fabs(ht), p.voce_m) * sgn(ht);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) h = h + f * fabs(gam[i]);
-  return tau_n + p.theta_0 * h;
+  for (int i = 0; i < NSL; ++i) h = h + f * fabs(gam[i]);
+  return tau_n + p.theta_0 * qsum(h);
 }
 
 // formR (7 residuals); records the hardening rate
-// (the reference evaluates the slips twice, in formR1 and here, from the
-// same arguments: once here, bitwise the same values)
-__device__ inline void formR(const Props& p, CState& s, const double* sn,
-                             double tau_n, const double* x, double* R) {
-  double rs[NS], gam[NS];
-  slips(p, s, x, x[6], rs, gam);
-  formR1_slips(p, s, sn, x, rs, gam, R);
+__device__ inline void formR(const Props& p, CState& s, double tau_n,
+                             const double* x, double* R) {
+  double rs[NSL], pw[NSL], gam[NSL];
+  slips(p, s, x, x[6], rs, pw, gam);
+  formR1_slips(p, s, x, rs, gam, R);
   double h = h_voche(p, gam, x[6], tau_n);
   R[6] = x[6] - h;
   s.tt_rate = (h - tau_n) / s.tinc;
 }
 
-// formJ11 (6x6, column-major) from the slips (rs, gam) at (x, tt); with
-// J12 also formJ's J12 column, from the same per-system vectors
-// 2 (sym(x) w_i) + C ms_i that J11 takes
-template <bool WITH_J12 = false>
-__device__ inline void formJ11_slips(const Props& p, const CState& s,
-                                     const double* x, double tt,
-                                     const double* rs, const double* gam,
-                                     double* J11, double* J12 = nullptr) {
-  const double* C = p.cr->C;
-  const double ptt = vpow(tt, p.rate_n);
-#pragma unroll
-  for (int k = 0; k < 36; ++k) J11[k] = 0.0;
-  double dp[NS];
-#pragma unroll
-  for (int i = 0; i < NS; ++i) dp[i] = fabs(rs[i]);
-  vpow_arr<NS>(dp, p.rate_n - 1.0);
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    double d = dp[i];
-    d = s.dg * p.rate_n / ptt * d;
-    double dgdt = d + s.tinc * p.iD_v;
-    double st[6], wv[6];
-    double qv[3];
-    s.qs3(i, qv);
-    symsw(x, qv, st);
-#pragma unroll
-    for (int r = 0; r < 6; ++r) wv[r] = 2.0 * st[r];
-#pragma unroll
-    for (int j = 0; j < 6; ++j)
-#pragma unroll
-      for (int r = 0; r < 6; ++r) wv[r] = wv[r] + C[r + 6 * j] * s.ms(i, j);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-      double t = dgdt * s.ms(i, c);
-#pragma unroll
-      for (int r = 0; r < 6; ++r) J11[r + 6 * c] = J11[r + 6 * c] + wv[r] * t;
-    }
-    if (WITH_J12) {
-      const double dgdh = -p.rate_n / tt * gam[i];
-#pragma unroll
-      for (int r = 0; r < 6; ++r) J12[r] = J12[r] + wv[r] * (1.0 * dgdh);
-    }
+// row r of column c (both known at compile time) of mm10_iw(w) + I
+template <int C>
+__device__ inline void add_iw(const double* w, double* col) {
+  if (C == 0) { col[3] = col[3] + w[2]; col[5] = col[5] + w[1]; }
+  if (C == 1) { col[3] = col[3] - w[2]; col[4] = col[4] + w[0]; }
+  if (C == 2) { col[4] = col[4] - w[0]; col[5] = col[5] - w[1]; }
+  if (C == 3) {
+    col[0] = col[0] + 2.0 * w[2]; col[1] = col[1] + 2.0 * w[2];
+    col[4] = col[4] + w[1]; col[5] = col[5] + w[0];
   }
-  double wp[3];
-  form_w(p, s, rs, gam, wp);
-  // + mm10_iw(wp), then + I
-  J11[0 + 6 * 3] = J11[0 + 6 * 3] + 2.0 * wp[2];
-  J11[0 + 6 * 5] = J11[0 + 6 * 5] + -2.0 * wp[1];
-  J11[1 + 6 * 3] = J11[1 + 6 * 3] + 2.0 * wp[2];
-  J11[1 + 6 * 4] = J11[1 + 6 * 4] + -2.0 * wp[0];
-  J11[2 + 6 * 4] = J11[2 + 6 * 4] + 2.0 * wp[0];
-  J11[2 + 6 * 5] = J11[2 + 6 * 5] + 2.0 * wp[1];
-  J11[3 + 6 * 0] = J11[3 + 6 * 0] + wp[2];
-  J11[3 + 6 * 1] = J11[3 + 6 * 1] + -wp[2];
-  J11[3 + 6 * 4] = J11[3 + 6 * 4] + -wp[1];
-  J11[3 + 6 * 5] = J11[3 + 6 * 5] + wp[0];
-  J11[4 + 6 * 1] = J11[4 + 6 * 1] + wp[0];
-  J11[4 + 6 * 2] = J11[4 + 6 * 2] + -wp[0];
-  J11[4 + 6 * 3] = J11[4 + 6 * 3] + wp[1];
-  J11[4 + 6 * 5] = J11[4 + 6 * 5] + wp[2];
-  J11[5 + 6 * 0] = J11[5 + 6 * 0] + wp[1];
-  J11[5 + 6 * 2] = J11[5 + 6 * 2] + -wp[1];
-  J11[5 + 6 * 3] = J11[5 + 6 * 3] + wp[0];
-  J11[5 + 6 * 4] = J11[5 + 6 * 4] + -wp[2];
-  // the zero entries of iw are added too: x + 0.0 == x
+  if (C == 4) {
+    col[1] = col[1] + -2.0 * w[0]; col[2] = col[2] + 2.0 * w[0];
+    col[3] = col[3] + -w[1]; col[5] = col[5] + -w[2];
+  }
+  if (C == 5) {
+    col[0] = col[0] + -2.0 * w[1]; col[2] = col[2] + 2.0 * w[1];
+    col[3] = col[3] + w[0]; col[4] = col[4] + w[2];
+  }
+  col[C] = col[C] + 1.0;
+}
+
+// formJ11 (N = 6) or formJ (N = 7) at (x, tt): the quad's lanes get the
+// columns they own (A[slot][row]), column by column, so that one column's
+// sums are live at a time.  |rs|^(n-1) / tau^n and the slips come from the
+// powers (|rs| / tau)^(n-1) of the residual's slips.
+template <int N, int C = 0>
+__device__ inline void jac_columns(const CState& s, const double (*wv)[6],
+                                   const double* dgdt, const double* e,
+                                   const double* wp, double sc,
+                                   double (&A)[2][7]) {
+  if constexpr (C < 6) {
+    double col[7];
 #pragma unroll
-  for (int i = 0; i < 6; ++i) J11[i + 6 * i] = J11[i + 6 * i] + 1.0;
+    for (int r = 0; r < 6; ++r) col[r] = 0.0;
+    double et = 0.0;
+#pragma unroll
+    for (int i = 0; i < NSL; ++i) {
+      const double t = dgdt[i] * s.ms[i][C];
+#pragma unroll
+      for (int r = 0; r < 6; ++r) col[r] = col[r] + wv[i][r] * t;
+      if (N == 7) et = et + e[i] * s.ms[i][C];
+    }
+#pragma unroll
+    for (int r = 0; r < 6; ++r) col[r] = qsum(col[r]);
+    add_iw<C>(wp, col);
+    if (N == 7) col[6] = -(sc * qsum(et));
+    const bool own = s.sub == (C & 3);
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+      A[C >> 2][r] = own ? col[r] : A[C >> 2][r];
+    jac_columns<N, C + 1>(s, wv, dgdt, e, wp, sc, A);
+  }
 }
 
-__device__ inline void formJ11(const Props& p, const CState& s,
-                               const double* x, double tt, double* J11) {
-  double rs[NS], gam[NS];
-  slips(p, s, x, tt, rs, gam);
-  formJ11_slips(p, s, x, tt, rs, gam, J11);
-}
-
-// formJ: the 7x7 Jacobian (column-major, leading dimension 7)
+template <int N>
 __device__ inline void formJ(const Props& p, const CState& s, const double* x,
-                             double* J) {
-  const double tt = x[6];
-  double rs[NS], gam[NS];
-  slips(p, s, x, tt, rs, gam);  // once for J11 and the rest (bitwise)
-  double J11[36];
-  double J12[6] = {0, 0, 0, 0, 0, 0};
-  formJ11_slips<true>(p, s, x, tt, rs, gam, J11, J12);
-  const double ht = 1.0 - (tt - p.tau_y) / p.tau_v + 0.0 / (tt - p.tau_y);
-  const double hm = vpow(fabs(ht), p.voce_m);
-  double et[6] = {0, 0, 0, 0, 0, 0};
-  double dp[NS];
+                             double tt, double (&A)[2][7]) {
+  double rs[NSL], pw[NSL], gam[NSL], wv[NSL][6], dgdt[NSL], e[NSL], wp[3];
+  slips(p, s, x, tt, rs, pw, gam);
+  const double itt = 1.0 / tt, nd = s.dg * p.rate_n * itt;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) dp[i] = fabs(rs[i]);
-  vpow_arr<NS>(dp, p.rate_n - 2.0);
+  for (int i = 0; i < NSL; ++i) {
+    dgdt[i] = nd * pw[i] + s.tinc * p.iD_v;
+    double st[6];
+    symsw(x, s.q[i], st);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    double c = hm * sgn(ht) * dp[i] * rs[i];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) et[k] = et[k] + c * s.ms(i, k);
+    for (int r = 0; r < 6; ++r) wv[i][r] = 2.0 * st[r] + s.cm(i, r);
   }
-  const double sc = p.theta_0 * s.dg * p.rate_n / vpow(tt, p.rate_n);
-  double etau = 0.0;
-  const double dty = tt - p.tau_y;
-  const double iht = 1.0 / fabs(ht), ntt = p.rate_n / tt;
+  form_w(p, s, rs, gam, wp);
+  double sc = 0.0, hm = 0.0, ht = 0.0;
+  if (N == 7) {
+    ht = 1.0 - (tt - p.tau_y) / p.tau_v + 0.0 / (tt - p.tau_y);
+    hm = vpow(fabs(ht), p.voce_m);
+    sc = p.theta_0 * nd;
 #pragma unroll
-  for (int i = 0; i < NS; ++i)
-    etau = etau + (p.voce_m * (-1.0 / p.tau_v - 0.0 / (dty * dty)) *
-                       (fabs(gam[i]) * iht) -
-                   fabs(gam[i]) * ntt * sgn(ht) * sgn(gam[i])) *
-                      hm;
-  etau = p.theta_0 * etau;
-  etau = 1.0 - etau;
+    for (int i = 0; i < NSL; ++i) e[i] = hm * sgn(ht) * sgn(rs[i]) * pw[i];
+  }
 #pragma unroll
-  for (int c = 0; c < 6; ++c)
+  for (int r = 0; r < 7; ++r) A[0][r] = A[1][r] = 0.0;
+  jac_columns<N>(s, wv, dgdt, e, wp, sc, A);
+  if (N == 7) {
+    // J12 and J22
+    double col[7], etau = 0.0;
 #pragma unroll
-    for (int r = 0; r < 6; ++r) J[r + 7 * c] = J11[r + 6 * c];
+    for (int r = 0; r < 6; ++r) col[r] = 0.0;
+    const double dty = tt - p.tau_y;
+    const double iht = 1.0 / fabs(ht), ntt = p.rate_n * itt;
 #pragma unroll
-  for (int r = 0; r < 6; ++r) J[r + 42] = J12[r];
+    for (int i = 0; i < NSL; ++i) {
+      const double dgdh = -ntt * gam[i];
 #pragma unroll
-  for (int c = 0; c < 6; ++c) J[6 + 7 * c] = -(sc * et[c]);
-  J[48] = etau;
+      for (int r = 0; r < 6; ++r) col[r] = col[r] + wv[i][r] * dgdh;
+      etau = etau + (p.voce_m * (-1.0 / p.tau_v - 0.0 / (dty * dty)) *
+                         (fabs(gam[i]) * iht) -
+                     fabs(gam[i]) * ntt * sgn(ht) * sgn(gam[i])) *
+                        hm;
+    }
+    const bool own = s.sub == 2;
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+      const double v = qsum(col[r]);
+      A[1][r] = own ? v : A[1][r];
+    }
+    const double v = 1.0 - p.theta_0 * qsum(etau);
+    A[1][6] = own ? v : A[1][6];
+  }
 }
 
 // (unrolled, so that the arrays it is given stay in registers)
@@ -596,14 +639,33 @@ __device__ inline double dot6(const double* a, const double* b) {
          a[5] * b[5];
 }
 
+// dx . (J^T R) of the columns the quad holds, then J dx = -R in place
+template <int N>
+__device__ inline double newton_step(double (&A)[2][7], const double* R,
+                                     int sub, double (&dx)[N]) {
+  double wv[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    wv[k] = 0.0;
+#pragma unroll
+    for (int l = 0; l < N; ++l) wv[k] = wv[k] + A[k][l] * R[l];
+  }
+#pragma unroll
+  for (int r = 0; r < N; ++r) A[1][r] = sub == 3 ? -R[r] : A[1][r];
+  quad_solve<N>(A, dx);
+  double d = qpick(sub, dx[0], dx[1], dx[2], dx[3]) * wv[0];
+  d = d + qpick(sub, dx[4], dx[5], N == 7 ? dx[N - 1] : 0.0, 0.0) * wv[1];
+  return qsum(d);
+}
+
 // mm10_solve: predictor (6x6 Newton at fixed extrapolated tau) then the
-// 7x7 corrector; Jg (49 words at stride jstride) receives the Jacobian of
-// the last corrector iteration
-__device__ __forceinline__ void solve(const Props& p, CState& s, const double* sn,
+// 7x7 corrector; Jl (49 words of the point at stride kPts, LDS) receives the
+// Jacobian of the last corrector iteration
+__device__ __forceinline__ void solve(const Props& p, CState& s, const double* D,
                       double tau_n, double tt_rate_n, const double* Dn,
                       int64_t dn_stride,
                       double* stress, double* tt, bool& fail, double dtinc,
-                      double* Jg, int64_t jstride) {
+                      double* Jl) {
   const double c = 1.0e-4, red = 0.5;
   const int mls = 10, mmin = 1;
   double x[7], inR1;
@@ -615,7 +677,7 @@ __device__ __forceinline__ void solve(const Props& p, CState& s, const double* s
 #pragma unroll
     for (int k = 0; k < 6; ++k) x1[k] = x[k];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) d1[k] = s.D[k];
+    for (int k = 0; k < 6; ++k) d1[k] = D[k];
     dtrace = (d1[0] + d1[1] + d1[2]) / 3.0;
     d1[0] = d1[0] - dtrace;
     d1[1] = d1[1] - dtrace;
@@ -648,37 +710,26 @@ __device__ __forceinline__ void solve(const Props& p, CState& s, const double* s
     t2 = d1[3] * d2[3] + d1[4] * d2[4] + d1[5] * d2[5];
     double cos_ang = t1 + t2 > 0.0 ? t1 + t2 : 0.0;
     double x2 = x[6] + cos_ang * tt_rate_n * dtinc;
-    formR1(p, s, sn, x1, x2, R1);
+    formR1(p, s, x1, x2, R1);
     double nR1 = sqrt(R1[0] * R1[0] + R1[1] * R1[1] + R1[2] * R1[2] +
                       R1[3] * R1[3] + R1[4] * R1[4] + R1[5] * R1[5]);
     inR1 = nR1;
     bool ok = true;
     int iter = 0;
     while (nR1 > p.atol1 && nR1 / inR1 > p.rtol1) {
-      double J11[36], dx1[6], wv[6];
-      formJ11(p, s, x1, x2, J11);
-      // J11^T R1 first: the factorisation below overwrites J11
-#pragma unroll
-      for (int j = 0; j < 6; ++j)
-        wv[j] = J11[0 + 6 * j] * R1[0] + J11[1 + 6 * j] * R1[1] +
-                J11[2 + 6 * j] * R1[2] + J11[3 + 6 * j] * R1[3] +
-                J11[4 + 6 * j] * R1[4] + J11[5 + 6 * j] * R1[5];
-      // J11 dx1 = -R1 in place: bitwise the solution of (-J11) dx1 = R1
-      // (the same pivots and multipliers; every other value negated)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) dx1[k] = -R1[k];
-      lu_solve<6, 1>(J11, dx1);
-      double alpha = 1.0;
+      double A[2][7], dx1[6];
+      formJ<6>(p, s, x1, x2, A);
       double dotR1 = R1[0] * R1[0] + R1[1] * R1[1] + R1[2] * R1[2] +
                      R1[3] * R1[3] + R1[4] * R1[4] + R1[5] * R1[5];
       double ls1 = 0.5 * dotR1;
-      double ls2 = c * dot6(dx1, wv);
+      double ls2 = c * newton_step<6>(A, R1, s.sub, dx1);
+      double alpha = 1.0;
       int ls = 0;
       for (;;) {
         double nlsx = ls1 + ls2 * alpha, xn[6];
 #pragma unroll
         for (int k = 0; k < 6; ++k) xn[k] = x1[k] + alpha * dx1[k];
-        formR1(p, s, sn, xn, x2, R1);
+        formR1(p, s, xn, x2, R1);
         dotR1 = R1[0] * R1[0] + R1[1] * R1[1] + R1[2] * R1[2] +
                 R1[3] * R1[3] + R1[4] * R1[4] + R1[5] * R1[5];
         nR1 = sqrt(dotR1);
@@ -707,45 +758,34 @@ __device__ __forceinline__ void solve(const Props& p, CState& s, const double* s
   {  // corrector
     int iter = 0;
     double R[7];
-    formR(p, s, sn, tau_n, x, R);
+    formR(p, s, tau_n, x, R);
     double dotR = 0.0;
 #pragma unroll
     for (int k = 0; k < 7; ++k) dotR = dotR + R[k] * R[k];
     double nR = sqrt(dotR), inR = nR;
     if (inR == 0.0) inR = inR1;
     while ((nR > p.atol && nR / inR > p.rtol) || iter < mmin) {
-      double J[49], dx[7], wv[7];
-      formJ(p, s, x, J);
-      // the tangent takes the last iteration's Jacobian: parked in
-      // global memory instead of held in registers across the loop
+      double A[2][7], dx[7];
+      formJ<7>(p, s, x, x[6], A);
+      // the tangent takes the last iteration's Jacobian: parked in LDS
+      // instead of held in registers across the loop
 #pragma unroll
-      for (int k = 0; k < 49; ++k) Jg[k * jstride] = J[k];
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int r = 0; r < 7; ++r)
+          if (s.sub + 4 * k < 7) Jl[(r + 7 * (s.sub + 4 * k)) * kPts] = A[k][r];
       dotR = 0.0;
 #pragma unroll
       for (int k = 0; k < 7; ++k) dotR = dotR + R[k] * R[k];
       double ls1 = 0.5 * dotR;
-#pragma unroll
-      for (int j = 0; j < 7; ++j) {
-        double t = 0.0;
-#pragma unroll
-        for (int l = 0; l < 7; ++l) t = t + J[l + 7 * j] * R[l];
-        wv[j] = t;
-      }
-      // J dx = -R in place: bitwise the solution of (-J) dx = R
-#pragma unroll
-      for (int k = 0; k < 7; ++k) dx[k] = -R[k];
-      lu_solve<7, 1>(J, dx);
+      double ls2 = c * newton_step<7>(A, R, s.sub, dx);
       double alpha = 1.0;
-      double dd = 0.0;
-#pragma unroll
-      for (int k = 0; k < 7; ++k) dd = dd + dx[k] * wv[k];
-      double ls2 = c * dd;
       int ls = 0;
       for (;;) {
         double nlsx = ls1 + ls2 * alpha, xn[7];
 #pragma unroll
         for (int k = 0; k < 7; ++k) xn[k] = x[k] + alpha * dx[k];
-        formR(p, s, sn, tau_n, xn, R);
+        formR(p, s, tau_n, xn, R);
         dotR = 0.0;
 #pragma unroll
         for (int k = 0; k < 7; ++k) dotR = dotR + R[k] * R[k];
@@ -820,141 +860,166 @@ __device__ inline void euler_angles(const Props& p, const double* Rp_in,
 }  // namespace
 
 // ---------------------------------------------------------------------
-// One thread per Gauss point of an mm10 block (all its crystals).
+// A quad of lanes per Gauss point of an mm10 block (all its crystals):
+// points kPts part .. kPts part + kPts - 1 of the work item on one wave.
+//
+// Latency and issue bound in FP64 (some 50 kflop a point in short dependent
+// runs).  With a lane a point the local problem's arrays (49 Jacobian words,
+// 12 systems) overflowed the 512 registers of a wave into 2.8 KB of scratch
+// a lane, whose reloads from the Infinity Cache every chain waited on at one
+// wave a SIMD; split over four lanes they fit half the registers, so two
+// waves share a SIMD, a wave runs the longest of 16 local solves instead of
+// 64, and small models spread over four times the waves.
 // ---------------------------------------------------------------------
+constexpr int kCmsWords = 6 * NSL * kLanes;  // LDS of a wave: C ms,
+constexpr int kJacWords = 49 * kPts;         // the parked Jacobians,
+constexpr int kTriWords = 6 * kPts;          // the trial stresses and the
+                                             // last accepted ones
+constexpr int kMemWords = kCmsWords + kJacWords + 2 * kTriWords;
+
 __device__ __forceinline__ void mm10_item(const DevModel& M,
-                                          const WorkItem wi, int step,
-                                          int iter0_off, double* s_geo) {
-  if ((int)threadIdx.x >= wi.count) return;
-  const BlockDesc bd = M.blocks[wi.blk];
-  const MatDesc md = M.mats[bd.mat];
-  const int G = bd.ngp;
-  const int64_t SG = (int64_t)bd.span * G;
-  const int64_t q = wi.first + threadIdx.x;  // point inside the block
+                                          const WorkItem wi, int part,
+                                          int step, int iter0_off,
+                                          double* s_mem) {
+  // (values the compiler may not carry in from outside the item, or across
+  // the local solves: addresses formed from them are formed where they are
+  // used instead of held in registers)
+  int lane = threadIdx.x;
+  asm volatile("" : "+v"(lane));
+  const int pt = lane >> 2;
+  int sub = lane & 3;
+  if (kPts * part + pt >= wi.count) return;
+  // (the block's and material's words are loaded per lane: the compiler
+  // cannot know that nothing written here aliases them)
+  const BlockDesc* bp = M.blocks + uniform(wi.blk);
+  struct {
+    int64_t q_off, hist_off;
+    int geonl;
+  } bd = {uniform(bp->q_off), uniform(bp->hist_off), uniform(bp->geonl)};
+  const CpDesc* mp = &M.mats[uniform(bp->mat)].cp;
+  const int G = uniform(bp->ngp);
+  const int64_t SG = (int64_t)uniform(bp->span) * G;
+  const int64_t crys_off = uniform(bp->crys_off);
+  const int64_t q = wi.first + kPts * part + pt;  // point inside the block
   const int elem = (int)(q / G);
-  const int ncry = bd.ncry;
+  const int ncry = uniform(bp->ncry);
   const double* hn = M.hist_n + bd.hist_off + q;
-  double* hn1 = M.hist_n1 + bd.hist_off + q;
   const double* sn9 = M.stress_n + 9 * bd.q_off + q;
-  double* sn1 = M.stress_n1 + 9 * bd.q_off + q;
-  double* cp = M.cep + 21 * bd.q_off + q;
   const double* ud = M.uddt + 6 * bd.q_off + q;
+  // the point's place in the output arrays
+  int qo = (int)q;
   // finite strains: [R n+1] of the point (the recovery's), else R = I
   const double* rot = bd.geonl ? M.rot_tmp + 9 * bd.q_off + q : nullptr;
-  // (inputs and sums are read from and kept in memory where they are
-  // needed, not held in registers across the local solves)
   const double dt = M.dt;
+  double* Jl = s_mem + kCmsWords + pt;
 
   Props p;
-  p.rate_n = md.cp.rate_n;
-  p.tau_y = md.cp.tau_y;
-  p.tau_v = md.cp.tau_v;
-  p.voce_m = md.cp.voce_m;
-  p.theta_0 = md.cp.theta_0;
-  p.iD_v = md.cp.iD_v;
-  p.eps_dot_0_y = md.cp.eps_dot_0_y;
-  p.atol = md.cp.atol;
-  p.atol1 = md.cp.atol1;
-  p.rtol = md.cp.rtol;
-  p.rtol1 = md.cp.rtol1;
-  p.miter = md.cp.miter;
-  p.alter_mode = md.cp.alter_mode;
-  p.angle_type = md.cp.angle_type;
+  p.rate_n = uniform(mp->rate_n);
+  p.tau_y = uniform(mp->tau_y);
+  p.tau_v = uniform(mp->tau_v);
+  p.voce_m = uniform(mp->voce_m);
+  p.theta_0 = uniform(mp->theta_0);
+  p.iD_v = uniform(mp->iD_v);
+  p.eps_dot_0_y = uniform(mp->eps_dot_0_y);
+  p.atol = uniform(mp->atol);
+  p.atol1 = uniform(mp->atol1);
+  p.rtol = uniform(mp->rtol);
+  p.rtol1 = uniform(mp->rtol1);
+  p.miter = uniform(mp->miter);
+  p.alter_mode = uniform(mp->alter_mode);
+  p.angle_type = uniform(mp->angle_type);
 
+  // words the quad holds alike are stored four at a time, a lane a word
+  // (n < 4: the last ones)
+  auto put = [&](double* w, int n, double a, double b, double c2, double d) {
+    const double v = qpick(sub, a, b, c2, d);
+    if (sub < n) w[sub * SG] = v;
+  };
   // crystal sums of the tangent, the stresses and the slips accumulate in
   // their output words (history 1-36, stress n+1 1-6, history 76-87), read
-  // back only by this thread
+  // back only by the lane that writes them
   double t_work = 0.0, p_work = 0.0, p_strain = 0.0;
   bool cut = false;
 
   for (int c = 0; c < ncry; ++c) {
-    p.cr = M.crys + bd.crys_off + (int64_t)elem * ncry + c;
+    p.cr = M.crys + crys_off + (int64_t)elem * ncry + c;
     const int64_t cb = (int64_t)(87 + 71 * c) * SG;
     // n-state of the crystal (mm10_copy_cc_hist; at step 1 the
     // mm10_init_cc_hist0 values)
     // (Dn, the n strain increment, is read where the predictor uses it)
-    double sn[6], Rpn[9], tau_n, tt_rate_n;
+    double tau_n, tt_rate_n;
     const double* Dn = step == 1 ? nullptr : hn + cb + 18 * SG;
-    if (step == 1) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sn[k] = sn9[k * SG];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) Rpn[k] = (k % 4 == 0) ? 1.0 : 0.0;
-      tau_n = p.tau_y + 1.0e-5;
-    } else {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sn[k] = hn[cb + k * SG];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) Rpn[k] = hn[cb + (9 + k) * SG];
-      tau_n = hn[cb + 42 * SG];
-    }
-    tt_rate_n = hn[cb + 58 * SG];
-
-    // np1 (mm10_setup_np1 + mm10_setup)
-    double* gl = s_geo + threadIdx.x;
+    const double* sn = step == 1 ? sn9 : hn + cb;
     CState np1;
-    slip_geometry(p, Rpn, gl, np1, rot, SG);
+    np1.sub = sub;
+    np1.trial = s_mem + kCmsWords + kJacWords + pt;
+    double* ostress = np1.trial + kTriWords;
+    {
+      double Rpn[9];
+      if (step == 1) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) np1.D[k] = ud[k * SG];
-    np1.tinc = dt;
-    np1.tt_rate = 0.0;
-    setup(p, np1);
-    // mm10_solve_strup
-    double stress[6], ostress[6], tt = tau_n, ott = tau_n;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) stress[k] = ostress[k] = sn[k];
-    double temp1 = dot6(np1.D, np1.D);
-    double temp2 = dot6(stress, stress);
-    const bool no_load = temp2 == 0.0 && temp1 == 0.0;
-    // the last corrector Jacobian lives in the crystal's n+1 history words
-    // 0-48 until the tangent has read it (mm10_store_cryhist then writes
-    // those words)
-    double* Jg = hn1 + cb;
-    bool fail = false;
-    double curr_tt_rate = 0.0;
-    double tangent[36];
-    // the crystal's tangent into the point's average (history words 0-35;
-    // stored as soon as it is formed, so that it does not stay live)
-    auto store_tangent = [&]() {
-      if (c == 0) {
-#pragma unroll
-        for (int k = 0; k < 36; ++k) hn1[k * SG] = tangent[k];
+        for (int k = 0; k < 9; ++k) Rpn[k] = (k % 4 == 0) ? 1.0 : 0.0;
+        tau_n = p.tau_y + 1.0e-5;
       } else {
 #pragma unroll
-        for (int k = 0; k < 36; ++k) hn1[k * SG] = hn1[k * SG] + tangent[k];
+        for (int k = 0; k < 9; ++k) Rpn[k] = hn[cb + (9 + k) * SG];
+        tau_n = hn[cb + 42 * SG];
       }
+      // np1 (mm10_setup_np1 + mm10_setup)
+      slip_geometry(p, Rpn, s_mem + lane, np1, rot, SG);
+    }
+    tt_rate_n = hn[cb + 58 * SG];
+    // mm10_solve_strup
+    double D[6], stress[6], tt = tau_n, ott = tau_n;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) D[k] = ud[k * SG];
+    np1.tt_rate = 0.0;
+    setup(p, np1, D, dt);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) stress[k] = sn[k * SG];
+    double temp1 = dot6(D, D);
+    double temp2 = dot6(stress, stress);
+    const bool no_load = temp2 == 0.0 && temp1 == 0.0;
+    bool fail = false;
+    double curr_tt_rate = 0.0;
+    // word k of the crystal's tangent into the point's average (history
+    // words 0-35, word sub + 4 i the lane's)
+    auto store_tangent = [&](int k, double v) {
+      double* hn1 = M.hist_n1 + bd.hist_off + qo;
+      hn1[k * SG] = c == 0 ? v : hn1[k * SG] + v;
     };
     if (iter0_off || no_load) {
       const double* C = p.cr->C;
 #pragma unroll
-      for (int k = 0; k < 36; ++k) tangent[k] = C[k];
-      store_tangent();
+      for (int i = 0; i < 9; ++i) store_tangent(sub + 4 * i, C[sub + 4 * i]);
       if (!no_load) {
         double R1[6];
-        formR1(p, np1, sn, stress, tt, R1);
+        set_trial(p, np1, D, sn, SG);
+        formR1(p, np1, stress, tt, R1);
 #pragma unroll
         for (int k = 0; k < 6; ++k) stress[k] = stress[k] - R1[k];
       }
     } else {
       // the sub-steps run on np1 itself, their increments scaled from
       // the point's full-step values in memory (ud, dt); np1's full-step
-      // D, tinc and dg are formed again after the loop, so that they are
-      // not held across the local solves
+      // values are formed again after the loop, so that they are not held
+      // across the local solves
       double frac = 0.0, sstep = 1.0;
       int cuts = 0;
-      CState& curr = np1;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) ostress[k * kPts] = stress[k];
       while (frac < 1.0) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) curr.D[k] = ud[k * SG] * (sstep + frac);
-        curr.tinc = dt * (sstep + frac);
-        curr.tt_rate = 0.0;
-        setup(p, curr);
+        for (int k = 0; k < 6; ++k) D[k] = ud[k * SG] * (sstep + frac);
+        np1.tt_rate = 0.0;
+        setup(p, np1, D, dt * (sstep + frac));
+        set_trial(p, np1, D, sn, SG);
         tt = tau_n;
-        solve(p, curr, sn, tau_n, tt_rate_n, Dn, SG, stress, &tt, fail,
-              dt * sstep, Jg, SG);
+        solve(p, np1, D, tau_n, tt_rate_n, Dn, SG, stress, &tt, fail,
+              dt * sstep, Jl);
         if (fail) {
 #pragma unroll
-          for (int k = 0; k < 6; ++k) stress[k] = ostress[k];
+          for (int k = 0; k < 6; ++k) stress[k] = ostress[k * kPts];
           tt = ott;
           sstep = sstep * 0.5;
           cuts = cuts + 1;
@@ -962,7 +1027,7 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
           fail = false;
         } else {
 #pragma unroll
-          for (int k = 0; k < 6; ++k) ostress[k] = stress[k];
+          for (int k = 0; k < 6; ++k) ostress[k * kPts] = stress[k];
           ott = tt;
           frac = frac + sstep;
         }
@@ -971,87 +1036,114 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
         cut = true;
         break;
       }
-      curr_tt_rate = curr.tt_rate;
+      curr_tt_rate = np1.tt_rate;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) np1.D[k] = ud[k * SG];
-      np1.tinc = dt;
-      setup(p, np1);
+      for (int k = 0; k < 6; ++k) D[k] = ud[k * SG];
+      setup(p, np1, D, dt);
     }
     np1.tt_rate = curr_tt_rate;
-    double eul[3] = {0, 0, 0}, Rp1[9], ee[6], slip[NS], u[15], ep6[6],
-           ed6[6];
-    double work_inc = 0.0, p_work_inc = 0.0, p_strain_inc = 0.0;
+    asm volatile("" : "+v"(sub), "+v"(qo));
+    // mm10_store_cryhist: each word is stored as soon as it is formed
+    double* h1 = M.hist_n1 + bd.hist_off + cb + qo;
+    double slip[NSL];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) Rp1[k] = 0.0;
+    for (int k = 0; k < NSL; ++k) slip[k] = 0.0;
+    put(h1, 4, stress[0], stress[1], stress[2], stress[3]);
+    put(h1 + 4 * SG, 2, stress[4], stress[5], 0.0, 0.0);
+    put(h1 + 18 * SG, 4, D[0], D[1], D[2], D[3]);
+    put(h1 + 22 * SG, 2, D[4], D[5], 0.0, 0.0);
+    put(h1 + 42 * SG, 4, tt, 0.0, 0.0, 0.0);  // and user words 1-3,
+    put(h1 + 46 * SG, 2, 0.0, 0.0, 0.0, 0.0);  // 4-5,
+    put(h1 + 51 * SG, 2, 0.0, 0.0, 0.0, 0.0);  // 9-10
+    put(h1 + 58 * SG, 1, np1.tt_rate, 0.0, 0.0, 0.0);
+    if (iter0_off || no_load) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) ee[k] = ep6[k] = ed6[k] = 0.0;
+      for (int k = 6; k < 18; k += 4) put(h1 + k * SG, 4, 0.0, 0.0, 0.0, 0.0);
+      put(h1 + 24 * SG, 4, 0.0, 0.0, 0.0, 0.0);
+      put(h1 + 28 * SG, 2, 0.0, 0.0, 0.0, 0.0);
+      put(h1 + 48 * SG, 3, 0.0, 0.0, 0.0, 0.0);
+      put(h1 + 53 * SG, 4, 0.0, 0.0, 0.0, 0.0);
+      put(h1 + 57 * SG, 1, 0.0, 0.0, 0.0, 0.0);
 #pragma unroll
-    for (int k = 0; k < NS; ++k) slip[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < 15; ++k) u[k] = 0.0;
-    if (!(iter0_off || no_load)) {
+      for (int k = 59; k < 71; k += 4) put(h1 + k * SG, 4, 0.0, 0.0, 0.0, 0.0);
+    } else {
       // ---- mm10_tangent: T = (J11 - J12 J21 / J22)^-1 C, symmetrised
-      // unless the assembly is asymmetric
-      double J[49], JJ[36], beta[12];
+      // unless the assembly is asymmetric.  Twelve columns in the quad: the
+      // six of J11 - J12 J21 / J22, then C's
+      {
+        const double* C = p.cr->C;
+        double A[3][7], rp[6], y[2][6];
+        wave_sync();
+        const double rj = 1.0 / Jl[48 * kPts];
 #pragma unroll
-      for (int k = 0; k < 49; ++k) J[k] = Jg[k * SG];
+        for (int k = 0; k < 2; ++k) {
+          const int cc = sub + 4 * k;
+          if (k == 0 || sub < 2) {
+            const double t = -(Jl[(6 + 7 * cc) * kPts] * rj);
 #pragma unroll
-      for (int cc = 0; cc < 6; ++cc)
+            for (int r = 0; r < 6; ++r)
+              A[k][r] = Jl[(r + 7 * cc) * kPts] + t * Jl[(r + 42) * kPts];
+          } else {
 #pragma unroll
-        for (int r = 0; r < 6; ++r) JJ[r + 6 * cc] = J[r + 7 * cc];
-      double a1 = J[48];
-#pragma unroll
-      for (int cc = 0; cc < 6; ++cc) {
-        beta[cc] = J[6 + 7 * cc];
-        beta[6 + cc] = 0.0;
-      }
-      lu_solve<1, 12>(&a1, beta);
-#pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        double t = -1.0 * beta[j];
-        if (t != 0.0) {
-#pragma unroll
-          for (int i = 0; i < 6; ++i) JJ[i + 6 * j] = JJ[i + 6 * j] + t * J[i + 42];
+            for (int r = 0; r < 6; ++r) A[k][r] = C[r + 6 * (sub - 2)];
+          }
         }
+#pragma unroll
+        for (int r = 0; r < 6; ++r) A[2][r] = C[r + 6 * (sub + 2)];
+        quad_eliminate<6, 3>(A, rp);
+#pragma unroll
+        for (int r = 0; r < 6; ++r) {
+          y[0][r] = A[1][r];
+          y[1][r] = A[2][r];
+        }
+        quad_backsub<6, 3, 2>(A, rp, y);
+        wave_sync();
+        if (sub >= 2)
+#pragma unroll
+          for (int r = 0; r < 6; ++r) Jl[(r + 6 * (sub - 2)) * kPts] = y[0][r];
+#pragma unroll
+        for (int r = 0; r < 6; ++r) Jl[(r + 6 * (sub + 2)) * kPts] = y[1][r];
+        wave_sync();
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+          const int k = sub + 4 * i;
+          double v = Jl[k * kPts];
+          // (kept as formed for asymmetric assembly, :1165)
+          if (!M.asym) v = (v + Jl[(k / 6 + 6 * (k % 6)) * kPts]) * 0.5;
+          store_tangent(k, v);
+        }
+        wave_sync();
       }
-      const double* C = p.cr->C;
-#pragma unroll
-      for (int k = 0; k < 36; ++k) tangent[k] = C[k] - 0.0 - 0.0;
-      lu_solve<6, 6>(JJ, tangent);
-      if (!M.asym) {  // kept as formed for asymmetric assembly (:1165)
-        double w[36];
-#pragma unroll
-        for (int j = 0; j < 6; ++j)
-#pragma unroll
-          for (int i = 0; i < 6; ++i)
-            w[i + 6 * j] = (tangent[i + 6 * j] + tangent[j + 6 * i]) * 0.5;
-#pragma unroll
-        for (int k = 0; k < 36; ++k) tangent[k] = w[k];
-      }
-      store_tangent();
       // ---- slips at the converged state (np1: full-step dg)
-      double rs[NS], gam[NS];
-      slips(p, np1, stress, tt, rs, gam);
+      double rs[NSL], pw[NSL], gam[NSL], wp[3];
+      slips(p, np1, stress, tt, rs, pw, gam);
+      form_w(p, np1, rs, gam, wp);
       // ---- mm10_update_rotation: Rp = expm(W(wbarp)) Rp_n (Rp_n read
       // again here)
       {
-        double Rpe[9];
+        double Rpe[9], Rp1[9], eul[3];
 #pragma unroll
         for (int k = 0; k < 9; ++k)
           Rpe[k] = step == 1 ? ((k % 4 == 0) ? 1.0 : 0.0)
                              : hn[cb + (9 + k) * SG];
-        double wb[3];
+        double wb[3] = {wp[0], wp[1], wp[2]};
         if (rot) {  // form_wbarp takes qs, of Rp_n alone
-          CState nq = np1;
-          double tn[9];
+          double tn[9], rw[9], w0[3] = {0.0, 0.0, 0.0};
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j) tn[i + 3 * j] = Rpe[j + 3 * i];
-          rt2rvw(tn, nq.rw);
-          form_w(p, nq, rs, gam, wb);
-        } else {
-          form_w(p, np1, rs, gam, wb);
+          rt2rvw(tn, rw);
+#pragma unroll
+          for (int i = 0; i < NSL; ++i) {
+            const double cw = rs[i] * np1.tinc * p.iD_v + gam[i];
+            double qi[3];
+            mv3(qi, rw, p.cr->qs[NSL * sub + i]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) w0[k] = w0[k] + cw * qi[k];
+          }
+#pragma unroll
+          for (int k = 0; k < 3; ++k) wb[k] = qsum(w0[k]);
         }
         double W[9] = {0.0, -wb[2], -wb[1], wb[2], 0.0, -wb[0],
                        wb[1], wb[0], 0.0};  // column-major of wv2wt
@@ -1087,28 +1179,38 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
           for (int i = 0; i < 3; ++i)
             Rp1[i + 3 * j] = A[i] * Rpe[0 + 3 * j] + A[i + 3] * Rpe[1 + 3 * j] +
                              A[i + 6] * Rpe[2 + 3 * j];
+        euler_angles(p, Rp1, eul, rot, SG);
+        put(h1 + 6 * SG, 4, eul[0], eul[1], eul[2], Rp1[0]);
+        put(h1 + 10 * SG, 4, Rp1[1], Rp1[2], Rp1[3], Rp1[4]);
+        put(h1 + 14 * SG, 4, Rp1[5], Rp1[6], Rp1[7], Rp1[8]);
       }
       // ---- mm10_output
+      double dif[NSL], edt[6], dbarp[6], t1, t2;
 #pragma unroll
-      for (int i = 0; i < NS; ++i) slip[i] = gam[i];
-      euler_angles(p, Rp1, eul, rot, SG);
-      double dif[NS], t1, t2;
+      for (int k = 0; k < 6; ++k) edt[k] = dbarp[k] = 0.0;
 #pragma unroll
-      for (int i = 0; i < NS; ++i) dif[i] = rs[i] * np1.tinc * p.iD_v;
+      for (int i = 0; i < NSL; ++i) {
+        dif[i] = rs[i] * np1.tinc * p.iD_v;
 #pragma unroll
-      for (int i = 0; i < NS; ++i)
+        for (int k = 0; k < 6; ++k) {
+          edt[k] = edt[k] + dif[i] * np1.ms[i][k];
+          dbarp[k] = dbarp[k] + gam[i] * np1.ms[i][k];
+        }
+      }
 #pragma unroll
-        for (int k = 0; k < 6; ++k) ed6[k] = ed6[k] + dif[i] * np1.ms(i, k);
-      double edt[6];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) edt[k] = ed6[k];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) ed6[k] = edt[k] / np1.tinc;
+      for (int k = 0; k < 6; ++k) {
+        edt[k] = qsum(edt[k]);
+        dbarp[k] = qsum(dbarp[k]);
+      }
+      put(h1 + 65 * SG, 4, edt[0] / np1.tinc, edt[1] / np1.tinc,
+          edt[2] / np1.tinc, edt[3] / np1.tinc);
+      put(h1 + 69 * SG, 2, edt[4] / np1.tinc, edt[5] / np1.tinc, 0.0, 0.0);
       t1 = edt[0] * edt[0] + edt[1] * edt[1] + edt[2] * edt[2];
       t2 = edt[3] * edt[3] + edt[4] * edt[4] + edt[5] * edt[5];
       double ed_dot = sqrt(2.0 / 3.0 * (t1 + 0.5 * t2));
-      u[14] = ed_dot / np1.tinc;
-      work_inc = dot6(stress, np1.D);
+      const double u14 = ed_dot / np1.tinc;
+      t_work = t_work + dot6(stress, D);
+      double ee[6];
 #pragma unroll
       for (int k = 0; k < 6; ++k) ee[k] = stress[k];
       chol_solve6(p.cr->C, ee);
@@ -1127,50 +1229,46 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
 #pragma unroll
         for (int k = 0; k < 6; ++k) ee[k] = t[k];
       }
-      double dbarp[6] = {0, 0, 0, 0, 0, 0}, wp[3], ewwe[6], ep[6];
-#pragma unroll
-      for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int k = 0; k < 6; ++k) dbarp[k] = dbarp[k] + slip[i] * np1.ms(i, k);
-      form_w(p, np1, rs, gam, wp);
+      put(h1 + 24 * SG, 4, ee[0], ee[1], ee[2], ee[3]);
+      put(h1 + 28 * SG, 2, ee[4], ee[5], 0.0, 0.0);
+      double ewwe[6], ep[6];
       symsw(ee, wp, ewwe);
 #pragma unroll
       for (int k = 0; k < 6; ++k) ep[k] = dbarp[k] + ewwe[k];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) ep6[k] = ep[k] / np1.tinc;
+      put(h1 + 59 * SG, 4, ep[0] / np1.tinc, ep[1] / np1.tinc,
+          ep[2] / np1.tinc, ep[3] / np1.tinc);
+      put(h1 + 63 * SG, 2, ep[4] / np1.tinc, ep[5] / np1.tinc, 0.0, 0.0);
       t1 = ep[0] * ep[0] + ep[1] * ep[1] + ep[2] * ep[2];
       t2 = ep[3] * ep[3] + ep[4] * ep[4] + ep[5] * ep[5];
-      u[10] = sqrt(2.0 / 3.0 * (t1 + 0.5 * t2)) / np1.tinc;
+      const double u10 = sqrt(2.0 / 3.0 * (t1 + 0.5 * t2)) / np1.tinc;
 #pragma unroll
       for (int k = 0; k < 6; ++k) ep[k] = ep[k] + edt[k];
       t1 = ep[0] * ep[0] + ep[1] * ep[1] + ep[2] * ep[2];
       t2 = ep[3] * ep[3] + ep[4] * ep[4] + ep[5] * ep[5];
-      p_strain_inc = sqrt(2.0 / 3.0 * (t1 + 0.5 * t2));
-      p_work_inc = dot6(stress, ep);
+      const double p_strain_inc = sqrt(2.0 / 3.0 * (t1 + 0.5 * t2));
+      p_strain = p_strain + p_strain_inc;
+      p_work = p_work + dot6(stress, ep);
       double ec_dot = p_strain_inc / np1.tinc, n_eff;
       if (ec_dot > 0.0) {
 #pragma unroll
         for (int k = 0; k < 6; ++k) ep[k] = ep[k] / np1.tinc;
         n_eff = 0.0;
-        const double ptt = vpow(tt, p.rate_n);
+        const double nd = np1.dg * p.rate_n / tt;
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-          double d = vpow(fabs(rs[i]), p.rate_n - 1.0);
-          d = np1.dg * p.rate_n / ptt * d;
-          double dgdt = d + np1.tinc * p.iD_v;
-          double a = np1.ms(i, 0) * ep[0] + np1.ms(i, 1) * ep[1] +
-                     np1.ms(i, 2) * ep[2];
-          double b = np1.ms(i, 3) * ep[3] + np1.ms(i, 4) * ep[4] +
-                     np1.ms(i, 5) * ep[5];
+        for (int i = 0; i < NSL; ++i) {
+          double dgdt = nd * pw[i] + np1.tinc * p.iD_v;
+          const double* m = np1.ms[i];
+          double a = m[0] * ep[0] + m[1] * ep[1] + m[2] * ep[2];
+          double b = m[3] * ep[3] + m[4] * ep[4] + m[5] * ep[5];
           double ec_slip = a + 0.5 * b;
           double q1 = rs[i] * dgdt / ec_dot;
           double q2 = ec_slip / ec_dot / np1.tinc;
           n_eff = n_eff + (2.0 / 3.0) * q1 * q2;
         }
+        n_eff = qsum(n_eff);
       } else {
         n_eff = 1.0e10;
       }
-      u[11] = n_eff;
       double s_tr = (stress[0] + stress[1] + stress[2]) / 3.0;
       double se0 = stress[0] - s_tr, se1 = stress[1] - s_tr,
              se2 = stress[2] - s_tr;
@@ -1178,7 +1276,6 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
       t2 = stress[3] * stress[3] + stress[4] * stress[4] +
            stress[5] * stress[5];
       s_tr = sqrt(1.5 * (t1 + 2.0 * t2));
-      u[12] = s_tr;
       double B_eff;
       if (ec_dot < 1.0e-100)
         B_eff = 0.0;
@@ -1186,102 +1283,100 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
         B_eff = -1.0;
       else
         B_eff = ec_dot / pow(s_tr, n_eff);
-      u[13] = B_eff;
+      put(h1 + 53 * SG, 4, u10, n_eff, s_tr, B_eff);
+      put(h1 + 57 * SG, 1, u14, 0.0, 0.0, 0.0);
 #pragma unroll
-      for (int i = 0; i < NS; ++i) slip[i] = slip[i] + dif[i];
+      for (int i = 0; i < NSL; ++i) slip[i] = gam[i] + dif[i];
+      // the first system of the largest slip, and the active systems
       double maxslip = 0.0;
       int sysID = 0;
 #pragma unroll
-      for (int i = 0; i < NS; ++i) {
+      for (int i = 0; i < NSL; ++i) {
         double cs = fabs(slip[i]);
         if (cs > maxslip) {
           maxslip = cs;
-          sysID = i + 1;
+          sysID = NSL * sub + i + 1;
         }
       }
-      u[5] = maxslip / np1.tinc;
-      u[6] = (double)sysID;
+      auto larger = [&](double om, int oid) {
+        const bool t = om > maxslip || (om == maxslip && oid < sysID);
+        maxslip = t ? om : maxslip;
+        sysID = t ? oid : sysID;
+      };
+      larger(qperm<kDppNext>(maxslip), qperm<kDppNext>(sysID));
+      larger(qperm<kDppCross>(maxslip), qperm<kDppCross>(sysID));
+      const double rate = maxslip / np1.tinc;
       int numAct = 0;
       maxslip = 0.1 * maxslip;
 #pragma unroll
-      for (int i = 0; i < NS; ++i)
+      for (int i = 0; i < NSL; ++i)
         if (fabs(slip[i]) >= maxslip) numAct = numAct + 1;
-      u[7] = (double)numAct;
+      put(h1 + 48 * SG, 3, rate, (double)sysID, (double)qsum(numAct), 0.0);
     }
     // accumulate for the averages
+    double* sn1 = M.stress_n1 + 9 * bd.q_off + qo;
+    double* hn1 = M.hist_n1 + bd.hist_off + qo;
 #pragma unroll
-    for (int k = 0; k < 6; ++k)
-      sn1[k * SG] = c == 0 ? stress[k] : sn1[k * SG] + stress[k];
+    for (int k = 0; k < 6; k += 4) {
+      const double v = qpick(sub, stress[k], stress[k + 1],
+                             k + 2 < 6 ? stress[(k + 2) % 6] : 0.0,
+                             k + 3 < 6 ? stress[(k + 3) % 6] : 0.0);
+      double* w = sn1 + (k + sub) * SG;
+      if (k + sub < 6) *w = c == 0 ? v : *w + v;
+    }
 #pragma unroll
-    for (int k = 0; k < NS; ++k)
-      hn1[(75 + k) * SG] = c == 0 ? slip[k] : hn1[(75 + k) * SG] + slip[k];
-    t_work = t_work + work_inc;
-    p_work = p_work + p_work_inc;
-    p_strain = p_strain + p_strain_inc;
-    // mm10_store_cryhist
-    double* h1 = hn1 + cb;
+    for (int i = 0; i < NSL; ++i) {
+      double* w = hn1 + (75 + NSL * sub + i) * SG;
+      *w = c == 0 ? slip[i] : *w + slip[i];
+    }
 #pragma unroll
-    for (int k = 0; k < 6; ++k) h1[k * SG] = stress[k];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) h1[(6 + k) * SG] = eul[k];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) h1[(9 + k) * SG] = Rp1[k];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) h1[(18 + k) * SG] = np1.D[k];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) h1[(24 + k) * SG] = ee[k];
-#pragma unroll
-    for (int k = 0; k < NS; ++k) h1[(30 + k) * SG] = slip[k];
-    h1[42 * SG] = tt;
-#pragma unroll
-    for (int k = 0; k < 15; ++k) h1[(43 + k) * SG] = u[k];
-    h1[58 * SG] = np1.tt_rate;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) h1[(59 + k) * SG] = ep6[k];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) h1[(65 + k) * SG] = ed6[k];
+    for (int i = 0; i < NSL; ++i) h1[(30 + NSL * sub + i) * SG] = slip[i];
   }
   if (cut) {
     atomicOr(&M.flags[1], 1);
     return;
   }
   const double rn = (double)ncry;
-  double tang_avg[36];
-#pragma unroll
-  for (int k = 0; k < 36; ++k) tang_avg[k] = hn1[k * SG] / rn;
+  double* sn1 = M.stress_n1 + 9 * bd.q_off + qo;
+  double* hn1 = M.hist_n1 + bd.hist_off + qo;
+  double* cp = M.cep + 21 * bd.q_off + qo;
   t_work = t_work / rn;
   p_work = p_work / rn;
   p_strain = p_strain / rn;
   // mm10_a_store_crystal
 #pragma unroll
-  for (int k = 0; k < 6; ++k) sn1[k * SG] = sn1[k * SG] / rn;
-  sn1[6 * SG] = sn9[6 * SG] + t_work;
-  sn1[7 * SG] = sn9[7 * SG] + p_work;
-  sn1[8 * SG] = sn9[8 * SG] + p_strain;
+  for (int k = 0; k < 6; k += 4)
+    if (k + sub < 6) sn1[(k + sub) * SG] = sn1[(k + sub) * SG] / rn;
+  // the tangent's average and [D] for the tangent kernel: the lower
+  // triangle of history words 1-36
 #pragma unroll
-  for (int k = 0; k < 36; ++k) hn1[k * SG] = tang_avg[k];
-#pragma unroll
-  for (int k = 36; k < 63; ++k) hn1[k * SG] = 0.0;
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-    hn1[(63 + k) * SG] = rot ? rot[k * SG] : ((k % 4 == 0) ? 1.0 : 0.0);
-  double w72 = step == 1 ? 0.0 : hn[72 * SG];
-  double w73 = step == 1 ? 0.0 : hn[73 * SG];
-  double w74 = step == 1 ? 0.0 : hn[74 * SG];
-  hn1[72 * SG] = w72 + t_work;
-  hn1[73 * SG] = w73 + p_work;
-  hn1[74 * SG] = w74 + p_strain;
-#pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    double base = step == 1 ? 0.0 : hn[(75 + k) * SG];
-    hn1[(75 + k) * SG] = base + hn1[(75 + k) * SG] / rn;
+  for (int i = 0; i < 9; ++i) {
+    const int k = sub + 4 * i, r = k % 6, cc = k / 6;
+    const double v = hn1[k * SG] / rn;
+    hn1[k * SG] = v;
+    if (cc <= r) cp[(r * (r + 1) / 2 + cc) * SG] = v;
   }
-  // [D] for the tangent kernel: the lower triangle of history words 1-36
 #pragma unroll
-  for (int r = 0; r < 6; ++r)
+  for (int i = 0; i < 7; ++i)
+    if (sub + 4 * i < 27) hn1[(36 + sub + 4 * i) * SG] = 0.0;
 #pragma unroll
-    for (int cc = 0; cc <= r; ++cc)
-      cp[tri(r, cc) * SG] = tang_avg[r + 6 * cc];
+  for (int i = 0; i < 3; ++i) {
+    const int k = sub + 4 * i;
+    if (k < 9)
+      hn1[(63 + k) * SG] = rot ? rot[k * SG] : ((k % 4 == 0) ? 1.0 : 0.0);
+  }
+  if (sub < 3) {  // energy, plastic work and strain
+    const double v = qpick(sub, t_work, p_work, p_strain, 0.0);
+    sn1[(6 + sub) * SG] = sn9[(6 + sub) * SG] + v;
+    const double base = step == 1 ? 0.0 : hn[(72 + sub) * SG];
+    hn1[(72 + sub) * SG] = base + v;
+  }
+#pragma unroll
+  for (int i = 0; i < NSL; ++i) {
+    const int64_t w = (75 + NSL * sub + i) * SG;
+    double base = step == 1 ? 0.0 : hn[w];
+    hn1[w] = base + hn1[w] / rn;
+  }
 }
 
 // ---------------------------------------------------------------------
@@ -1441,22 +1536,26 @@ int launch_mm10_grads(const DevModel& M, const int32_t* d_blks, int nblks,
 }
 
 // Persistent over the work list: each workgroup (one wave) takes the next
-// item of 64 points from a device counter until the list is exhausted, so
-// points whose local solves sub-step or iterate longer do not hold back a
-// fixed share of the grid.  The counter starts at zero (launch_mm10 clears
-// it with a fill kernel first).
+// part of kPts points of a work item from a device counter until the list
+// is exhausted, so points whose local solves sub-step or iterate longer do
+// not hold back a fixed share of the grid.  The counter starts at zero
+// (launch_mm10 clears it with a fill kernel first).
+constexpr int kItemParts = 64 / kPts;  // parts of a 64-point item
+
 __global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(2)))
     k_mm10(DevModel M, const WorkItem* __restrict__ work, int nwork,
            int* __restrict__ counter, int step, int iter0_off) {
-  __shared__ double s_geo[kGeoWords * kLanes];
+  __shared__ double s_mem[kMemWords];
   __shared__ int s_item;
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(counter, 1);
     __syncthreads();
-    const int item = s_item;
+    const int unit = __builtin_amdgcn_readfirstlane(s_item);
     __syncthreads();
-    if (item >= nwork) break;  // uniform across the workgroup
-    mm10_item(M, work[item], step, iter0_off, s_geo);
+    if (unit >= kItemParts * nwork) break;  // uniform across the workgroup
+    mm10_item(M, work[unit / kItemParts], unit % kItemParts, step, iter0_off,
+              s_mem);
   }
 }
 
@@ -1464,16 +1563,18 @@ __global__ void __launch_bounds__(64)
 // global items [item0_s, item0_s + nwork_s); the workgroup finds its slot
 // by bisection over the slots' item0 (ascending).
 __global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(2)))
     k_mm10_batch(const Mm10Slot* __restrict__ slots, int nslot,
                  int nwork_total, int* __restrict__ counter) {
-  __shared__ double s_geo[kGeoWords * kLanes];
+  __shared__ double s_mem[kMemWords];
   __shared__ int s_item;
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(counter, 1);
     __syncthreads();
-    const int item = __builtin_amdgcn_readfirstlane(s_item);
+    const int unit = __builtin_amdgcn_readfirstlane(s_item);
     __syncthreads();
-    if (item >= nwork_total) break;  // uniform across the workgroup
+    if (unit >= kItemParts * nwork_total) break;  // uniform
+    const int item = unit / kItemParts;
     int lo = 0, hi = nslot - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
@@ -1483,7 +1584,8 @@ __global__ void __launch_bounds__(64)
         hi = mid - 1;
     }
     const Mm10Slot& sl = slots[lo];
-    mm10_item(sl.M, sl.work[item - sl.item0], sl.step, sl.iter0_off, s_geo);
+    mm10_item(sl.M, sl.work[item - sl.item0], unit % kItemParts, sl.step,
+              sl.iter0_off, s_mem);
   }
 }
 
@@ -1493,7 +1595,7 @@ int launch_mm10_batch(const Mm10Slot* d_slots, int nslot, int nwork_total,
   int rc = launch_fill_i32(d_counter, 1, 0, s);
   if (rc) return rc;
   hipLaunchKernelGGL(k_mm10_batch,
-                     dim3(grid < nwork_total ? grid : nwork_total), dim3(64),
+                     dim3(std::min(grid, kItemParts * nwork_total)), dim3(64),
                      0, s, d_slots, nslot, nwork_total, d_counter);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
@@ -1504,8 +1606,9 @@ int launch_mm10(const DevModel& M, const WorkItem* d_work, int nwork,
   if (nwork <= 0) return W3D_OK;
   int rc = launch_fill_i32(d_counter, 1, 0, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_mm10, dim3(grid < nwork ? grid : nwork), dim3(64), 0,
-                     s, M, d_work, nwork, d_counter, step, iter0_off);
+  hipLaunchKernelGGL(k_mm10, dim3(std::min(grid, kItemParts * nwork)),
+                     dim3(64), 0, s, M, d_work, nwork, d_counter, step,
+                     iter0_off);
   return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
 }
 

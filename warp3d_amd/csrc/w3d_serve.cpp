@@ -389,7 +389,7 @@ int w3d_batch_create(int32_t device, w3d_batch** out) {
     return fail(W3D_ERR_DEVICE, "w3d_batch_create: device set-up");
   }
   b->n_cu = prop.multiProcessorCount;
-  b->mm10_grid = 4 * std::max(b->n_cu, 1);
+  b->mm10_grid = 8 * std::max(b->n_cu, 1);
   for (int ph = 0; ph < w3d_batch::kPhases; ++ph)
     for (int k = 0; k < 2; ++k)
       if (hipEventCreate(&b->ev[ph][k]) != hipSuccess) b->ev[ph][k] = nullptr;
