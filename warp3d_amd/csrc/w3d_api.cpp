@@ -913,39 +913,32 @@ int recover_impl(w3d_ctx* c, int step, int iter, int extrapolated,
 }
 
 // Jacobi-PCG on an assembled matrix (diag, coef device arrays); b and x
-// device arrays of neqns (x: initial guess in, solution out).  work: 5
-// neqns doubles of vectors, then kPcgTail words.
+// device arrays of neqns (x: initial guess in, solution out).  work: kPcgVectors
+// neqns doubles of vectors, tail: kPcgTail.
 int pcg_impl(w3d_ctx* c, const double* d_diag, const double* d_coef,
              const double* d_b, double* d_x, double rtol, int maxit,
              int32_t* iters, double* relres, double* work, double* tail) {
   const int n = c->neqns;
   hipStream_t s = c->stream;
   PcgSys S{};
-  S.rp = c->d_csr_rp;
-  S.col = c->d_csr_col;
-  S.grp = c->d_csr_grp;
+  S.A = c->groups();
   S.val = c->d_csr_val;
   S.diag = d_diag;
   S.b = d_b;
   S.x = d_x;
-  S.zp = reinterpret_cast<double2*>(work);
-  S.r = work + 2 * (int64_t)n;
-  S.p = S.r + n;
-  S.q = S.p + n;
   S.part = tail + 8;
   S.rtol = rtol;
   S.maxit = maxit;
   S.n = n;
-  S.ngrp = c->csr_ngrp;
-  S.nmul = pcg_mul_wgs(S.ngrp);
-  S.nvec = pcg_vec_wgs(n);
+  S.set_work(work);
+  S.nwg = pcg_mul_wgs(S.A.ngrp);
   S.single = 1;
   double* sc = tail;
   int32_t* state = reinterpret_cast<int32_t*>(tail + 2);
   int rc = solver_csr_values(d_diag, d_coef, n, c->d_csr_vidx, c->csr_nnz,
                              c->d_csr_val, s);
-  // r = A x, then b - A x by the initialisation
-  if (!rc) rc = solver_spmv(c->groups(), c->d_csr_val, d_x, S.r, s);
+  // A x, then r = b - A x by the initialisation
+  if (!rc) rc = solver_spmv(c->groups(), c->d_csr_val, d_x, S.p, s);
   if (!rc) rc = launch_pcg_init(S, s, state, sc);
   const int32_t* st = nullptr;
   if (!rc)
@@ -1631,15 +1624,19 @@ static int finish_pattern(w3d_ctx* c, int32_t* neqns_out,
                 rp[r + 1] - rp[r] == rp[r] - rp[r - 1] &&
                 std::equal(col.begin() + rp[r], col.begin() + rp[r + 1],
                            col.begin() + rp[r - 1]);
-    std::vector<int32_t> grp{0};
-    for (int r = 1; r < neq; ++r)
-      if (!same[r] || r - grp.back() >= 3) grp.push_back(r);
-    c->csr_ngrp = neq > 0 ? (int)grp.size() : 0;
-    grp.push_back(neq);
+    std::vector<RowGroup> grp;
+    for (int r = 0; r < neq; ++r) {
+      if (r > 0 && same[r] && grp.back().rows() < 3)
+        grp.back().nl += 1;
+      else
+        grp.push_back({rp[r], r, (int32_t)(rp[r + 1] - rp[r]) << 2 | 1});
+    }
+    c->csr_ngrp = (int)grp.size();
     dfree(c->d_csr_grp);
     if ((rc = upload(&c->d_csr_grp, grp))) return rc;
-    // the solver's work array (5 neq and its tail), b and x
-    if ((rc = dalloc(&c->d_pcg, 7 * (int64_t)neq + kPcgTail))) return rc;
+    // the solver's work array and its tail, b and x
+    if ((rc = dalloc(&c->d_pcg, (kPcgVectors + 2) * (int64_t)neq + kPcgTail)))
+      return rc;
     c->csr_nnz = nnz;
     c->csr_serial = -1;
     c->assembled = 0;
@@ -2071,7 +2068,8 @@ int w3d_solve_pcg_dev(w3d_ctx* c, const double* d_k_diag,
     return fail(W3D_ERR_ARG, "w3d_solve_pcg: rtol > 0 and maxit >= 1");
   HIPCHK(hipSetDevice(c->device));
   return pcg_impl(c, d_k_diag, d_k_coeffs, d_rhs, d_x, rtol, maxit, iters,
-                  relres, c->d_pcg, c->d_pcg + 5 * (int64_t)c->neqns);
+                  relres, c->d_pcg,
+                  c->d_pcg + kPcgVectors * (int64_t)c->neqns);
 }
 
 int w3d_solve_pcg_static(w3d_ctx* c, const double* d_k_diag,
@@ -2094,7 +2092,8 @@ int w3d_solve_pcg_static(w3d_ctx* c, const double* d_k_diag,
   int rc = w3d::solver_static_scratch(c->device, &work);
   if (rc) return fail(rc, "w3d_solve_pcg_static: static work memory");
   return pcg_impl(c, d_k_diag, d_k_coeffs, d_rhs, d_x, rtol, maxit, iters,
-                  relres, work, work + 5 * (int64_t)w3d::kStaticMaxEq);
+                  relres, work,
+                  work + kPcgVectors * (int64_t)w3d::kStaticMaxEq);
 }
 
 int w3d_solve_pcg(w3d_ctx* c, const double* rhs, double* x, double rtol,
@@ -2108,14 +2107,14 @@ int w3d_solve_pcg(w3d_ctx* c, const double* rhs, double* x, double rtol,
     return fail(W3D_ERR_ARG, "w3d_solve_pcg: rtol > 0 and maxit >= 1");
   HIPCHK(hipSetDevice(c->device));
   const int n = c->neqns;
-  double* b = c->d_pcg + 5 * (int64_t)n + kPcgTail;
+  double* b = c->d_pcg + kPcgVectors * (int64_t)n + kPcgTail;
   double* xd = b + n;
   HIPCHK(hipMemcpyAsync(b, rhs, n * sizeof(double), hipMemcpyHostToDevice,
                         c->stream));
   HIPCHK(hipMemcpyAsync(xd, x, n * sizeof(double), hipMemcpyHostToDevice,
                         c->stream));
   int rc = pcg_impl(c, c->d_kout, c->d_kout + n, b, xd, rtol, maxit, iters,
-                    relres, c->d_pcg, c->d_pcg + 5 * (int64_t)n);
+                    relres, c->d_pcg, c->d_pcg + kPcgVectors * (int64_t)n);
   if (rc < 0 && rc != W3D_ERR_NUMERIC) return rc;
   HIPCHK(hipMemcpyAsync(x, xd, n * sizeof(double), hipMemcpyDeviceToHost,
                         c->stream));

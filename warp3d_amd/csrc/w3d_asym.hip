@@ -50,9 +50,10 @@ __global__ void __launch_bounds__(64 * kAsmWaves)
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int g = blockIdx.x * (blockDim.x >> 6) + wv;
   if (g >= A.ngrp) return;  // uniform across the wave
-  const int r0 = A.grp[g], nr = A.grp[g + 1] - r0;
-  const int64_t v0 = A.rp[r0];
-  const int len = (int)(A.rp[r0 + 1] - v0);  // <= maxrow
+  const RowGroup gd = A.grp[g];
+  const int r0 = gd.row0, nr = gd.rows();
+  const int64_t v0 = gd.k0;
+  const int len = gd.len();  // <= maxrow
   double* row = s_rows + (size_t)wv * 3 * maxrow;
   for (int k = lane; k < nr * len; k += 64) row[k] = 0.0;
   wave_fence();

@@ -198,10 +198,10 @@ struct w3d_ctx {
   int32_t* d_csr_col = nullptr;
   uint32_t* d_csr_vidx = nullptr;
   double* d_csr_val = nullptr;
-  int32_t* d_csr_grp = nullptr;  // row groups (RowGroups)
+  w3d::RowGroup* d_csr_grp = nullptr;
   int csr_ngrp = 0;
   w3d::RowGroups groups() const {
-    return {d_csr_rp, d_csr_col, d_csr_grp, csr_ngrp};
+    return {d_csr_col, d_csr_grp, csr_ngrp};
   }
   double* d_pcg = nullptr;   // solver work vectors and scalars
   // solve_poll's pinned state images (2 words each) and events, and the

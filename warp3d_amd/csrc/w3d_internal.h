@@ -219,12 +219,19 @@ int launch_assemble(const double* ek64, const float* ek32, int fp32,
                     const int64_t* wbase, int64_t nseg, int64_t neq,
                     double* diag, double* coef, hipStream_t s);
 // Full CSR rows in groups of consecutive rows that share their columns:
-// the free equations of one structure node (at most 3 rows; group g is
-// rows grp[g] .. grp[g + 1] - 1, their lengths equal).
+// the free equations of one structure node (at most 3 rows of one length).
+// One 16-byte word a group: its first entry, first row, and rows and
+// entries per row packed, so that a lane needs one load to start on it.
+struct alignas(16) RowGroup {
+  int64_t k0;
+  int32_t row0;
+  int32_t nl;
+  __host__ __device__ int rows() const { return nl & 3; }
+  __host__ __device__ int len() const { return nl >> 2; }
+};
 struct RowGroups {
-  const int64_t* rp;
   const int32_t* col;
-  const int32_t* grp;
+  const RowGroup* grp;
   int32_t ngrp;
 };
 
@@ -285,45 +292,56 @@ int solver_spmv(const RowGroups& A, const double* val, const double* x,
                 double* y, hipStream_t s);
 
 // One system of a Jacobi-PCG: the full CSR rows of its assembled matrix,
-// its diagonal, right-hand side and vectors, the workgroups of its matrix
-// and vector launches (from its size alone) and their partial sums.
-// single: x holds the initial guess and r A x on entry, the convergence
+// its diagonal, right-hand side and vectors, the workgroups of its launches
+// (from its size alone) and their partial sums.
+// single: x holds the initial guess and p A x on entry, the convergence
 // test runs before the first iteration too and a residual that is no
 // number ends the solve; a system of a batch starts from x = 0.
-constexpr int kPcgMaxMul = 2048, kPcgMaxVec = 1024;
+constexpr int kPcgMaxMul = 1024, kPcgMaxVec = 1024;
 constexpr int32_t kPcgZeroRhs = 4;  // a single solve's state on |b| = 0
+// PcgRow: residual, w = A D^-1 r, s and 1 / diagonal of one equation.
+struct alignas(32) PcgRow {
+  double r, w, s, rd;
+};
 struct PcgSys {
-  const int64_t* rp;
-  const int32_t* col;
-  const int32_t* grp;
+  RowGroups A;
   const double* val;
   const double* diag;
   const double* b;
   double* x;
-  double* r;
   double* p;
-  double* q;
-  double2* zp;            // (z, p) of every equation
-  double* part;           // pcg_part_words of partial sums
+  PcgRow* row[2];         // by the parity of the launch that reads it
+  double* part;           // pcg_part_words of partial sums and scalars
   double rtol;            // |r| <= rtol |b| ends the solve
   int32_t maxit;          // or this many iterations
-  int32_t n, ngrp;
-  int32_t mul0, nmul;     // workgroups of the matrix launch
-  int32_t vec0, nvec;     // and of the vector launch
+  int32_t n;
+  int32_t wg0, nwg;       // its workgroups
   int32_t single;
-  __host__ __device__ int off_pq() const { return 0; }
-  __host__ __device__ int off_bb() const { return nmul; }
-  __host__ __device__ int off_rr() const { return nmul + nvec; }
-  __host__ __device__ int off_rz(int k) const { return nmul + (2 + k) * nvec; }
+  // the vectors in an array of kPcgVectors n doubles
+  void set_work(double* w) {
+    row[0] = reinterpret_cast<PcgRow*>(w);
+    row[1] = row[0] + n;
+    p = w + 8 * (int64_t)n;
+  }
+  // per workgroup b.b, then the three sums of each parity, then (r.u,
+  // alpha) of each parity
+  __host__ __device__ int off_bb() const { return 0; }
+  __host__ __device__ int off_sums(int par) const {
+    return (1 + 3 * par) * nwg;
+  }
+  __host__ __device__ int off_scalars(int par) const {
+    return 7 * nwg + 2 * par;
+  }
 };
 int pcg_mul_wgs(int ngrp);
 int pcg_vec_wgs(int n);
-inline int pcg_part_words(int nmul, int nvec) { return nmul + 4 * nvec; }
-// A single solve's work array: 5 n doubles of vectors ((z, p) pairs, r, p,
-// q), then 2 scalars (|b|, r.r), the state (done: 0 running, 1 converged,
+constexpr int pcg_part_words(int nwg) { return 7 * nwg + 4; }
+// A single solve's work array: kPcgVectors n doubles (the rows twice, p),
+// then 2 scalars (|b|, r.r), the state (done: 0 running, 1 converged,
 // 2 iteration limit, kPcgZeroRhs; iterations; two gates) and the partial
 // sums.
-constexpr int kPcgTail = 8 + kPcgMaxMul + 4 * kPcgMaxVec;
+constexpr int kPcgVectors = 9;
+constexpr int kPcgTail = 8 + pcg_part_words(kPcgMaxMul);
 int launch_pcg_init(const PcgSys& one, hipStream_t s, int32_t* state,
                     double* sc);
 int launch_pcg_iter(const PcgSys& one, int it, int32_t* state, double* sc,
@@ -394,19 +412,18 @@ int launch_mm10_batch(const Mm10Slot* d_slots, int nslot, int nwork_total,
 // Rows of one tile of a batched vector kernel (one workgroup each).
 constexpr int kTileRows = 128;
 
-// A batch of Jacobi-PCG systems: owner tables give each workgroup of the
-// two launches its system.
+// A batch of Jacobi-PCG systems: the owner table gives each workgroup of a
+// launch its system.
 struct PcgBatch {
   const PcgSys* sys;
-  const int32_t* mul_owner;
-  const int32_t* vec_owner;
-  int nsys, nmul, nvec;
+  const int32_t* owner;
+  int nsys, nwg;
 };
-// x = 0, r = b, z = D^-1 b and the partial sums; then |b| per system
+// x = 0, r = b and |b| per system, then w = A D^-1 r
 int launch_pcg_batch_init(const PcgBatch& b, int32_t* state, double* sc,
                           hipStream_t s);
-// iteration it (0-based) of every running system (last: the test alone)
-int launch_pcg_batch_iter(const PcgBatch& b, int it, int last, int32_t* state,
+// iteration it (0-based) of every running system
+int launch_pcg_batch_iter(const PcgBatch& b, int it, int32_t* state,
                           double* sc, hipStream_t s);
 
 // One problem's Newton bookkeeping for the batched residual and update:

@@ -96,7 +96,7 @@ struct w3d_problem {
   int64_t nd = 0;
   double *d_u = nullptr, *d_du = nullptr, *d_ifv = nullptr;
   double* d_k = nullptr;  // assembled diagonal, then coefficients
-  // the solver's vectors: rhs, x, then (z, p) pairs, r, p, q in d_work
+  // the solver's vectors: rhs, x, then kPcgVectors in d_work
   double *d_rhs = nullptr, *d_x = nullptr, *d_work = nullptr;
   double* d_cimp = nullptr;  // a full step's imposed increments (cdof order)
   int32_t *d_eqdof = nullptr, *d_cdof = nullptr, *d_ldof = nullptr;
@@ -300,7 +300,7 @@ int w3d_problem_create(w3d_ctx* c, const int32_t* cstmap, const double* du0,
       (rc = dalloc(&p->d_ifv, p->nd)) ||
       (rc = dalloc(&p->d_k, neq + (size_t)nco)) ||
       (rc = dalloc(&p->d_rhs, neq)) || (rc = dalloc(&p->d_x, neq)) ||
-      (rc = dalloc(&p->d_work, 5 * (int64_t)neq)) ||
+      (rc = dalloc(&p->d_work, kPcgVectors * (int64_t)neq)) ||
       (rc = upload(&p->d_cimp, cimp)) ||
       (rc = upload(&p->d_eqdof, eqdof)) ||
       (rc = upload(&p->d_cdof, cdof)) || (rc = upload(&p->d_ldof, ldof))) {
@@ -622,7 +622,7 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
   // 4. tangents, assemblies and the batched solve
   const int ns = (int)solve.size();
   if (ns > 0) {
-    int nmul = 0, nvec = 0, maxit = 0;
+    int nwg = 0, maxit = 0;
     int64_t npart = 0;
     b->mark(3, 0);
     for (int i = 0; i < ns; ++i) {
@@ -637,49 +637,38 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
       if (rc) return fail(rc, "w3d_batch_advance: tangent/assembly launch");
       c->tangent_precision = p->o.precision;
       PcgSys& S = b->h_pcg[i];
-      S.rp = c->d_csr_rp;
-      S.col = c->d_csr_col;
-      S.grp = c->d_csr_grp;
+      S.A = c->groups();
       S.val = c->d_csr_val;
       S.diag = p->d_k;
       S.b = p->d_rhs;
       S.x = p->d_x;
-      S.zp = reinterpret_cast<double2*>(p->d_work);
-      S.r = p->d_work + 2 * (int64_t)p->neq;
-      S.p = S.r + p->neq;
-      S.q = S.p + p->neq;
       S.rtol = p->o.pcg_rtol;
       S.maxit = p->o.pcg_maxit;
       S.n = p->neq;
-      S.ngrp = c->csr_ngrp;
-      S.mul0 = nmul;
-      S.nmul = pcg_mul_wgs(S.ngrp);
-      S.vec0 = nvec;
-      S.nvec = pcg_vec_wgs(S.n);
+      S.set_work(p->d_work);
+      S.wg0 = nwg;
+      S.nwg = pcg_mul_wgs(S.A.ngrp);
       S.single = 0;
-      nmul += S.nmul;
-      nvec += S.nvec;
-      npart += pcg_part_words(S.nmul, S.nvec);
+      nwg += S.nwg;
+      npart += pcg_part_words(S.nwg);
       maxit = std::max(maxit, S.maxit);
     }
     b->mark(3, 1);
     // the solve's partial sums follow the residual's in d_part
-    if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res + npart, nmul + nvec)))
+    if ((rc = reserve(b, nr, 3 * (int64_t)ntile_res + npart, nwg)))
       return rc;
     double* part = b->d_part + 3 * (int64_t)ntile_res;
     for (int i = 0; i < ns; ++i) {
       PcgSys& S = b->h_pcg[i];
       S.part = part;
-      part += pcg_part_words(S.nmul, S.nvec);
-      for (int k = 0; k < S.nmul; ++k) b->h_owner[S.mul0 + k] = i;
-      for (int k = 0; k < S.nvec; ++k) b->h_owner[nmul + S.vec0 + k] = i;
+      part += pcg_part_words(S.nwg);
+      for (int k = 0; k < S.nwg; ++k) b->h_owner[S.wg0 + k] = i;
     }
     HIPCHK(hipMemcpyAsync(b->d_pcg, b->h_pcg, ns * sizeof(PcgSys),
                           hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(b->d_owner, b->h_owner,
-                          (nmul + nvec) * sizeof(int32_t),
+    HIPCHK(hipMemcpyAsync(b->d_owner, b->h_owner, nwg * sizeof(int32_t),
                           hipMemcpyHostToDevice, s));
-    const PcgBatch B{b->d_pcg, b->d_owner, b->d_owner + nmul, ns, nmul, nvec};
+    const PcgBatch B{b->d_pcg, b->d_owner, ns, nwg};
     b->mark(4, 0);
     if ((rc = launch_pcg_batch_init(B, b->d_state, b->d_sc, s)))
       return fail(rc, "w3d_batch_advance: solver launch");
@@ -687,8 +676,7 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
     const int32_t* st = nullptr;
     rc = solve_poll(
         [&](int it) {
-          return launch_pcg_batch_iter(B, it, it >= maxit, b->d_state,
-                                       b->d_sc, s);
+          return launch_pcg_batch_iter(B, it, b->d_state, b->d_sc, s);
         },
         ns, maxit, kPollChunk, b->d_state, b->h_state, b->poll_ev, s, &st);
     if (rc) return fail(rc, "w3d_batch_advance: solver launch");
