@@ -391,13 +391,14 @@ __device__ inline void slip_geometry(const Props& p, const double* Rpn,
   } else {
     rt2rvw(tn, rw);
   }
+#pragma unroll
+  for (int i = 0; i < NSL; ++i) mv3(s.q[i], rw, p.cr->qs[NSL * s.sub + i]);
   {
     double RE[36];
     rt2rve(tn, RE);
 #pragma unroll
     for (int i = 0; i < NSL; ++i) {
       const double* m0 = p.cr->ms[NSL * s.sub + i];
-      mv3(s.q[i], rw, p.cr->qs[NSL * s.sub + i]);
 #pragma unroll
       for (int r = 0; r < 6; ++r) s.ms[i][r] = RE[r] * m0[0];
 #pragma unroll
@@ -903,13 +904,18 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
   const int64_t q = wi.first + kPts * part + pt;  // point inside the block
   const int elem = (int)(q / G);
   const int ncry = uniform(bp->ncry);
-  const double* hn = M.hist_n + bd.hist_off + q;
-  const double* sn9 = M.stress_n + 9 * bd.q_off + q;
-  const double* ud = M.uddt + 6 * bd.q_off + q;
-  // the point's place in the output arrays
+  // the point's place in its block's arrays
   int qo = (int)q;
+  auto fresh = [&](const double* base) {
+    int k = qo;
+    asm volatile("" : "+v"(k));
+    return base + k;
+  };
+  const double* hist_n = M.hist_n + bd.hist_off;
+  const double* uddt = M.uddt + 6 * bd.q_off;
+  const double* stress_n = M.stress_n + 9 * bd.q_off;
   // finite strains: [R n+1] of the point (the recovery's), else R = I
-  const double* rot = bd.geonl ? M.rot_tmp + 9 * bd.q_off + q : nullptr;
+  const double* rot_b = bd.geonl ? M.rot_tmp + 9 * bd.q_off : nullptr;
   const double dt = M.dt;
   double* Jl = s_mem + kCmsWords + pt;
 
@@ -946,15 +952,14 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
     const int64_t cb = (int64_t)(87 + 71 * c) * SG;
     // n-state of the crystal (mm10_copy_cc_hist; at step 1 the
     // mm10_init_cc_hist0 values)
-    // (Dn, the n strain increment, is read where the predictor uses it)
     double tau_n, tt_rate_n;
-    const double* Dn = step == 1 ? nullptr : hn + cb + 18 * SG;
-    const double* sn = step == 1 ? sn9 : hn + cb;
+    const double* stress_c = step == 1 ? stress_n : hist_n + cb;
     CState np1;
     np1.sub = sub;
     np1.trial = s_mem + kCmsWords + kJacWords + pt;
     double* ostress = np1.trial + kTriWords;
     {
+      const double* hn = fresh(hist_n);
       double Rpn[9];
       if (step == 1) {
 #pragma unroll
@@ -966,17 +971,24 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
         tau_n = hn[cb + 42 * SG];
       }
       // np1 (mm10_setup_np1 + mm10_setup)
-      slip_geometry(p, Rpn, s_mem + lane, np1, rot, SG);
+      slip_geometry(p, Rpn, s_mem + lane, np1,
+                    rot_b ? fresh(rot_b) : nullptr, SG);
+      tt_rate_n = hn[cb + 58 * SG];
     }
-    tt_rate_n = hn[cb + 58 * SG];
+    // (C is read again where it is used, not held from here on)
+    asm volatile("" : "+v"(p.cr));
     // mm10_solve_strup
     double D[6], stress[6], tt = tau_n, ott = tau_n;
+    {
+      const double* ud = fresh(uddt);
+      const double* sn = fresh(stress_c);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) D[k] = ud[k * SG];
+      for (int k = 0; k < 6; ++k) D[k] = ud[k * SG];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) stress[k] = sn[k * SG];
+    }
     np1.tt_rate = 0.0;
     setup(p, np1, D, dt);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) stress[k] = sn[k * SG];
     double temp1 = dot6(D, D);
     double temp2 = dot6(stress, stress);
     const bool no_load = temp2 == 0.0 && temp1 == 0.0;
@@ -994,7 +1006,7 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
       for (int i = 0; i < 9; ++i) store_tangent(sub + 4 * i, C[sub + 4 * i]);
       if (!no_load) {
         double R1[6];
-        set_trial(p, np1, D, sn, SG);
+        set_trial(p, np1, D, fresh(stress_c), SG);
         formR1(p, np1, stress, tt, R1);
 #pragma unroll
         for (int k = 0; k < 6; ++k) stress[k] = stress[k] - R1[k];
@@ -1009,14 +1021,18 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
 #pragma unroll
       for (int k = 0; k < 6; ++k) ostress[k * kPts] = stress[k];
       while (frac < 1.0) {
+        const double* ud = fresh(uddt);
 #pragma unroll
         for (int k = 0; k < 6; ++k) D[k] = ud[k * SG] * (sstep + frac);
         np1.tt_rate = 0.0;
         setup(p, np1, D, dt * (sstep + frac));
-        set_trial(p, np1, D, sn, SG);
+        set_trial(p, np1, D, fresh(stress_c), SG);
+        asm volatile("" : "+v"(p.cr));
         tt = tau_n;
-        solve(p, np1, D, tau_n, tt_rate_n, Dn, SG, stress, &tt, fail,
-              dt * sstep, Jl);
+        // (Dn, the n strain increment)
+        solve(p, np1, D, tau_n, tt_rate_n,
+              step == 1 ? nullptr : fresh(hist_n) + cb + 18 * SG, SG, stress,
+              &tt, fail, dt * sstep, Jl);
         if (fail) {
 #pragma unroll
           for (int k = 0; k < 6; ++k) stress[k] = ostress[k * kPts];
@@ -1037,12 +1053,13 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
         break;
       }
       curr_tt_rate = np1.tt_rate;
+      const double* ud = fresh(uddt);
 #pragma unroll
       for (int k = 0; k < 6; ++k) D[k] = ud[k * SG];
       setup(p, np1, D, dt);
     }
     np1.tt_rate = curr_tt_rate;
-    asm volatile("" : "+v"(sub), "+v"(qo));
+    asm volatile("" : "+v"(sub), "+v"(qo), "+v"(p.cr));
     // mm10_store_cryhist: each word is stored as soon as it is formed
     double* h1 = M.hist_n1 + bd.hist_off + cb + qo;
     double slip[NSL];
@@ -1122,6 +1139,8 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
       // again here)
       {
         double Rpe[9], Rp1[9], eul[3];
+        const double* hn = fresh(hist_n);
+        const double* rot = rot_b ? fresh(rot_b) : nullptr;
 #pragma unroll
         for (int k = 0; k < 9; ++k)
           Rpe[k] = step == 1 ? ((k % 4 == 0) ? 1.0 : 0.0)
@@ -1214,7 +1233,8 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
 #pragma unroll
       for (int k = 0; k < 6; ++k) ee[k] = stress[k];
       chol_solve6(p.cr->C, ee);
-      if (rot) {  // ee = RT2RVE(R) C^-1 sigma (exact for R = I)
+      if (rot_b) {  // ee = RT2RVE(R) C^-1 sigma (exact for R = I)
+        const double* rot = fresh(rot_b);
         double R[9], er[36], t[6];
 #pragma unroll
         for (int k = 0; k < 9; ++k) R[k] = rot[k * SG];
@@ -1337,6 +1357,9 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
     return;
   }
   const double rn = (double)ncry;
+  const double* hn = fresh(hist_n);
+  const double* sn9 = fresh(stress_n);
+  const double* rot = rot_b ? fresh(rot_b) : nullptr;
   double* sn1 = M.stress_n1 + 9 * bd.q_off + qo;
   double* hn1 = M.hist_n1 + bd.hist_off + qo;
   double* cp = M.cep + 21 * bd.q_off + qo;
