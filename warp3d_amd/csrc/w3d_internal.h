@@ -297,7 +297,7 @@ int solver_spmv(const RowGroups& A, const double* val, const double* x,
 // single: x holds the initial guess and p A x on entry, the convergence
 // test runs before the first iteration too and a residual that is no
 // number ends the solve; a system of a batch starts from x = 0.
-constexpr int kPcgMaxMul = 1024, kPcgMaxVec = 1024;
+constexpr int kPcgMaxMul = 768, kPcgMaxVec = 1024;
 constexpr int32_t kPcgZeroRhs = 4;  // a single solve's state on |b| = 0
 // PcgRow: residual, w = A D^-1 r, s and 1 / diagonal of one equation.
 struct alignas(32) PcgRow {

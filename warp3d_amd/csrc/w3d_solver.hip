@@ -68,10 +68,10 @@ __global__ void k_csr_values(const double* __restrict__ diag,
 // lanes: the 81 columns of a structured brick's node are three entries a
 // lane, loaded together, and a 1,000-node system still spreads over 32,000
 // lanes.  Bound by memory on large systems (124,740 equations, 9.5 M
-// entries: 30 us, 3 TB/s).  Each row sums its lanes' strided shares in a
+// entries: 27 us, 3.3 TB/s).  Each row sums its lanes' strided shares in a
 // fixed butterfly, so products are bitwise repeatable.  Workgroups of 256:
 // of 512, an iteration on one to three systems of 2,000 to 3,600 equations
-// took 7.3 to 7.8 us for 6.0 to 7.4, one on 124,740 29.8 for 30.4.
+// took 7.3 to 7.8 us for 6.0 to 7.4.
 // ---------------------------------------------------------------------
 constexpr int kGrpLanes = 32;
 constexpr int kMulBlock = 256;
@@ -83,31 +83,39 @@ constexpr int kGrpAhead = 3;
 template <typename W>
 struct GrpTile {
   RowGroup d;
+  int c[kGrpAhead];
   double a[3][kGrpAhead];
   W x[kGrpAhead];
 };
 template <typename W>
-__device__ __forceinline__ void tile_entries(const RowGroups& A,
-                                             const double* __restrict__ val,
+__device__ __forceinline__ void tile_columns(const RowGroups& A, int lane,
+                                             int from, GrpTile<W>& t) {
+  const int len = t.d.len();
+  const int32_t* cp = A.col + t.d.k0;
+#pragma unroll
+  for (int u = 0; u < kGrpAhead; ++u) {
+    const int k = from + lane + u * kGrpLanes;
+    t.c[u] = cp[k < len ? k : len - 1];
+  }
+}
+template <typename W>
+__device__ __forceinline__ void tile_entries(const double* __restrict__ val,
                                              const W* __restrict__ x,
                                              int lane, int from,
                                              GrpTile<W>& t) {
   const int len = t.d.len(), nr = t.d.rows();
-  const int32_t* cp = A.col + t.d.k0;
   const double* v = val + t.d.k0;
   const int o1 = nr > 1 ? len : 0, o2 = nr > 2 ? 2 * len : 0;
-  int c[kGrpAhead];
 #pragma unroll
   for (int u = 0; u < kGrpAhead; ++u) {
     const int k = from + lane + u * kGrpLanes;
     const int kk = k < len ? k : len - 1;
-    c[u] = cp[kk];
     t.a[0][u] = v[kk];
     t.a[1][u] = v[o1 + kk];
     t.a[2][u] = v[o2 + kk];
   }
 #pragma unroll
-  for (int u = 0; u < kGrpAhead; ++u) t.x[u] = x[c[u]];
+  for (int u = 0; u < kGrpAhead; ++u) t.x[u] = x[t.c[u]];
 }
 // the first entries of group g, loaded ahead of the scalars a product needs
 template <typename W>
@@ -116,7 +124,8 @@ __device__ __forceinline__ void tile_load(const RowGroups& A,
                                           const W* __restrict__ x, int g,
                                           int lane, GrpTile<W>& t) {
   t.d = A.grp[g];
-  tile_entries(A, val, x, lane, 0, t);
+  tile_columns(A, lane, 0, t);
+  tile_entries(val, x, lane, 0, t);
 }
 
 // s[k] = row (row0 + k) . f(x) over the rows of the loaded group, every lane
@@ -138,7 +147,8 @@ __device__ __forceinline__ void tile_product(const RowGroups& A,
     }
     from += kGrpAhead * kGrpLanes;
     if (from >= t.d.len()) break;
-    tile_entries(A, val, x, lane, from, t);
+    tile_columns(A, lane, from, t);
+    tile_entries(val, x, lane, from, t);
   }
 #pragma unroll
   for (int off = kGrpLanes / 2; off >= 1; off >>= 1)
@@ -199,9 +209,10 @@ __global__ void __launch_bounds__(kMulBlock)
 // A launch is a chain of dependent loads and two workgroup sums on small
 // systems, and the host reads the states behind the device, so an iteration
 // costs no synchronisation.  Measured an iteration, against two launches
-// (product, vector update) of the usual recurrences: 10.4 -> 7.4 us on three
-// systems of 2,000 to 3,600 equations, 32.4 -> 30.4 us on 124,740, and a
-// launch gap less.
+// (product, vector update) of the usual recurrences: 10.4 -> 7.5 us on three
+// systems of 2,000 to 3,600 equations, 32.4 -> 27.4 us on 124,740, and a
+// launch gap less.  Three waves a SIMD: at four, the next group's words
+// (below) spilled, and a solve of 124,740 equations took 41 us an iteration.
 // Each system's reductions run over its own workgroups in a
 // fixed order, whose number depends on the system's size alone, so a
 // system's iterates do not depend on the batch.  Every workgroup of a system
@@ -265,7 +276,7 @@ __global__ void __launch_bounds__(kRedBlock)
 
 template <bool BATCH>
 __global__ void __launch_bounds__(kMulBlock)
-    __attribute__((amdgpu_waves_per_eu(4)))
+    __attribute__((amdgpu_waves_per_eu(3)))
     k_pcg_iter(const PcgSys one, const PcgSys* __restrict__ sys,
                const int32_t* __restrict__ owner, int it,
                int32_t* __restrict__ state, int32_t* __restrict__ gate,
@@ -285,14 +296,18 @@ __global__ void __launch_bounds__(kMulBlock)
   GrpTile<PcgRow> t;
   PcgRow o;          // lane k < rows: row k's own vectors
   double po, xo;
-  auto load = [&]() {
-    tile_load(S.A, S.val, row, g, lane, t);
+  auto load = [&]() {  // of the group whose word and columns t has
+    tile_entries(S.val, row, lane, 0, t);
     const int i = t.d.row0 + (lane < t.d.rows() ? lane : 0);
     o = row[i];
     po = S.p[i];
     xo = S.x[i];
   };
-  if (g < S.A.ngrp) load();
+  if (g < S.A.ngrp) {
+    t.d = S.A.grp[g];
+    tile_columns(S.A, lane, 0, t);
+    load();
+  }
   double alpha = 0.0, beta = 0.0;
   if (it >= 0) {
     const double* pt = S.part + S.off_sums(par);
@@ -336,6 +351,11 @@ __global__ void __launch_bounds__(kMulBlock)
   };
   double v[3] = {0.0, 0.0, 0.0};
   while (g < S.A.ngrp) {
+    // the next group's word and columns come in behind this one's products
+    const int gn = g + S.nwg * kGrpPerWg;
+    GrpTile<PcgRow> nx;
+    nx.d = S.A.grp[gn < S.A.ngrp ? gn : g];
+    tile_columns(S.A, lane, 0, nx);
     const int i = t.d.row0 + lane;
     const bool own = lane < t.d.rows();
     PcgRow n;
@@ -363,8 +383,13 @@ __global__ void __launch_bounds__(kMulBlock)
       v[1] = v[1] + n.r * u;
       v[2] = v[2] + n.w * u;
     }
-    g += S.nwg * kGrpPerWg;
-    if (g < S.A.ngrp) load();
+    g = gn;
+    if (g < S.A.ngrp) {
+      t.d = nx.d;
+#pragma unroll
+      for (int u = 0; u < kGrpAhead; ++u) t.c[u] = nx.c[u];
+      load();
+    }
   }
   block_sums<3, kMulBlock>(v, s_red);
   if (tid == 0)
@@ -376,7 +401,8 @@ __global__ void __launch_bounds__(kMulBlock)
 // Workgroups of one system's launches: a tile of groups (rows) each up to
 // the cap, then equal shares.  The caps bound the partial sums that every
 // workgroup of the next launch reads again, and keep a launch's workgroups
-// resident together (124,740 equations: 30.8 us on 867, 35.4 on 1,300).
+// resident together at three waves a SIMD (124,740 equations: 27.4 us an
+// iteration on 743, 34.1 on 867).
 int pcg_mul_wgs(int ngrp) {
   const int t = (ngrp + kGrpPerWg - 1) / kGrpPerWg;
   if (t < 1) return 1;
