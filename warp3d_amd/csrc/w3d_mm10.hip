@@ -434,6 +434,21 @@ __device__ inline void symsw(const double* s, const double* w, double* sw) {
   sw[5] = 0.5 * (w[1] * (s[0] - s[2]) + w[0] * s[3] - w[2] * s[4]);
 }
 
+// dg n |tau|^(n-1) / tau^n: times (|rs| / tau)^(n-1) the slip's derivative
+// dg n |rs|^(n-1) / tau^n.  Its sign on the negative tau of a stray iterate
+// is that of tau^n, and the power of a broken exponent has none.
+__device__ inline double flow_scale(const Props& p, double dg, double itt) {
+  double v = dg * p.rate_n * itt;
+  if (itt < 0.0) {
+    const int k = (int)p.rate_n;
+    if ((double)k != p.rate_n)
+      v = __builtin_nan("");
+    else if (!(k & 1))
+      v = -v;
+  }
+  return v;
+}
+
 // resolved shears, (|rs| / tau)^(n-1) and slip increments of the lane's
 // systems at x (stress) and tau
 __device__ inline void slips(const Props& p, const CState& s, const double* x,
@@ -577,7 +592,7 @@ __device__ inline void formJ(const Props& p, const CState& s, const double* x,
                              double tt, double (&A)[2][7]) {
   double rs[NSL], pw[NSL], gam[NSL], wv[NSL][6], dgdt[NSL], e[NSL], wp[3];
   slips(p, s, x, tt, rs, pw, gam);
-  const double itt = 1.0 / tt, nd = s.dg * p.rate_n * itt;
+  const double itt = 1.0 / tt, nd = flow_scale(p, s.dg, itt);
 #pragma unroll
   for (int i = 0; i < NSL; ++i) {
     dgdt[i] = nd * pw[i] + s.tinc * p.iD_v;
@@ -1273,7 +1288,7 @@ __device__ __forceinline__ void mm10_item(const DevModel& M,
 #pragma unroll
         for (int k = 0; k < 6; ++k) ep[k] = ep[k] / np1.tinc;
         n_eff = 0.0;
-        const double nd = np1.dg * p.rate_n / tt;
+        const double nd = flow_scale(p, np1.dg, 1.0 / tt);
 #pragma unroll
         for (int i = 0; i < NSL; ++i) {
           double dgdt = nd * pw[i] + np1.tinc * p.iD_v;
