@@ -419,7 +419,7 @@ int w3d_solve_pcg_dev(w3d_ctx* ctx, const double* d_k_diag,
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * It has no counterpart in the reference.  Same arguments and results as
  * w3d_solve_pcg_dev, but its work vectors live in a static device array of
- * the library (9 * 2^19 + 7180 doubles, about 37.8 MB per device, held
+ * the library (9 * 2^19 + 5388 doubles, about 37.8 MB per device, held
  * until the process ends) instead of the context's pattern-time workspace;
  * it calls no allocator.  Limit: at most 2^19 = 524,288 equations
  * (W3D_ERR_ARG beyond).  Every call on one device shares that array:
