@@ -185,8 +185,9 @@ int launch_recover(const DevModel& M, const std::vector<BlockDesc>& hblocks,
                    const std::vector<int>& group_count, int step, int iter,
                    int nonlinear, const double* d_u, const double* d_du,
                    int want_energy, double* en_wg, int pass, hipStream_t s);
-// mm10 update, one thread per point over work items of <= 64 points,
-// persistent: grid workgroups take items from the counter d_counter.
+// mm10 update, four lanes a point over work items of <= 64 points,
+// persistent: grid workgroups take 16 points at a time from the counter
+// d_counter.
 int launch_mm10(const DevModel& M, const WorkItem* d_work, int nwork,
                 int* d_counter, int grid, int step, int iter0_off,
                 hipStream_t s);
@@ -194,7 +195,7 @@ int launch_mm10(const DevModel& M, const WorkItem* d_work, int nwork,
 // graph in place of a memset)
 int launch_fill_i32(int32_t* d, int n, int32_t v, hipStream_t s);
 // grad Fe words of the small-strain mm10 blocks listed in d_blks whose
-// index lies in [lo, hi) (rknstr_finish_cp), one workgroup per block.
+// index lies in [lo, hi) (rknstr_finish_cp), several workgroups a block.
 int launch_mm10_grads(const DevModel& M, const int32_t* d_blks, int nblks,
                       int lo, int hi, int step, hipStream_t s);
 // The start of a recovery: flags cleared, and n words of u and du copied

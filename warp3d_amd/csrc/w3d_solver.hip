@@ -6,8 +6,9 @@
 // (drive_assemble_solve.f:654 -> drive_pardiso.f:11, and the MKL iterative
 // option of the same driver); the reference's element-by-element PCG
 // (old_code/EBE_solver/lnpcg_ser/lnpcg.f) is the precedent for a Jacobi
-// preconditioner.  Every reduction is a fixed tree (per-block partial sums
-// then one block over the partials), so a solve is bitwise repeatable.
+// preconditioner.  Every reduction is a fixed tree (per-workgroup partial
+// sums, then every workgroup over the partials), so a solve is bitwise
+// repeatable.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
