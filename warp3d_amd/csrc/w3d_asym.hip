@@ -31,7 +31,8 @@ namespace w3d {
 // Bound by the chain of dependent loads of a wave (group, node, incidences,
 // positions and Ke words).  A wave per equation row walked it three times a
 // node, with 24 of the 64 lanes at work on bricks, and its fixed 768-word
-// row held a CU to 24 waves; the rows' LDS is now the pattern's longest row.
+// row held a CU to 24 waves; the rows' LDS is now the pattern's longest row
+// (21,924 bricks: 110 -> 62 us, 2.3 TB/s of Ke words and values).
 constexpr int kAsmWaves = 4;
 constexpr int kAsmChunk = 4;  // elements whose loads are in flight together
 constexpr int kAsmRounds = (3 * kMaxDof + 63) / 64;  // (row, ecol) pairs

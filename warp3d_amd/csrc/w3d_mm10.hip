@@ -885,7 +885,9 @@ __device__ inline void euler_angles(const Props& p, const double* Rp_in,
 // a lane, whose reloads from the Infinity Cache every chain waited on at one
 // wave a SIMD; split over four lanes they fit half the registers, so two
 // waves share a SIMD, a wave runs the longest of 16 local solves instead of
-// 64, and small models spread over four times the waves.
+// 64, and small models spread over four times the waves.  167,000 points of
+// a mixed mesh: 1,636 -> 672 us (54 % of the vector issue); 1.9 million:
+// 32.6 -> 10.3 ms (72 %).
 // ---------------------------------------------------------------------
 constexpr int kCmsWords = 6 * NSL * kLanes;  // LDS of a wave: C ms,
 constexpr int kJacWords = 49 * kPts;         // the parked Jacobians,

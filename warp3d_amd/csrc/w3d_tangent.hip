@@ -40,7 +40,9 @@
 // over every 16x16 tile, in the element's own dof order, with the whole
 // 6x6 [D] (mm10: the point's history words 1-36, unsymmetrised; mm01: its
 // cep).  Word col T + row is sum_k B(k, col) BD(k, row), so the B columns
-// are the A operand and lanes walk consecutive words.  FP64 only.
+// are the A operand and lanes walk consecutive words.  FP64 only.  Against a
+// workgroup an element through LDS on the vector units: 21,924 bricks 329 ->
+// 72 us, 64,000 quadratic bricks 3.67 -> 1.63 ms (50 TFLOP/s).
 #include <hip/hip_runtime.h>
 
 #include "w3d_geonl.h"
