@@ -401,7 +401,10 @@ int w3d_solve_bicgstab(w3d_ctx* ctx, const double* rhs, double* x,
  * equations.  x holds the initial guess on entry and the solution on
  * return.  Stops when ||rhs - K x|| <= rtol ||rhs|| (W3D_OK) or after maxit
  * iterations (W3D_ERR_NUMERIC, x the last iterate); iters and relres (either
- * may be NULL) receive the iterations and the final relative residual.
+ * may be NULL) receive the iterations and the final relative residual.  The
+ * residual is the one the iteration carries: on ill-conditioned systems
+ * rounding leaves the true one larger (a row of 200 bricks, rtol 1e-8:
+ * 1.7e-7 to 5.4e-7, as the usual recurrences do on a host).
  * Replaces the reference's assembled-equation solve (drive_assemble_solve.f
  * :654 -> drive_pardiso.f:11; eqn_solve in mnralg.f:503).
  */
@@ -419,7 +422,7 @@ int w3d_solve_pcg_dev(w3d_ctx* ctx, const double* d_k_diag,
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * It has no counterpart in the reference.  Same arguments and results as
  * w3d_solve_pcg_dev, but its work vectors live in a static device array of
- * the library (9 * 2^19 + 5388 doubles, about 37.8 MB per device, held
+ * the library (8 * 2^19 + 8456 doubles, about 33.6 MB per device, held
  * until the process ends) instead of the context's pattern-time workspace;
  * it calls no allocator.  Limit: at most 2^19 = 524,288 equations
  * (W3D_ERR_ARG beyond).  Every call on one device shares that array:

@@ -938,7 +938,7 @@ int pcg_impl(w3d_ctx* c, const double* d_diag, const double* d_coef,
   int rc = solver_csr_values(d_diag, d_coef, n, c->d_csr_vidx, c->csr_nnz,
                              c->d_csr_val, s);
   // A x, then r = b - A x by the initialisation
-  if (!rc) rc = solver_spmv(c->groups(), c->d_csr_val, d_x, S.p, s);
+  if (!rc) rc = solver_spmv(c->groups(), c->d_csr_val, d_x, S.ax(), s);
   if (!rc) rc = launch_pcg_init(S, s, state, sc);
   const int32_t* st = nullptr;
   if (!rc)

@@ -295,22 +295,22 @@ int solver_spmv(const RowGroups& A, const double* val, const double* x,
 // One system of a Jacobi-PCG: the full CSR rows of its assembled matrix,
 // its diagonal, right-hand side and vectors, the workgroups of its launches
 // (from its size alone) and their partial sums.
-// single: x holds the initial guess and p A x on entry, the convergence
-// test runs before the first iteration too and a residual that is no
-// number ends the solve; a system of a batch starts from x = 0.
+// single: x holds the initial guess and row[0]'s memory A x on entry, the
+// convergence test runs before the first iteration too and a residual that
+// is no number ends the solve; a system of a batch starts from x = 0.
 constexpr int kPcgMaxMul = 768, kPcgMaxVec = 1024;
 constexpr int32_t kPcgZeroRhs = 4;  // a single solve's state on |b| = 0
-// PcgRow: residual, w = A D^-1 r, s and 1 / diagonal of one equation.
+// PcgRow: residual, direction, s = A p and 1 / diagonal of one equation.
 struct alignas(32) PcgRow {
-  double r, w, s, rd;
+  double r, p, s, rd;
 };
+constexpr int kPcgSums = 5;  // of an iteration (k_pcg_iter)
 struct PcgSys {
   RowGroups A;
   const double* val;
   const double* diag;
   const double* b;
   double* x;
-  double* p;
   PcgRow* row[2];         // by the parity of the launch that reads it
   double* part;           // pcg_part_words of partial sums and scalars
   double rtol;            // |r| <= rtol |b| ends the solve
@@ -322,34 +322,31 @@ struct PcgSys {
   void set_work(double* w) {
     row[0] = reinterpret_cast<PcgRow*>(w);
     row[1] = row[0] + n;
-    p = w + 8 * (int64_t)n;
   }
-  // per workgroup b.b, then the three sums of each parity, then (r.u,
-  // alpha) of each parity
+  __host__ __device__ double* ax() const {
+    return reinterpret_cast<double*>(row[0]);
+  }
+  // per workgroup b.b, then the sums of each parity
   __host__ __device__ int off_bb() const { return 0; }
   __host__ __device__ int off_sums(int par) const {
-    return (1 + 3 * par) * nwg;
-  }
-  __host__ __device__ int off_scalars(int par) const {
-    return 7 * nwg + 2 * par;
+    return (1 + kPcgSums * par) * nwg;
   }
 };
 int pcg_mul_wgs(int ngrp);
 int pcg_vec_wgs(int n);
-constexpr int pcg_part_words(int nwg) { return 7 * nwg + 4; }
-// A single solve's work array: kPcgVectors n doubles (the rows twice, p),
-// then 2 scalars (|b|, r.r), the state (done: 0 running, 1 converged,
-// 2 iteration limit, kPcgZeroRhs; iterations; two gates) and the partial
-// sums.
-constexpr int kPcgVectors = 9;
+constexpr int pcg_part_words(int nwg) { return (1 + 2 * kPcgSums) * nwg; }
+// A single solve's work array: kPcgVectors n doubles (the rows twice), then
+// 2 scalars (|b|, r.r), the state (done: 0 running, 1 converged, 2 iteration
+// limit, kPcgZeroRhs; iterations; two gates) and the partial sums.
+constexpr int kPcgVectors = 8;
 constexpr int kPcgTail = 8 + pcg_part_words(kPcgMaxMul);
 int launch_pcg_init(const PcgSys& one, hipStream_t s, int32_t* state,
                     double* sc);
 int launch_pcg_iter(const PcgSys& one, int it, int32_t* state, double* sc,
                     hipStream_t s);
 // w3d_solve_pcg_static's work memory: a file-scope device array of
-// 5 kStaticMaxEq + kPcgTail doubles, its address on `device` (the caller
-// has made that device current)
+// kPcgVectors kStaticMaxEq + kPcgTail doubles, its address on `device` (the
+// caller has made that device current)
 constexpr int kStaticMaxEq = 1 << 19;
 constexpr int kMaxDevices = 64;
 int solver_static_scratch(int device, double** out);

@@ -69,7 +69,7 @@ __global__ void k_csr_values(const double* __restrict__ diag,
 // lanes: the 81 columns of a structured brick's node are three entries a
 // lane, loaded together, and a 1,000-node system still spreads over 32,000
 // lanes.  Bound by memory on large systems (124,740 equations, 9.5 M
-// entries: 27 us, 3.3 TB/s).  Each row sums its lanes' strided shares in a
+// entries: 28 us, 3.2 TB/s).  Each row sums its lanes' strided shares in a
 // fixed butterfly, so products are bitwise repeatable.  Workgroups of 256:
 // of 512, an iteration on one to three systems of 2,000 to 3,600 equations
 // took 7.3 to 7.8 us for 6.0 to 7.4.
@@ -196,32 +196,44 @@ __global__ void __launch_bounds__(kMulBlock)
 
 // ---------------------------------------------------------------------
 // Jacobi-PCG over one system or a batch of independent ones, one launch an
-// iteration, in the single-reduction form of the recurrences (Chronopoulos
-// and Gear 1989): with u = D^-1 r and w = A u
-//   beta = g / g-, alpha = g / (d - beta g / alpha-),  g = (r, u), d = (w, u)
-//   p = u + beta p, s = w + beta s, x += alpha p, r -= alpha s
-// so that one product and one set of sums (r.r, r.u, w.u) make an iteration.
-// A launch forms the scalars from the last launch's partial sums, the new r
-// and u at the columns it gathers (from the old r, w, s and 1 / diag, 32
-// bytes a column, kept in two buffers by the launch's parity) and w = A u of
-// its own rows.  The matrix, column and vector words of a workgroup's first
-// tile are loaded before the scalars are known: neither needs the other.
+// iteration, in the form of the usual recurrences that needs one set of sums
+// (Meurant 1984): with u = D^-1 r and s = A p
+//   alpha = g / (p, s),  g = (r, u)
+//   beta = (g - 2 alpha (s, u) + alpha^2 (s, D^-1 s)) / g
+//   x += alpha p, r -= alpha s, p = D^-1 r + beta p
+// The bracket is (r, u) of the new r, formed from sums the old vectors give,
+// so that beta does not wait for them; the next alpha takes the new (r, u)
+// as summed.  A launch forms the scalars from the last launch's partial sums,
+// the new r and p at the columns it gathers (from the old r, p, s and
+// 1 / diag, 32 bytes a column, kept in two buffers by the launch's parity),
+// s = A p of its own rows and the five sums (with r.r, for the test).  The
+// matrix, column and vector words of a workgroup's first tile are loaded
+// before the scalars are known: neither needs the other.
+//
+// s is a product and alpha a quotient of sums taken directly: with
+// w = A u as the product, s = w + beta s and alpha = g / ((w, u) - beta g /
+// alpha-) (Chronopoulos and Gear 1989, three sums) the recurrence's rounding
+// errors cost slender or nearly incompressible models 5 to 60 % more
+// iterations and up to twice the true residual (bricks in a row of 200, to
+// 1e-8: 8,200 to 8,600 iterations, 11,700 to 12,800 so).
 //
 // A launch is a chain of dependent loads and two workgroup sums on small
 // systems, and the host reads the states behind the device, so an iteration
 // costs no synchronisation.  Measured an iteration, against two launches
-// (product, vector update) of the usual recurrences: 10.4 -> 7.5 us on three
-// systems of 2,000 to 3,600 equations, 32.4 -> 27.4 us on 124,740, and a
-// launch gap less.  Three waves a SIMD: at four, the next group's words
-// (below) spilled, and a solve of 124,740 equations took 41 us an iteration.
+// (product, vector update): 10.4 -> 7.5 us on three systems of 2,000 to 3,600
+// equations, 32.4 -> 28.1 us on 124,740 (27.4 with three sums, a solve 2 %
+// less; a request of three served models the same within 1 %).  Three waves
+// a SIMD: at four, the next group's words (below) spilled, and a solve of
+// 124,740 equations took 41 us an iteration.
 // Each system's reductions run over its own workgroups in a
 // fixed order, whose number depends on the system's size alone, so a
 // system's iterates do not depend on the batch.  Every workgroup of a system
 // reaches the same end-of-solve decision from the same partials and the
-// first one writes it.  A launch never reads a word that it writes: state
-// (done, iterations per system) is the host's, and the vectors, partial
-// sums, scalars and gates are double, read at the launch's parity and
-// written at the other.
+// first one writes it.  What other lanes read is never written by the same
+// launch: the gathered rows, the partial sums and the gates are double, read
+// at the launch's parity and written at the other, and state (done,
+// iterations per system) is the host's.  x is updated in place, each entry
+// by the one lane that reads it.
 // ---------------------------------------------------------------------
 template <bool BATCH>
 __global__ void __launch_bounds__(kMulBlock)
@@ -238,13 +250,12 @@ __global__ void __launch_bounds__(kMulBlock)
     const double bi = S.b[i];
     double ri = bi;
     if (S.single)
-      ri = bi - S.p[i];  // p holds A x0
+      ri = bi - S.ax()[i];
     else
       S.x[i] = 0.0;
-    S.p[i] = 0.0;
     PcgRow q;
     q.r = ri;
-    q.w = q.s = 0.0;
+    q.p = q.s = 0.0;
     q.rd = 1.0 / S.diag[i];
     S.row[1][i] = q;
     v[0] = v[0] + bi * bi;
@@ -282,7 +293,7 @@ __global__ void __launch_bounds__(kMulBlock)
                const int32_t* __restrict__ owner, int it,
                int32_t* __restrict__ state, int32_t* __restrict__ gate,
                double* __restrict__ sc) {
-  __shared__ double s_red[3][kMulBlock / 64];
+  __shared__ double s_red[kPcgSums][kMulBlock / 64];
   const int si =
       BATCH ? __builtin_amdgcn_readfirstlane(owner[blockIdx.x]) : 0;
   const PcgSys& S = BATCH ? sys[si] : one;
@@ -296,12 +307,11 @@ __global__ void __launch_bounds__(kMulBlock)
   int g = wg * kGrpPerWg + tid / kGrpLanes;
   GrpTile<PcgRow> t;
   PcgRow o;          // lane k < rows: row k's own vectors
-  double po, xo;
+  double xo;
   auto load = [&]() {  // of the group whose word and columns t has
     tile_entries(S.val, row, lane, 0, t);
     const int i = t.d.row0 + (lane < t.d.rows() ? lane : 0);
     o = row[i];
-    po = S.p[i];
     xo = S.x[i];
   };
   if (g < S.A.ngrp) {
@@ -312,11 +322,11 @@ __global__ void __launch_bounds__(kMulBlock)
   double alpha = 0.0, beta = 0.0;
   if (it >= 0) {
     const double* pt = S.part + S.off_sums(par);
-    double v[3] = {0.0, 0.0, 0.0};  // r.r, r.u, w.u
+    double v[kPcgSums] = {};  // r.r, r.u, p.s, s.u, s.(s / diag)
     for (int i = tid; i < S.nwg; i += kMulBlock)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) v[k] = v[k] + pt[k * S.nwg + i];
-    block_sums<3, kMulBlock>(v, s_red);
+      for (int k = 0; k < kPcgSums; ++k) v[k] = v[k] + pt[k * S.nwg + i];
+    block_sums<kPcgSums, kMulBlock>(v, s_red);
     // the end of the solve: |r| <= rtol |b| or the iteration limit (a batch
     // tests neither before its first iteration; a single solve also stops
     // on a residual that is no number)
@@ -332,25 +342,15 @@ __global__ void __launch_bounds__(kMulBlock)
       }
       return;
     }
-    const double* last = S.part + S.off_scalars(par);  // g, alpha
-    double* next = S.part + S.off_scalars(par ^ 1);
-    if (it > 0) {
-      beta = v[1] / last[0];
-      alpha = v[1] / (v[2] - beta * v[1] / last[1]);
-    } else {
-      alpha = v[1] / v[2];
-    }
-    if (wg == 0 && tid == 0) {
-      next[0] = v[1];
-      next[1] = alpha;
-    }
+    alpha = v[1] / v[2];
+    beta = (v[1] + alpha * (alpha * v[4] - 2.0 * v[3])) / v[1];
   }
-  // the new residual of a row from its old vectors
-  auto residual = [&](const PcgRow& q, double& s) {
-    s = q.w + beta * q.s;
-    return q.r - alpha * s;
+  // the new residual and direction of a row from its old vectors
+  auto residual = [&](const PcgRow& q) { return q.r - alpha * q.s; };
+  auto direction = [&](const PcgRow& q, double r) {
+    return r * q.rd + beta * q.p;
   };
-  double v[3] = {0.0, 0.0, 0.0};
+  double v[kPcgSums] = {};
   while (g < S.A.ngrp) {
     // the next group's word and columns come in behind this one's products
     const int gn = g + S.nwg * kGrpPerWg;
@@ -362,27 +362,23 @@ __global__ void __launch_bounds__(kMulBlock)
     PcgRow n;
     if (own) {
       n.rd = o.rd;
-      n.r = residual(o, n.s);
-      if (it >= 0) {
-        const double p = o.r * n.rd + beta * po;
-        S.p[i] = p;
-        S.x[i] = xo + alpha * p;
-      }
+      n.r = residual(o);
+      n.p = direction(o, n.r);
+      if (it >= 0) S.x[i] = xo + alpha * o.p;
     }
     double y[3];
     tile_product(S.A, S.val, row, lane, t,
-                 [&](const PcgRow& q) {
-                   double s;
-                   return residual(q, s) * q.rd;
-                 },
+                 [&](const PcgRow& q) { return direction(q, residual(q)); },
                  y);
     if (own) {
-      n.w = lane == 0 ? y[0] : lane == 1 ? y[1] : y[2];
+      n.s = lane == 0 ? y[0] : lane == 1 ? y[1] : y[2];
       S.row[par ^ 1][i] = n;
       const double u = n.r * n.rd;
       v[0] = v[0] + n.r * n.r;
       v[1] = v[1] + n.r * u;
-      v[2] = v[2] + n.w * u;
+      v[2] = v[2] + n.p * n.s;
+      v[3] = v[3] + n.s * u;
+      v[4] = v[4] + n.s * (n.s * n.rd);
     }
     g = gn;
     if (g < S.A.ngrp) {
@@ -392,18 +388,18 @@ __global__ void __launch_bounds__(kMulBlock)
       load();
     }
   }
-  block_sums<3, kMulBlock>(v, s_red);
+  block_sums<kPcgSums, kMulBlock>(v, s_red);
   if (tid == 0)
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
+    for (int k = 0; k < kPcgSums; ++k)
       S.part[S.off_sums(par ^ 1) + k * S.nwg + wg] = v[k];
 }
 
 // Workgroups of one system's launches: a tile of groups (rows) each up to
 // the cap, then equal shares.  The caps bound the partial sums that every
 // workgroup of the next launch reads again, and keep a launch's workgroups
-// resident together at three waves a SIMD (124,740 equations: 27.4 us an
-// iteration on 743, 34.1 on 867).
+// resident together at three waves a SIMD (124,740 equations: 28.1 us an
+// iteration on 743; 27.4 and, on 867, 34.1 before the five sums).
 int pcg_mul_wgs(int ngrp) {
   const int t = (ngrp + kGrpPerWg - 1) / kGrpPerWg;
   if (t < 1) return 1;
