@@ -144,6 +144,32 @@ def test_block_ranges_and_fp32_subrange():
     dev.close()
 
 
+def test_a_crystal_block_takes_no_longer_than_a_model_of_it():
+    """The crystal update of a block called alone runs on as many waves as
+    that of a model whose only block it is: with a quarter of them the call
+    took 279 us, the model's 141 (both are the same launches, the model's with
+    its sums in one; the shortest of many calls of each)."""
+    import time
+    from warp3d_amd.model import BlockModel
+    m = M.box_hex8(8, 4, 4, jitter=0.1, seed=45)
+    dev = BlockModel(m.model(cubic_fcc(), auto_size=128,
+                             angles=M.random_orientations(128, seed=46)))
+    assert dev.nelblk == 1
+    u, du = np.zeros(3 * m.nonode), smooth_field(m, 0.0005, seed=3)
+    dev.set_displacements(u, du)
+    calls = {"model": lambda: dev.recover(1, 1, u, du),
+             "block": lambda: dev.recover_block(1, 1, 1)}
+    best = {}
+    for _ in range(20):
+        for k, f in calls.items():
+            t = time.perf_counter()
+            f()
+            t = time.perf_counter() - t
+            best[k] = min(t, best.get(k, t))
+    print({k: f"{1e6 * t:.0f} us" for k, t in best.items()})
+    assert best["block"] <= 1.5 * best["model"], best
+
+
 def test_a_cut_is_reported_by_its_block():
     """Only the blocks whose crystals cannot take the increment report the
     cut; the oracle's blocks agree one by one."""

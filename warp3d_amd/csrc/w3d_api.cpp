@@ -699,7 +699,8 @@ void return_stream(w3d_ctx* c, hipStream_t s) {
 
 // The recovery of block b (0-based) on stream s, with the displacements of
 // w3d_set_displacements: the block's flags cleared, the first pass, for
-// mm10 the material update over the block's own items (its own counter),
+// mm10 the material update over the block's own items (its own counter; a
+// workgroup for each part of an item: 128 bricks 279 -> 130 us a call),
 // grad Fe and the second pass, then the block's sums.
 int enqueue_block_recover(w3d_ctx* c, int b, hipStream_t s, int step,
                           int iter, int extrapolated) {
@@ -716,8 +717,8 @@ int enqueue_block_recover(w3d_ctx* c, int b, hipStream_t s, int step,
                         0, s);
   if (!rc && R.mm10_n > 0) {
     rc = launch_mm10(M, c->d_work_mm10 + R.mm10_first, R.mm10_n,
-                     c->d_blk_counter + b, std::min(c->mm10_grid, R.mm10_n),
-                     step, mm10_iter0_off(step, iter, extrapolated), s);
+                     c->d_blk_counter + b, c->mm10_grid, step,
+                     mm10_iter0_off(step, iter, extrapolated), s);
     if (!rc)
       rc = launch_mm10_grads(M, c->d_mm10_blks + R.mm10_idx, 1, b, b + 1,
                              step, s);
