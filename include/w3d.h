@@ -474,12 +474,13 @@ int w3d_iteration_dev(w3d_ctx* ctx, int32_t step, int32_t iter,
 /*
  * Autotuner (no reference counterpart: the reference's block size is the
  * fixed mxvl): times the block tangent of every kernel group with work
- * items of 8, 16, 32 and 64 elements and keeps the fastest, and the
- * persistent mm10 kernel with 2, 4 and 8 workgroups per compute unit.  Run
- * it after a recovery of a representative iteration (mm10 is timed on the
- * increments in place).  choices receives (group key, elements) pairs, then
- * (-1, mm10 workgroups) when the model has mm10 blocks; *n_choices their
- * number of words.  Captured iterations are dropped.
+ * items of the library's own size and of 8, 16, 32 and 64 elements and keeps
+ * the fastest, and the persistent mm10 kernel with 2, 4 and 8 workgroups per
+ * compute unit.  Run it after a recovery of a representative iteration (mm10
+ * is timed on the increments in place).  choices receives a (group key, elements) pair for
+ * each group that leaves the library's own size, then (-1, mm10 workgroups)
+ * when the model has mm10 blocks; *n_choices their number of words.
+ * Captured iterations are dropped.
  */
 int w3d_autotune(w3d_ctx* ctx, int32_t precision, int32_t* choices,
                  int32_t capacity, int32_t* n_choices);

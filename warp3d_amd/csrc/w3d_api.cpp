@@ -2290,19 +2290,21 @@ int w3d_autotune(w3d_ctx* c, int32_t precision, int32_t* choices,
   std::vector<int32_t> out;
   int rc = W3D_OK;
   // tangent: per kernel group the work-item size, in elements, with the
-  // shortest launch (the mean of three, after one untimed launch)
+  // shortest launch (the mean of three, after one untimed launch); 0 is
+  // build_work's own
+  auto set_chunk = [&](int key, int chunk) {
+    auto& tc = c->tan_chunk;
+    tc.erase(std::remove_if(tc.begin(), tc.end(),
+                            [&](const auto& kc) { return kc.first == key; }),
+             tc.end());
+    if (chunk > 0) tc.push_back({key, chunk});
+  };
   const std::vector<int> groups = c->tan_groups;
   for (int key : groups) {
     int best = 0;
     float best_ms = 0.0f;
-    for (int chunk : {8, 16, 32, 64}) {
-      bool found = false;
-      for (auto& kc : c->tan_chunk)
-        if (kc.first == key) {
-          kc.second = chunk;
-          found = true;
-        }
-      if (!found) c->tan_chunk.push_back({key, chunk});
+    for (int chunk : {0, 8, 16, 32, 64}) {
+      set_chunk(key, chunk);
       std::vector<WorkItem> items;
       std::vector<int> g, st, cnt;
       build_work(c, true, items, g, st, cnt);
@@ -2324,14 +2326,14 @@ int w3d_autotune(w3d_ctx* c, int32_t precision, int32_t* choices,
       if (rc) break;
       float ms = 0.0f;
       (void)hipEventElapsedTime(&ms, ea, eb);
-      if (!best || ms < best_ms) {
+      if (!chunk || ms < best_ms) {
         best = chunk;
         best_ms = ms;
       }
     }
+    set_chunk(key, rc ? 0 : best);
     if (rc) break;
-    for (auto& kc : c->tan_chunk)
-      if (kc.first == key) kc.second = best;
+    if (!best) continue;
     out.push_back(key);
     out.push_back(best);
   }

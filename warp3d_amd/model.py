@@ -318,7 +318,8 @@ class BlockModel:
 
     def autotune(self, precision=0):
         """Runs the autotuner; returns {group key: elements per work item}
-        and, with mm10 blocks, {-1: mm10 workgroups}."""
+        of the groups that leave the library's own size and, with mm10
+        blocks, {-1: mm10 workgroups}."""
         buf = (C.c_int32 * 64)()
         n = C.c_int32()
         _chk(lib().w3d_autotune(self.h, precision, buf, 64, C.byref(n)),
