@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include "w3d_internal.h"
+#include "w3d_wave.h"
 
 namespace w3d {
 
@@ -36,7 +37,6 @@ namespace w3d {
 constexpr int kAsmWaves = 4;
 constexpr int kAsmChunk = 4;  // elements whose loads are in flight together
 constexpr int kAsmRounds = (3 * kMaxDof + 63) / 64;  // (row, ecol) pairs
-__device__ inline void wave_fence() { __builtin_amdgcn_wave_barrier(); }
 
 __global__ void __launch_bounds__(64 * kAsmWaves)
     k_assemble_full(const double* __restrict__ ekf,
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves)
   const int len = gd.len();  // <= maxrow
   double* row = s_rows + (size_t)wv * 3 * maxrow;
   for (int k = lane; k < nr * len; k += 64) row[k] = 0.0;
-  wave_fence();
+  wave_sync();
   const int d0 = eq_dof[r0], node = d0 / 3;
   const int comp0 = d0 % 3;
   const int comp1 = nr > 1 ? eq_dof[r0 + 1] % 3 : 0;
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves)
 #pragma unroll
       for (int m = 0; m < kAsmRounds; ++m)
         if (pos[j][m] >= 0) row[pos[j][m]] = row[pos[j][m]] + v[j][m];
-      wave_fence();
+      wave_sync();
     }
   }
   for (int k = lane; k < nr * len; k += 64) val[v0 + k] = row[k];

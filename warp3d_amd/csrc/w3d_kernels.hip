@@ -16,6 +16,7 @@
 
 #include "w3d_geonl.h"
 #include "w3d_internal.h"
+#include "w3d_wave.h"
 
 namespace w3d {
 
@@ -954,13 +955,14 @@ __global__ void __launch_bounds__(64 * kAsmVssWaves)
   constexpr int U = kAsmVssWindow / 64;
   // a window's words, then the wave's (at most 192) outputs
   constexpr int kIn = 3 * kAsmVssWindow * (int)sizeof(KT), kOut = 192 * 8;
-  __shared__ double s_all[kAsmVssWaves][(kIn > kOut ? kIn : kOut) / 8];
+  __shared__ __align__(8) unsigned char
+      s_all[kAsmVssWaves][kIn > kOut ? kIn : kOut];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t w = (int64_t)blockIdx.x * kAsmVssWaves + wv;
   if (w * 64 >= nseg) return;  // uniform across the wave
   const int64_t t = w * 64 + lane;
   KT* in = reinterpret_cast<KT*>(s_all[wv]);
-  double* out = s_all[wv];
+  double* out = reinterpret_cast<double*>(s_all[wv]);
   const int h = t < nseg ? hdr[t] : 0;
   const int n = h & 255, mask = (h >> 8) & 7, len = __popc(mask);
   // contributions (at most 64 * 255) and outputs scanned together
@@ -984,7 +986,7 @@ __global__ void __launch_bounds__(64 * kAsmVssWaves)
 #pragma unroll
     for (int j = 0; j < U; ++j)
       v[j] = *reinterpret_cast<const Ke3<KT>*>(ek + b[j]);
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       const int k = 64 * j + lane;
@@ -994,7 +996,7 @@ __global__ void __launch_bounds__(64 * kAsmVssWaves)
         in[3 * k + 2] = v[j].w[2];
       }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     const int ka = (n0 > c0 ? n0 : c0) - c0;
     const int ke = (n1 < c0 + m ? n1 : c0 + m) - c0;
     for (int k = ka; k < ke; ++k) {
@@ -1003,12 +1005,12 @@ __global__ void __launch_bounds__(64 * kAsmVssWaves)
       s2 = s2 + (double)in[3 * k + 2];
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   int o = l0;
   if (mask & 1) out[o++] = s0;
   if (mask & 2) out[o++] = s1;
   if (mask & 4) out[o++] = s2;
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   for (int k = lane; k < ltot; k += 64) {
     if (oo + k < neq)
       diag[oo + k] = out[k];

@@ -30,6 +30,7 @@
 #include <algorithm>
 
 #include "w3d_internal.h"
+#include "w3d_wave.h"
 
 namespace w3d {
 namespace {
@@ -106,13 +107,6 @@ __device__ inline double uniform(double v) {
 __device__ inline int64_t uniform(int64_t v) {
   return (int64_t)(uint32_t)uniform((int)v) |
          (int64_t)uniform((int)(v >> 32)) << 32;
-}
-
-// Orders a wave's own LDS traffic (its quads exchange through their slabs).
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ inline double sgn(double x) { return x >= 0.0 ? 1.0 : -1.0; }

@@ -47,6 +47,7 @@
 
 #include "w3d_geonl.h"
 #include "w3d_internal.h"
+#include "w3d_wave.h"
 
 namespace w3d {
 
@@ -69,14 +70,6 @@ struct Mfma<double> {
   }
   __device__ static int row(int l, int v) { return (l >> 4) + 4 * v; }
 };
-
-// Wave-level synchronisation: the lanes of one wave exchange data through
-// their own LDS slab, so the wave only has to order its own LDS traffic.
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The B columns of a node's three components (x, y, z) from its gradient
 // (bx, by, bz) and, for B-bar, its volume-averaged gradient vol[3 j + c]:
