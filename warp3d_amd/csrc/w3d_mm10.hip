@@ -68,34 +68,6 @@ struct CState {
   __device__ double cm(int j, int r) const { return cms[(6 * j + r) * kLanes]; }
 };
 
-template <int CTRL>
-__device__ inline int qperm(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ inline double qperm(double v) {
-  return __hiloint2double(qperm<CTRL>(__double2hiint(v)),
-                          qperm<CTRL>(__double2loint(v)));
-}
-// the quad's exchanges: with the neighbour (1 0 3 2), across (2 3 0 1)
-constexpr int kDppNext = 0xB1, kDppCross = 0x4E;
-template <typename T>
-__device__ inline T qsum(T v) {
-  v = v + qperm<kDppNext>(v);
-  return v + qperm<kDppCross>(v);
-}
-// the value of the quad's lane S
-template <int S, typename T>
-__device__ inline T qbcast(T v) {
-  return qperm<S * 0x55>(v);
-}
-// the argument of the lane's own number
-__device__ inline double qpick(int sub, double a, double b, double c,
-                               double d) {
-  const double lo = sub & 1 ? b : a, hi = sub & 1 ? d : c;
-  return sub & 2 ? hi : lo;
-}
-
 // a value that is the same in every lane, in scalar registers
 __device__ inline int uniform(int v) {
   return __builtin_amdgcn_readfirstlane(v);
