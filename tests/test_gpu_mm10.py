@@ -174,3 +174,30 @@ def test_mm10_parts_and_exponents(W, span, ncry, n, m_exp):
     arr = m.model(mat, auto_size=span, angles=ang, angle_stride=ncry)
     run(W.BlockModel(arr), O.OracleModel(arr), m, ncry=ncry,
         tag=f"span {span}")
+
+
+@pytest.mark.parametrize("n,rc", [(20.0, 0), (17.0, 0),
+                                  (17.5, _abi.W3D_CUT_STEP)])
+def test_mm10_negative_tau(W, n, rc):
+    """A hardening variable below zero, as stray iterates have: the slips'
+    derivative carries tau^n, positive for an even exponent, negative for an
+    odd one and no number (a step cut) for a broken one.  With the sign of
+    the even exponent turned, the oracle's [D] moves by 2.3e-3 relative."""
+    m = M.box_hex8(2, jitter=0.1, seed=9)
+    arr = m.model(cubic_fcc(harden_n=n, theta_0=20.0), auto_size=4,
+                  angles=M.random_orientations(m.noelem, seed=4))
+    dev, orc = W.BlockModel(arr), O.OracleModel(arr)
+    u, du = np.zeros(3 * m.nonode), smooth_field(m, 0.0005, seed=1)
+    for x in (dev, orc):
+        assert x.recover(1, 1, u, du)[3] == 0
+        x.commit_step()
+    for b in range(1, orc.nelblk + 1):
+        h = orc.get_block_state(b, _abi.HIST_N).reshape(-1, 87 + 71)
+        h[:, 87 + 42] = -80.0
+        for x in (dev, orc):
+            x.set_block_state(b, _abi.HIST_N, h.ravel())
+    du2 = smooth_field(m, 0.0002, seed=2)
+    assert orc.recover(2, 1, u + du, du2)[3] == rc
+    assert dev.recover(2, 1, u + du, du2)[3] == rc
+    if rc == 0:
+        compare(dev, orc, 1, f"n {n}")
