@@ -60,10 +60,10 @@ def kernel_name(phase, workload, fp32=True):
             "mixed": "8, 8, true"}[workload]
     prec = "float" if fp32 else "double"
     return {"recover": f"k_recover<{tmpl}, 0, false>",
-            "ifv_gather": "k_ifv_gather",
-            "tangent": f"k_tangent_mfma<{tmpl}, {prec}, false, false>",
+            "ifv_gather": "k_recover_end",
+            "tangent": f"k_tangent_mfma<{tmpl}, {prec}, false, false, false>",
             "assemble": f"k_assemble<{prec}>",
-            "energy_reduce": "k_energy_reduce",
+            "energy_reduce": "k_recover_end",
             "mm10": "k_mm10"}[phase]
 FP64_PEAK_TFS = 78.6          # MI355X FP64 (vector and matrix)
 FP32_MFMA_PEAK_TFS = 157.3    # MI355X dense FP32 matrix

@@ -152,3 +152,21 @@ def test_tuning_a_small_model_does_not_slow_it(W, prec):
             best[k] = min(t[1] / t[0], best.get(k, 1e9))
     print(best)
     assert best["tuned"] <= 1.05 * best["plain"], best
+
+
+def test_pattern_leaves_no_spinning_threads(W):
+    """After w3d_pattern of a large model the host's threads are idle: its
+    last parallel loop lies before some 300 ms of serial work and copies, past
+    the 200 ms for which OpenMP's threads spin.  With one at the end they
+    used 2.8 s of processor time in the next 250 ms, and calls beside a
+    caller's own threads stalled for 4 ms each."""
+    import time
+    m = M.box_hex8(64)
+    dev = W.BlockModel(m.model(
+        _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0), auto_size=128))
+    cst = np.zeros(3 * m.nonode, np.int32)
+    cst[:3] = 1
+    dev.pattern(cst)
+    t = time.process_time()
+    time.sleep(0.25)
+    assert time.process_time() - t < 0.2

@@ -1595,6 +1595,11 @@ static int finish_pattern(w3d_ctx* c, int32_t* neqns_out,
         vidx[f] = (uint32_t)(neq + k);
       }
     }
+    // rows in groups that share their columns: the consecutive equations
+    // of one node (a row's columns compared with the row before it, while
+    // they are at hand; a parallel loop here, the last of the set-up, left
+    // its threads spinning for 200 ms beside the caller's first iterations)
+    std::vector<RowGroup> grp;
     for (int r = 0; r < neq; ++r) {
       int64_t f = fill[r];
       col[f] = r;
@@ -1604,6 +1609,14 @@ static int finish_pattern(w3d_ctx* c, int32_t* neqns_out,
         col[f] = c->k_indexes[k] - 1;
         vidx[f] = (uint32_t)(neq + k);
       }
+      const int32_t len = (int32_t)(rp[r + 1] - rp[r]);
+      if (r > 0 && c->eqn_node_map[r] == c->eqn_node_map[r - 1] &&
+          grp.back().len() == len && grp.back().rows() < 3 &&
+          std::equal(col.begin() + rp[r], col.begin() + rp[r + 1],
+                     col.begin() + rp[r - 1]))
+        grp.back().nl += 1;
+      else
+        grp.push_back({rp[r], r, len << 2 | 1});
     }
     dfree(c->d_csr_rp);
     dfree(c->d_csr_col);
@@ -1616,22 +1629,6 @@ static int finish_pattern(w3d_ctx* c, int32_t* neqns_out,
     if ((rc = upload(&c->d_csr_col, col))) return rc;
     if ((rc = upload(&c->d_csr_vidx, vidx))) return rc;
     if ((rc = dalloc(&c->d_csr_val, nnz))) return rc;
-    // rows in groups that share their columns: the consecutive equations
-    // of one node (a row's columns compared with the row before it)
-    std::vector<uint8_t> same(neq > 0 ? neq : 1, 0);
-#pragma omp parallel for schedule(static)
-    for (int r = 1; r < neq; ++r)
-      same[r] = c->eqn_node_map[r] == c->eqn_node_map[r - 1] &&
-                rp[r + 1] - rp[r] == rp[r] - rp[r - 1] &&
-                std::equal(col.begin() + rp[r], col.begin() + rp[r + 1],
-                           col.begin() + rp[r - 1]);
-    std::vector<RowGroup> grp;
-    for (int r = 0; r < neq; ++r) {
-      if (r > 0 && same[r] && grp.back().rows() < 3)
-        grp.back().nl += 1;
-      else
-        grp.push_back({rp[r], r, (int32_t)(rp[r + 1] - rp[r]) << 2 | 1});
-    }
     c->csr_ngrp = (int)grp.size();
     dfree(c->d_csr_grp);
     if ((rc = upload(&c->d_csr_grp, grp))) return rc;

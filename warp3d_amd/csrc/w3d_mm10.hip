@@ -35,7 +35,6 @@
 namespace w3d {
 namespace {
 
-constexpr int NS = 12;
 // Four lanes (a quad) share a point: lane `sub` of the quad owns the slip
 // systems 3 sub .. 3 sub + 2 and, of a matrix, the columns sub, sub + 4 (and
 // sub + 8).  Sums over the systems are a partial sum of the lane's three and

@@ -69,7 +69,7 @@ __global__ void k_csr_values(const double* __restrict__ diag,
 // lanes: the 81 columns of a structured brick's node are three entries a
 // lane, loaded together, and a 1,000-node system still spreads over 32,000
 // lanes.  Bound by memory on large systems (124,740 equations, 9.5 M
-// entries: 28 us, 3.2 TB/s).  Each row sums its lanes' strided shares in a
+// entries: 28 us, 4.7 TB/s).  Each row sums its lanes' strided shares in a
 // fixed butterfly, so products are bitwise repeatable.  Workgroups of 256:
 // of 512, an iteration on one to three systems of 2,000 to 3,600 equations
 // took 7.3 to 7.8 us for 6.0 to 7.4.
@@ -220,9 +220,9 @@ __global__ void __launch_bounds__(kMulBlock)
 // A launch is a chain of dependent loads and two workgroup sums on small
 // systems, and the host reads the states behind the device, so an iteration
 // costs no synchronisation.  Measured an iteration, against two launches
-// (product, vector update): 10.4 -> 7.5 us on three systems of 2,000 to 3,600
-// equations, 32.4 -> 28.1 us on 124,740 (27.4 with three sums, a solve 2 %
-// less; a request of three served models the same within 1 %).  Three waves
+// (product, vector update): 10.5 -> 8.0 us on three systems of 2,000 to 3,600
+// equations, 32.4 -> 28.2 us (4.7 TB/s) on 124,740; with three sums 7.4 and
+// 27.4, the request of three served models the same within 1 %.  Three waves
 // a SIMD: at four, the next group's words (below) spilled, and a solve of
 // 124,740 equations took 41 us an iteration.
 // Each system's reductions run over its own workgroups in a
