@@ -944,7 +944,7 @@ int pcg_impl(w3d_ctx* c, const double* d_diag, const double* d_coef,
   const int32_t* st = nullptr;
   if (!rc)
     rc = solve_poll([&](int it) { return launch_pcg_iter(S, it, state, sc, s); },
-                    1, maxit, kPollChunk, state, c->h_poll, c->poll_ev, s,
+                    1, maxit, 1, kPollChunk, state, c->h_poll, c->poll_ev, s,
                     &st);
   double v[2] = {0.0, 0.0};  // |b|, r.r
   if (!rc && (hipMemcpyAsync(c->h_poll_sc, sc, sizeof v,

@@ -355,19 +355,22 @@ int solver_static_scratch(int device, double** out);
 // on a few thousand equations, so the enqueueing host stays ahead.
 constexpr int kPollChunk = 8;
 
-// Iterations enqueued ahead of the host: chunks of `chunk` iterations with
-// a copy of the systems' states behind each; the host looks at a chunk's
-// states while the next one runs, so the device never waits for it (an
-// iteration of a finished system returns at once).  enqueue(it) launches
+// Iterations enqueued ahead of the host: chunks of `chunk` iterations (the
+// first of `first`, then twice as many until then: 1 where the guess may
+// already be the solution) with a copy of the systems' states behind each;
+// the host looks at a chunk's states while the next one runs, so the device
+// never waits for it (an iteration of a finished system returns at once:
+// some 2 us).  enqueue(it) launches
 // iteration it (0 .. maxit; maxit only tests).  h[0], h[1]: pinned images
 // of 2 nsys words; *out points to the one with the final states.
 template <typename Enq>
-int solve_poll(const Enq& enqueue, int nsys, int maxit, int chunk,
+int solve_poll(const Enq& enqueue, int nsys, int maxit, int first, int chunk,
                const int32_t* d_state, int32_t* const h[2],
                const hipEvent_t ev[2], hipStream_t s, const int32_t** out) {
   int rc;
   for (int it = 0, k = 0;; ++k) {
-    const int end = maxit - it > chunk ? it + chunk : maxit;
+    const int end = maxit - it > first ? it + first : maxit;
+    first = 2 * first < chunk ? 2 * first : chunk;
     for (; it < end; ++it)
       if ((rc = enqueue(it))) return rc;
     const bool last = it >= maxit;

@@ -678,7 +678,7 @@ int w3d_batch_advance(w3d_batch* b, w3d_problem* const* ps, int32_t n,
         [&](int it) {
           return launch_pcg_batch_iter(B, it, b->d_state, b->d_sc, s);
         },
-        ns, maxit, kPollChunk, b->d_state, b->h_state, b->poll_ev, s, &st);
+        ns, maxit, kPollChunk, kPollChunk, b->d_state, b->h_state, b->poll_ev, s, &st);
     if (rc) return fail(rc, "w3d_batch_advance: solver launch");
     b->mark(4, 1);
     int it = 0;

@@ -743,7 +743,7 @@ int bicgstab(int n, const RowGroups& A, const double* val, const double* b,
         }
         return hipGetLastError() == hipSuccess ? W3D_OK : W3D_ERR_DEVICE;
       },
-      1, maxit, kPollChunk, S.state, h, ev, st, &state);
+      1, maxit, kPollChunk, kPollChunk, S.state, h, ev, st, &state);
   if (rc) return rc;
   const int end = state[0];
   *iters = state[1];
