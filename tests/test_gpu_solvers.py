@@ -159,7 +159,7 @@ def test_pcg_from_the_solution():
     """A guess that is the solution costs little more than the same call
     limited to one iteration: the host sees the first iteration's state
     behind two more.  Bound: two launches, a copy and an event, some 20 us, on
-    the 90 us of the limited call, and as much again for the box; the 16
+    the 90 us of the limited call, and as much again for the machine; the 16
     iterations enqueued before it looked took 1.47 times the limited call."""
     import time
     mat = _abi.mm01_material(200e3, 0.3, 400.0, hprime=2000.0)
