@@ -155,11 +155,12 @@ def test_tuning_a_small_model_does_not_slow_it(W, prec):
 
 
 def test_pattern_leaves_no_spinning_threads(W):
-    """After w3d_pattern of a large model the host's threads are idle: its
-    last parallel loop lies before some 300 ms of serial work and copies, past
-    the 200 ms for which OpenMP's threads spin.  With one at the end they
-    used 2.8 s of processor time in the next 250 ms, and calls beside a
-    caller's own threads stalled for 4 ms each."""
+    """After w3d_pattern of a large model the host's threads are soon idle:
+    its last parallel loop lies before some 200 to 300 ms of serial work and
+    copies, and OpenMP's threads spin for 200 ms.  With one at the end they
+    used 2.8 to 3 s of processor time in the next 250 ms, and calls beside a
+    caller's own threads stalled for 4 ms each.  Bound: half of that, 15
+    threads for the 100 ms that remain where the serial part takes 100."""
     import time
     m = M.box_hex8(64)
     dev = W.BlockModel(m.model(
@@ -169,4 +170,4 @@ def test_pattern_leaves_no_spinning_threads(W):
     dev.pattern(cst)
     t = time.process_time()
     time.sleep(0.25)
-    assert time.process_time() - t < 0.2
+    assert time.process_time() - t < 1.5
